@@ -21,9 +21,10 @@
  *   stored in that permuted order (fp16, scaled per row by a power of two), so
  *   A and B agree and the dot product is unchanged.
  *   Q6_K: 1024 + q is built as an fp16 bit pattern with v_perm_b32, then
- *   fma(1024 + q, sc, -1056 sc) = sc (q - 32) exactly and one multiply by d
- *   rounds once: the fp16 weight is the reference's f32 weight (kernels.c:
- *   1855-1874) rounded to nearest even.  Q4_K: d sc q - dmin m in f32 with one
+ *   ((1024 + q) - 1056) sc = sc (q - 32), exact up to 2048 in magnitude, and one
+ *   multiply by d rounds once: the fp16 weight is the reference's f32 weight
+ *   (kernels.c:1855-1874) rounded to nearest even (scales of 65 and more round
+ *   the largest products to 11 bits first).  Q4_K: d sc q - dmin m in f32 with one
  *   fused multiply-add (kernels.c:1844-1852), then rounded to fp16.
  *
  * v1 (PF_SPLIT, PF_BF16) -- 64 x 64 output tiles, 256 threads, operands of
@@ -274,7 +275,7 @@ template <> struct RawOf<true> { typedef RawQ6 T; };
 template <> struct RawOf<false> { typedef RawQ4 T; };
 
 /* Per super-block constants of one lane's half. */
-struct ConstQ6 { f16x2 sc[8], bias[8], d; };   /* sc[s] = (S[s], S[s]), bias = -1056 sc */
+struct ConstQ6 { f16x2 sc[8], d; };            /* sc[s] = (S[s], S[s]) */
 struct ConstQ4 { float s[4], m[4]; };          /* sub-blocks 4h .. 4h+3: d*sc, dmin*m */
 template <bool Q6> struct ConstOf;
 template <> struct ConstOf<true> { typedef ConstQ6 T; };
@@ -288,7 +289,6 @@ __device__ __forceinline__ void raw_consts(const RawQ6 &r, int h, ConstQ6 &c)
         const int v = (int)(int8_t)((r.S[s >> 2] >> (8 * (s & 3))) & 0xFFu);
         const _Float16 f = (_Float16)v;
         c.sc[s] = (f16x2){ f, f };
-        c.bias[s] = c.sc[s] * (f16x2){ (_Float16)-1056.0f, (_Float16)-1056.0f };   /* exact: 33 * 32 * sc */
     }
     const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)r.d);
     c.d = (f16x2){ d, d };
@@ -317,9 +317,12 @@ __device__ __forceinline__ void raw_consts(const RawQ4 &r, int h, ConstQ4 &c)
 __device__ __forceinline__ f16x2 magic_lo(uint32_t q) { return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(q, 0x64646464u, 0x00050004u)); }
 __device__ __forceinline__ f16x2 magic_hi(uint32_t q) { return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(q, 0x64646464u, 0x00070006u)); }
 
-__device__ __forceinline__ uint32_t q6_pair(f16x2 v, f16x2 sc, f16x2 bias, f16x2 d)
+/* v holds 1024 + q; the offset comes off before the product with the scale
+ * (an int8: -1056 sc would overflow fp16 from |sc| = 63 on). */
+__device__ __forceinline__ uint32_t q6_pair(f16x2 v, f16x2 sc, f16x2 d)
 {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, sc, bias) * d);
+    const f16x2 off = { (_Float16)-1056.0f, (_Float16)-1056.0f };
+    return __builtin_bit_cast(uint32_t, (v + off) * sc * d);
 }
 
 /* B operands of k-slices j and j + 8 (j = 0..7). */
@@ -331,13 +334,13 @@ __device__ __forceinline__ void dequant_pair(const RawQ6 &r, const ConstQ6 &c, i
     const uint32_t qc = ((A >> 4) & 0x0F0F0F0Fu) | (C & 0x30303030u);
     const uint32_t qd = ((B >> 4) & 0x0F0F0F0Fu) | ((C >> 2) & 0x30303030u);
     const int s = j >> 2;
-    const uint4 u0 = { q6_pair(magic_lo(qa), c.sc[s], c.bias[s], c.d), q6_pair(magic_hi(qa), c.sc[s], c.bias[s], c.d),
-                       q6_pair(magic_lo(qb), c.sc[s + 2], c.bias[s + 2], c.d),
-                       q6_pair(magic_hi(qb), c.sc[s + 2], c.bias[s + 2], c.d) };
-    const uint4 u1 = { q6_pair(magic_lo(qc), c.sc[s + 4], c.bias[s + 4], c.d),
-                       q6_pair(magic_hi(qc), c.sc[s + 4], c.bias[s + 4], c.d),
-                       q6_pair(magic_lo(qd), c.sc[s + 6], c.bias[s + 6], c.d),
-                       q6_pair(magic_hi(qd), c.sc[s + 6], c.bias[s + 6], c.d) };
+    const uint4 u0 = { q6_pair(magic_lo(qa), c.sc[s], c.d), q6_pair(magic_hi(qa), c.sc[s], c.d),
+                       q6_pair(magic_lo(qb), c.sc[s + 2], c.d),
+                       q6_pair(magic_hi(qb), c.sc[s + 2], c.d) };
+    const uint4 u1 = { q6_pair(magic_lo(qc), c.sc[s + 4], c.d),
+                       q6_pair(magic_hi(qc), c.sc[s + 4], c.d),
+                       q6_pair(magic_lo(qd), c.sc[s + 6], c.d),
+                       q6_pair(magic_hi(qd), c.sc[s + 6], c.d) };
     b0 = __builtin_bit_cast(f16x8, u0);
     b1 = __builtin_bit_cast(f16x8, u1);
 }
