@@ -38,7 +38,8 @@ extern "C" {
 /* Prefill GEMM operand precision (fp32 accumulation in every mode). */
 #define ROASTER_PREC_F16   0   /* fp16 operands, activations scaled per row by a power of two; the
                                   per-(token, expert) down rows kept in fp16 until the combine (default) */
-#define ROASTER_PREC_SPLIT 1   /* bf16 hi+lo split of both operands, 3 MFMAs per product block */
+#define ROASTER_PREC_SPLIT 1   /* nearest f32: fp16 hi+lo activations on exact integer weights (inter <= 512, gate
+                                  and up of one type), else bf16 hi+lo of both operands, 3 MFMAs per block */
 #define ROASTER_PREC_BF16  2   /* bf16 operands: fastest to convert, about 8 significant bits */
 
 /* ---- runtime ------------------------------------------------------------ */
@@ -245,7 +246,10 @@ int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, int T, float
  * tiles (0); -1 queries.  Both give bit-identical results.  Returns the mode
  * in force. */
 int roaster_prefill_balanced_down(int enable);
-/* The fp16-mode gate/up GEMM on a persistent grid, one workgroup per CU taking
+/* The fp16-mode gate/up GEMM of longer prompts (past 28 rows per expert on
+ * average for Q6_K gate matrices, 36 for Q4_K; shorter ones run on
+ * 32-row tiles where gate and up types match, whatever this says) on
+ * a persistent grid, one workgroup per CU taking
  * (tile, 128-column) units from work counters and preparing the next unit
  * while one runs (1, default; layers whose routed and shared gate and up
  * matrices share one type and whose hidden size is a multiple of 512, at

@@ -213,4 +213,13 @@ __device__ __forceinline__ void row_scale(float amax, float &inv, float &fwd)
     fwd = __builtin_bit_cast(float, (uint32_t)(127 + s) << 23);
 }
 
+/* The same over every finite amax (a row near the largest f32 included). */
+__device__ __forceinline__ void row_scale_wide(float amax, float &inv, float &fwd)
+{
+    int s = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 255u) - 127 - 14;
+    s = s < -112 ? -112 : (s > 113 ? 113 : s);
+    inv = __builtin_bit_cast(float, (uint32_t)(127 - s) << 23);
+    fwd = __builtin_bit_cast(float, (uint32_t)(127 + s) << 23);
+}
+
 #endif

@@ -27,7 +27,9 @@
  *   the largest products to 11 bits first).  Q4_K: d sc q - dmin m in f32 with one
  *   fused multiply-add (kernels.c:1844-1852), then rounded to fp16.
  *
- * v1 (PF_SPLIT, PF_BF16) -- 64 x 64 output tiles, 256 threads, operands of
+ * Short prompts' fp16 gate/up and most of PF_SPLIT run on pf_narrow.hip.
+ *
+ * v1 (PF_BF16; PF_SPLIT where pf_narrow.hip does not take it) -- 64 x 64 output tiles, 256 threads, operands of
  * both sides dequantised / converted into LDS (gemm.h).
  */
 #include <type_traits>
@@ -35,7 +37,7 @@
 #include "internal.h"
 #include "gemm.h"
 #include "prefill.h"
-#include "tile.h"
+#include "pf_tile.h"
 
 /* Opt-in timing (build with -DROASTER_PF_TS): thread 0 of each of the first
  * 4096 workgroups of a GEMM launch records the 100 MHz real-time counter at
@@ -83,34 +85,6 @@ extern "C" int roaster_pf_ts2(unsigned long long *out)
 #define PF_TSD(i) do { } while (0)
 #define PF_TSUV(u, i, v) do { } while (0)
 #endif
-
-static __device__ __forceinline__ float pf_silu_mul(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
-/* The exponent s of row_scale(amax): fwd = 2^s, clamped to [-100, 100]. */
-static __device__ __forceinline__ int pf_scale_exp(float amax)
-{
-    const int s = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 255u) - 127 - 14;
-    return s < -100 ? -100 : (s > 100 ? 100 : s);
-}
-/* SiLU(g) * u with the hardware exp and reciprocal (v_exp_f32, v_rcp_f32: a
- * few ulp in f32; the result is rounded to fp16 for the next GEMM anyway). */
-static __device__ __forceinline__ float pf_silu_mul_fast(float g, float u)
-{
-    return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
-}
-
-/* A workgroup barrier that orders LDS accesses only: every wave's LDS reads
- * and writes complete, global loads may stay in flight (__syncthreads()
- * waits for those too). */
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-/* Virtual block id: blocks b < R = ntiles * nblk run; on a grid dispatched
- * round-robin over the 8 XCDs, XCD b % 8 takes the contiguous range of
- * virtual ids [(b % 8) * R / 8, ...), so the n-blocks of one tile and the
- * consecutive tiles of one expert share an L2. */
-__device__ __forceinline__ int pf_virtual_block(int b, int R)
-{
-    return (R & 7) ? b : (b & 7) * (R >> 3) + (b >> 3);
-}
 
 struct PfRowMeta {
     const float *src[GM];
@@ -264,16 +238,6 @@ static_assert(V2_DN_N == PF_DN_ROWS, "the down GEMM's unit is the plan kernel's"
 #define PF_DN_NT 4                /* down output tiles per workgroup (inter <= 512) */
 #endif
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-
-/* One lane's raw share of a super-block: half h (weights 128h .. 128h+127). */
-struct RawQ6 { uint32_t L[16], Hh[8], S[2], d; };
-struct RawQ4 { uint32_t hd[4], Q[16]; };
-template <bool Q6> struct RawOf;
-template <> struct RawOf<true> { typedef RawQ6 T; };
-template <> struct RawOf<false> { typedef RawQ4 T; };
-
 /* Per super-block constants of one lane's half. */
 struct ConstQ6 { f16x2 sc[8], d; };            /* sc[s] = (S[s], S[s]) */
 struct ConstQ4 { float s[4], m[4]; };          /* sub-blocks 4h .. 4h+3: d*sc, dmin*m */
@@ -312,10 +276,6 @@ __device__ __forceinline__ void raw_consts(const RawQ4 &r, int h, ConstQ4 &c)
         c.m[i] = dmin * (float)m;
     }
 }
-
-/* fp16 pairs (1024 + b0, 1024 + b1) and (1024 + b2, 1024 + b3) of the bytes of q. */
-__device__ __forceinline__ f16x2 magic_lo(uint32_t q) { return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(q, 0x64646464u, 0x00050004u)); }
-__device__ __forceinline__ f16x2 magic_hi(uint32_t q) { return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(q, 0x64646464u, 0x00070006u)); }
 
 /* v holds 1024 + q; the offset comes off before the product with the scale
  * (an int8: -1056 sc would overflow fp16 from |sc| = 63 on). */
@@ -362,15 +322,6 @@ __device__ __forceinline__ void dequant_pair(const RawQ4 &r, const ConstQ4 &c, i
     b0 = q4_slice(r.Q[j], c.s[0], c.m[0], c.s[1], c.m[1]);
     b1 = q4_slice(r.Q[8 + j], c.s[2], c.m[2], c.s[3], c.m[3]);
 }
-
-/* Natural position p (multiple of 4) of a super-block -> its permuted slot. */
-__device__ __forceinline__ int perm_slot4(int p)
-{
-    const int h = p >> 7, q = p & 127, hi = q >> 6, r = q & 63;
-    const int l0 = r < 32 ? r : r - 32, i0 = r < 32 ? 0 : 4;
-    return (8 * hi + (l0 >> 2)) * 16 + 8 * h + i0;
-}
-
 
 /* ---- v2 workgroup: 8 waves, two per SIMD -------------------------------------
  * Each wave owns one 32-row MFMA column block of weights: for gate/up, lanes
@@ -452,39 +403,6 @@ __device__ __forceinline__ void v4_mfma_mixed(f32x16 (&acc)[MS], const _Float16 
  * rows with 16 up rows).  The raw registers are double-buffered per wave: step
  * kb + 1's loads are issued before step kb's MFMA work, with no workgroup
  * barrier for them, and the LDS holds activations only. */
-__device__ __forceinline__ void tile_load(RawQ6 &r, const uint8_t *tile, int lane)
-{
-    const uint8_t *p = tile + 16 * lane;
-    uint4 s[6];
-#pragma unroll
-    for (int i = 0; i < 6; i++) s[i] = gld_u4(p + 1024 * i);
-    const uint3 s6 = gld_u3(p + 1024 * 6);          /* the record's last dword is padding */
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        r.L[4 * i] = s[i].x; r.L[4 * i + 1] = s[i].y; r.L[4 * i + 2] = s[i].z; r.L[4 * i + 3] = s[i].w;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        r.Hh[4 * i] = s[4 + i].x; r.Hh[4 * i + 1] = s[4 + i].y; r.Hh[4 * i + 2] = s[4 + i].z; r.Hh[4 * i + 3] = s[4 + i].w;
-    }
-    r.S[0] = s6.x;
-    r.S[1] = s6.y;
-    r.d = s6.z & 0xFFFFu;
-}
-
-__device__ __forceinline__ void tile_load(RawQ4 &r, const uint8_t *tile, int lane)
-{
-    const uint8_t *p = tile + 16 * lane;
-    uint4 s[5];
-#pragma unroll
-    for (int i = 0; i < 5; i++) s[i] = gld_u4(p + 1024 * i);
-    r.hd[0] = s[0].x; r.hd[1] = s[0].y; r.hd[2] = s[0].z; r.hd[3] = s[0].w;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        r.Q[4 * i] = s[1 + i].x; r.Q[4 * i + 1] = s[1 + i].y; r.Q[4 * i + 2] = s[1 + i].z; r.Q[4 * i + 3] = s[1 + i].w;
-    }
-}
-
 /* Slice i of a lane's record (one 16-byte load, the last Q6_K slice 12
  * bytes): the pieces of tile_load, issued one at a time. */
 __device__ __forceinline__ void tile_slice(RawQ6 &r, const uint8_t *tile, int lane, int i)
@@ -1770,7 +1688,7 @@ int pf_matmul_launch(const PfGemmArgs &A, int max_tiles)
  * the register budget of two waves per SIMD). */
 int pf_gemm_chunk(int op, bool mixed_gate_up) { return op == PF_F16 ? (mixed_gate_up ? 64 : V2_MC) : GM; }
 
-int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op)
+int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op, int max_nw)
 {
     if (max_tiles <= 0) return 0;
     if (op == PF_SPLIT) return launch_v1<PF_SPLIT>(A, max_tiles);
@@ -1782,7 +1700,9 @@ int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op)
         hipLaunchKernelGGL(pf2_fused_kernel, dim3(R.n_cu), dim3(V2_T), (size_t)GP_LDS, R.stream, A);
         return rt_check(hipGetLastError(), "prefill fused GEMM launch") ? ROASTER_EDEVICE : 0;
     }
-    if (A.gu_pers && g_pf_gu_pers)
+    if (max_nw > 0) {
+        if (int rc = pf_narrow_gu_launch(A, max_nw, false)) return rc;
+    } else if (A.gu_pers && g_pf_gu_pers)
         hipLaunchKernelGGL(pf2_gu_pers_kernel, dim3(R.n_cu), dim3(V2_T), (size_t)GP_LDS, R.stream, A);
     else
         hipLaunchKernelGGL(pf2_gu_kernel, dim3(max_tiles * (A.I / V2_GU_J)), dim3(V2_T), lds_gu, R.stream, A);

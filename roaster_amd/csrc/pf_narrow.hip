@@ -23,23 +23,13 @@
  * activations 6 bits less.
  */
 #include <type_traits>
-#include <stdlib.h>
 
 #include "internal.h"
 #include "gemm.h"
 #include "prefill.h"
 #include "pf_tile.h"
 
-#ifndef DN_OCC
-#define DN_OCC 3
-#endif
-#ifndef GUS_OCC
-#define GUS_OCC 3
-#endif
-#ifndef DN_NTMAX
-#define DN_NTMAX 2
-#endif
-#define NW_ROWS 32
+#define NW_ROWS 32                /* operand rows */
 #define NW_SUM GK                 /* a staged row: 256 activations, 16 sub-block sums, padding */
 #define NW_LD (GK + 16 + 8)       /* fp16 row pitch: 35 16-byte granules, so the 32 rows of an operand
                                      read start in different bank groups */
@@ -207,7 +197,19 @@ __device__ __forceinline__ void nw_block(NwAcc<N> &acc, const _Float16 *Xs, cons
     for (int i = 0; i < N; i++) acc.v[i] = fmaf(d, SPLIT ? z[i] + z[(i + 8) & 15] : z[i], acc.v[i]);
 }
 
-/* ---- gate/up -------------------------------------------------------------- */
+/* ---- gate/up -----------------------------------------------------------------
+ * Bound by the weights' bytes: short prompts touch nearly every expert with a
+ * few rows each.  Four waves (64 columns) per workgroup and three workgroups
+ * per CU (168 registers, 36 KB of LDS) keep 60-84 KB of weights in flight per
+ * CU, each super-block's loads issued a whole step ahead, and one workgroup's
+ * barriers, prologue and epilogue run under the others' loads; 45 tokens make
+ * 1,568 workgroups of even size where one workgroup per CU over 128-column
+ * units left a fourth round for a quarter of the CUs.  Q4_K, 256 experts,
+ * hidden 2048, inter 512, kernel trace: 45 tokens 100 -> 54 us (257 MB of
+ * weights: 4.8 TB/s, the rate of a large copy), 512 skewed tokens 133 -> 86.
+ * Split mode (16-row tiles), 256 tokens: gate/up 671 -> 75 us against the
+ * 64 x 64 tiles of gemm.h; 32-row tiles with separate hi and lo products took
+ * 100 us (twice the MFMAs and staging registers, two waves per SIMD). */
 struct NwMeta {
     int tok[NW_ROWS];
     float fwd[NW_ROWS];
@@ -333,7 +335,7 @@ __device__ __forceinline__ void nw_gu_body(const PfGemmArgs &A, const PfGroup &G
 }
 
 template <int NWV, bool SPLIT>
-__global__ void __launch_bounds__(64 * NWV, SPLIT ? GUS_OCC : 3) pfn_gu_kernel(PfGemmArgs A)
+__global__ void __launch_bounds__(64 * NWV, 3) pfn_gu_kernel(PfGemmArgs A)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t nw_lds[];
     __shared__ NwMeta meta;
@@ -352,10 +354,9 @@ __global__ void __launch_bounds__(64 * NWV, SPLIT ? GUS_OCC : 3) pfn_gu_kernel(P
  * of the f32 SiLU*up rows, scaled by the row's power of two (from its part
  * maxima) and split into fp16 hi + lo, with their sub-block sums -- and walks
  * dn_nt blocks of 128 output rows, the next block's weights loaded as each
- * super-block's registers come free. */
-#ifndef NWD_T
+ * super-block's registers come free.  256 tokens, Q6_K: 386 -> 60 us against
+ * the 64 x 64 tiles of gemm.h; 8-wave workgroups 65 us. */
 #define NWD_T 256
-#endif
 #define NWD_N (NWD_T / 2)         /* output rows per block: 32 a wave */
 
 template <bool Q6, int NKB>
@@ -457,7 +458,7 @@ __device__ __forceinline__ void nw_dn_body(const PfGemmArgs &A, const PfGroup &G
     }
 }
 
-extern "C" __global__ void __launch_bounds__(NWD_T, DN_OCC) pfn_down_kernel(PfGemmArgs A)
+extern "C" __global__ void __launch_bounds__(NWD_T, 3) pfn_down_kernel(PfGemmArgs A)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t nw_lds[];
     __shared__ __attribute__((aligned(16))) float fwd[2 * NW_ROWS];
@@ -490,18 +491,20 @@ int pf_narrow_gu_launch(const PfGemmArgs &A, int max_tiles, bool split)
     return rt_check(hipGetLastError(), "prefill gate/up launch") ? ROASTER_EDEVICE : 0;
 }
 
-int pf_narrow_max_t()
-{
-    static const int v = getenv("NW_MAXT") ? atoi(getenv("NW_MAXT")) : 768;
-    return v;
-}
+/* Where the line lies: fp16 mode's wide tiles (pf_gemm.hip) dequantise a weight
+ * once per 96 rows, these once per 32, but run at three waves per SIMD and
+ * balance in units of 64 columns.  Measured per layer (256 experts, hidden
+ * 2048, inter 512, Q6_K down; wide -> narrow, us): Q4_K gate/up 512 tokens 206
+ * -> 174, 768 226 -> 190, 1024 236 -> 214, 2048 302 -> 316; Q6_K gate/up 512
+ * 211 -> 200, 768 233 -> 217, 1024 239 -> 240, 2048 301 -> 347. */
+bool pf_narrow_f16(int T, int E, int q6) { return 8 * (long long)T <= (long long)E * (q6 ? 28 : 36); }
 
 int pf_narrow_launch(const PfGemmArgs &A, int max_tiles)
 {
     if (int rc = pf_narrow_gu_launch(A, max_tiles, true)) return rc;
     PfGemmArgs D = A;
-    const int nb = A.H / NWD_N;
-    D.dn_nt = DN_NTMAX >= 8 && nb % 8 == 0 ? 8 : DN_NTMAX >= 4 && nb % 4 == 0 ? 4 : 2;
+    const int nb = A.H / NWD_N;                      /* even: H is a multiple of 256 */
+    D.dn_nt = 2;                                     /* 1 / 2 / 4 / 8 blocks: 256 tokens 2 and 4 within 1%, 8 +3% */
     const size_t lds = (size_t)(A.I / GK) * NW_BUF * 2;
     hipLaunchKernelGGL(pfn_down_kernel, dim3((unsigned)(max_tiles * (nb / D.dn_nt))), dim3(NWD_T), lds, rt().stream, D);
     return rt_check(hipGetLastError(), "prefill down launch") ? ROASTER_EDEVICE : 0;

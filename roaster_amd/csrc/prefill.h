@@ -43,6 +43,11 @@ struct PfGemmArgs {
     const int *ntiles;              /* device count of valid tiles */
     const float *X;                 /* [* x H] activations (f32, natural order) */
     const uint16_t *X16;            /* [* x H] fp16 activations, scaled, permuted (v2), or NULL */
+    const uint16_t *X16l;           /* [* x H] what X16 rounded off, fp16 (split mode on narrow tiles), or NULL */
+    const uint16_t *xs16;           /* [*][H / 256][16] sums of X16 (+ X16l) over the 32-column sub-blocks, scaled
+                                       by 2^-6: eight fp16 hi, eight lo (narrow tiles), or NULL */
+    const PfTile *gu_tiles;         /* the groups cut into narrow tiles, and their device count, or NULL */
+    const int *gu_ntiles;
     const float *xinv, *xfwd;       /* per X row power-of-two scales (fp16 mode), or NULL */
     float *act;                     /* [slots x I]: silu(gate) * up (f32 operand modes) */
     uint16_t *act16;                /* [slots x I]: the same in fp16, each 16-column part scaled by the
@@ -102,8 +107,18 @@ bool pf_fused_enabled();
 int pf_gemm_chunk(int op, bool mixed_gate_up);
 
 /* Launch the gate/up and down GEMMs over up to max_tiles tiles.  op: PF_F16,
- * PF_SPLIT or PF_BF16 (gemm.h).  0 or ROASTER_EDEVICE. */
-int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op);
+ * PF_SPLIT or PF_BF16 (gemm.h).  max_nw > 0 (PF_F16): gate/up on up to max_nw
+ * narrow tiles (pf_narrow.hip).  0 or ROASTER_EDEVICE. */
+int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op, int max_nw = 0);
+
+/* The GEMMs on narrow tiles (pf_narrow_rows rows) with exact integer weights
+ * (pf_narrow.hip): gate/up in fp16 or split mode, down in split mode.  They
+ * read gu_tiles and xs16, the matrices' tile layout, gate and up matrices of
+ * one type per group; down needs inter <= 512.  0 or ROASTER_EDEVICE. */
+int pf_narrow_rows(bool split);
+bool pf_narrow_f16(int T, int E, int q6);                        /* whether fp16 mode's gate/up GEMM runs on them */
+int pf_narrow_gu_launch(const PfGemmArgs &A, int max_tiles, bool split);
+int pf_narrow_launch(const PfGemmArgs &A, int max_tiles);        /* both GEMMs, split mode */
 
 /* The down GEMM alone in split mode as a plain product: out[slot][r] =
  * act[slot] . W[r] over A.I columns for A.H (a multiple of 64) rows of each

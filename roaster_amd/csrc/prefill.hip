@@ -168,6 +168,8 @@ struct PfTokArgs {
     float *sg;                  /* [T] */
     float *xinv, *xfwd;         /* [T] (fp16 mode) or NULL */
     uint16_t *x16;              /* [T x H] fp16 X * xinv in the GEMM's permuted K order, or NULL */
+    uint16_t *x16l;             /* [T x H] what x16 rounded off (split mode on narrow tiles), or NULL */
+    uint16_t *xs16;             /* [T][H / 256][16] sub-block sums of x16 + x16l, scaled by 2^-6 (hi, lo), or NULL */
     int *err;
     int T, E, H;
 };
@@ -250,7 +252,8 @@ extern "C" __global__ void __launch_bounds__(256) pf_token_kernel(PfTokArgs A)
     for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
     if (A.xinv) {
         float inv, fwd;
-        row_scale(mx, inv, fwd);
+        if (A.x16l) row_scale_wide(mx, inv, fwd);
+        else row_scale(mx, inv, fwd);
         if (lane == 0) {
             A.xinv[t] = inv;
             A.xfwd[t] = fwd;
@@ -262,8 +265,27 @@ extern "C" __global__ void __launch_bounds__(256) pf_token_kernel(PfTokArgs A)
                 if (k < A.H) {
                     const float4 v = xv[i];
                     const f32x8 e = { v.x * inv, v.y * inv, v.z * inv, v.w * inv, 0.f, 0.f, 0.f, 0.f };
-                    const uint4 c = __builtin_bit_cast(uint4, __builtin_convertvector(e, f16x8));
-                    *(uint2 *)(A.x16 + (size_t)t * A.H + (k & ~255) + pf_perm_slot4(k & 255)) = make_uint2(c.x, c.y);
+                    const f16x8 hi = __builtin_convertvector(e, f16x8);
+                    const uint4 c = __builtin_bit_cast(uint4, hi);
+                    const size_t at = (size_t)t * A.H + (k & ~255) + pf_perm_slot4(k & 255);
+                    *(uint2 *)(A.x16 + at) = make_uint2(c.x, c.y);
+                    f32x8 used = __builtin_convertvector(hi, f32x8);
+                    if (A.x16l) {
+                        const f16x8 lo = __builtin_convertvector(e - used, f16x8);
+                        const uint4 lc = __builtin_bit_cast(uint4, lo);
+                        *(uint2 *)(A.x16l + at) = make_uint2(lc.x, lc.y);
+                        used = used + __builtin_convertvector(lo, f32x8);
+                    }
+                    if (A.xs16) {
+                        /* a 32-column sub-block is 8 neighbouring lanes */
+                        const float sum = group_sum<8>((used[0] + used[1]) + (used[2] + used[3])) * 0.015625f;
+                        const _Float16 sh = (_Float16)sum, sl = (_Float16)(sum - (float)sh);
+                        uint16_t *o = A.xs16 + ((size_t)t * (A.H / 256) + i) * 16 + (lane >> 3);
+                        if ((lane & 7) == 0) {
+                            o[0] = __builtin_bit_cast(uint16_t, sh);
+                            o[8] = __builtin_bit_cast(uint16_t, sl);
+                        }
+                    }
                 }
             }
         }
@@ -346,6 +368,9 @@ struct PfPlanArgs {
     int nt_out;                 /* its units per tile: H / PF_DN_ROWS */
     int T, E;
     int chunk;                  /* rows per tile */
+    PfTile *nw_tiles;           /* the groups cut into nw_rows-row tiles too, or NULL */
+    int *nw_ntiles;
+    int nw_rows;
 };
 
 /* Cost of the down-GEMM units of a group of c rows cut into tiles of chunk
@@ -361,34 +386,34 @@ __device__ __forceinline__ int pf_dn_group_cost(int c, int chunk, int nt_out)
     return (nt - 1) * pf_dn_tile_cost(chunk, nt_out) + pf_dn_tile_cost(c - (nt - 1) * chunk, nt_out);
 }
 
-/* Three exclusive prefix sums over a 256-thread workgroup in one pass (one
+/* Four exclusive prefix sums over a 256-thread workgroup in one pass (one
  * LDS exchange); *total gets the sums. */
-__device__ int3 block_scan3_256(int3 v, int *lds, int3 *total)
+__device__ int4 block_scan4_256(int4 v, int *lds, int4 *total)
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int3 inc = v;
+    int4 inc = v;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        const int ox = __shfl_up(inc.x, d), oy = __shfl_up(inc.y, d), oz = __shfl_up(inc.z, d);
-        if (lane >= d) { inc.x += ox; inc.y += oy; inc.z += oz; }
+        const int ox = __shfl_up(inc.x, d), oy = __shfl_up(inc.y, d), oz = __shfl_up(inc.z, d), ow = __shfl_up(inc.w, d);
+        if (lane >= d) { inc.x += ox; inc.y += oy; inc.z += oz; inc.w += ow; }
     }
-    if (lane == 63) { lds[w] = inc.x; lds[4 + w] = inc.y; lds[8 + w] = inc.z; }
+    if (lane == 63) { lds[w] = inc.x; lds[4 + w] = inc.y; lds[8 + w] = inc.z; lds[12 + w] = inc.w; }
     __syncthreads();
-    int3 before = make_int3(0, 0, 0), all = make_int3(0, 0, 0);
+    int4 before = make_int4(0, 0, 0, 0), all = make_int4(0, 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const int cx = lds[i], cy = lds[4 + i], cz = lds[8 + i];
-        if (i < w) { before.x += cx; before.y += cy; before.z += cz; }
-        all.x += cx; all.y += cy; all.z += cz;
+        const int cx = lds[i], cy = lds[4 + i], cz = lds[8 + i], cw = lds[12 + i];
+        if (i < w) { before.x += cx; before.y += cy; before.z += cz; before.w += cw; }
+        all.x += cx; all.y += cy; all.z += cz; all.w += cw;
     }
     __syncthreads();
     *total = all;
-    return make_int3(before.x + inc.x - v.x, before.y + inc.y - v.y, before.z + inc.z - v.z);
+    return make_int4(before.x + inc.x - v.x, before.y + inc.y - v.y, before.z + inc.z - v.z, before.w + inc.w - v.w);
 }
 
 extern "C" __global__ void __launch_bounds__(256) pf_plan_kernel(PfPlanArgs A)
 {
-    __shared__ int wsum[12];
+    __shared__ int wsum[16];
     __shared__ int s_gc[258], s_toff[257], s_c[257];
     const int e = threadIdx.x;
     if (e < 8) A.gu_ctr[e] = 0;
@@ -397,9 +422,17 @@ extern "C" __global__ void __launch_bounds__(256) pf_plan_kernel(PfPlanArgs A)
     const float dbnd = e < A.E ? A.dbound[e] : 0.0f, sdbnd = A.dbound[A.E];
     const int nt = (c + A.chunk - 1) / A.chunk;
     const int cost = A.dn_bnd && e < A.E ? pf_dn_group_cost(c, A.chunk, A.nt_out) : 0;
-    int3 tot;
-    const int3 pre = block_scan3_256(make_int3(c, nt, cost), wsum, &tot);
+    const int nn = A.nw_tiles ? (c + A.nw_rows - 1) / A.nw_rows : 0;
+    int4 tot;
+    const int4 pre = block_scan4_256(make_int4(c, nt, cost, nn), wsum, &tot);
     const int off = pre.x, toff = pre.y, tot_tiles = tot.y;
+    if (A.nw_tiles) {
+        const int no = pre.w, ntot = tot.w, nns = (A.T + A.nw_rows - 1) / A.nw_rows;
+        if (e < A.E)
+            for (int i = 0; i < nn; i++) A.nw_tiles[no + i] = PfTile{ e, i * A.nw_rows };
+        for (int i = e; i < nns; i += 256) A.nw_tiles[ntot + i] = PfTile{ A.E, i * A.nw_rows };
+        if (e == 0) *A.nw_ntiles = ntot + nns;
+    }
     const int nsh = (A.T + A.chunk - 1) / A.chunk;
     /* per group: tile offset and rows (group E: the shared expert); with the
      * balanced down GEMM, its cost prefix (each tile a range start plus its
@@ -664,6 +697,14 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     const LayerGeo &LG = t->geo[layer];
     const int chunk = pf_gemm_chunk(op, LG.q6[0] != LG.q6[1] || LG.sh_q6[0] != LG.sh_q6[1]);
     const int max_tiles = (int)((8 * TT + chunk - 1) / chunk + E + (TT + chunk - 1) / chunk);
+    /* narrow tiles with exact integer weights (pf_narrow.hip): the routed and
+     * the shared expert's gate and up matrices each of one type */
+    const bool one_type = LG.q6[0] == LG.q6[1] && LG.sh_q6[0] == LG.sh_q6[1];
+    const bool nw_split = op == PF_SPLIT && one_type && I <= 2 * GK;
+    const bool nw_f16 = op == PF_F16 && one_type && pf_narrow_f16(T, E, LG.q6[0]);
+    const bool narrow = nw_split || nw_f16;
+    const int nw_rows = pf_narrow_rows(nw_split);
+    const int max_nw = (int)((8 * TT + nw_rows - 1) / nw_rows + E + (TT + nw_rows - 1) / nw_rows);
 
     /* workspace */
     size_t sz = 0;
@@ -671,7 +712,10 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     const size_t o_part = opt.logits_in ? 0 : take((size_t)RT_KSPLIT * TT * E * 4);
     const size_t o_ids = take(TT * 8 * 4), o_w = take(TT * 8 * 4), o_rank = take(TT * 8 * 4);
     const size_t o_sg = take(TT * 4), o_xinv = take(TT * 4), o_xfwd = take(TT * 4);
-    const size_t o_x16 = op == PF_F16 ? take(TT * H * 2) : 0;
+    const size_t o_x16 = op == PF_F16 || nw_split ? take(TT * H * 2) : 0;
+    const size_t o_x16l = nw_split ? take(TT * H * 2) : 0;
+    const size_t o_xs16 = narrow ? take(TT * (H / RQK) * 32) : 0;
+    const size_t o_nwt = narrow ? take(sizeof(PfTile) * max_nw) : 0, o_nwn = narrow ? take(4) : 0;
     const size_t o_cnt = take((size_t)E * 4), o_off = take((size_t)E * 4), o_list = take((size_t)E * TT * 4);
     const size_t o_grp = take(sizeof(PfGroup) * (E + 1)), o_tiles = take(sizeof(PfTile) * max_tiles);
     const size_t o_nt = take(4), o_pmax = take(slots * (size_t)(I / 16) * 4);
@@ -705,9 +749,11 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     ta.ids_out = opt.ids_out;
     ta.w_out = opt.w_out;
     ta.sg = (float *)(ws + o_sg);
-    ta.xinv = op == PF_F16 ? (float *)(ws + o_xinv) : nullptr;
-    ta.xfwd = op == PF_F16 ? (float *)(ws + o_xfwd) : nullptr;
-    ta.x16 = op == PF_F16 ? (uint16_t *)(ws + o_x16) : nullptr;
+    ta.xinv = op == PF_F16 || nw_split ? (float *)(ws + o_xinv) : nullptr;
+    ta.xfwd = op == PF_F16 || nw_split ? (float *)(ws + o_xfwd) : nullptr;
+    ta.x16 = op == PF_F16 || nw_split ? (uint16_t *)(ws + o_x16) : nullptr;
+    ta.x16l = nw_split ? (uint16_t *)(ws + o_x16l) : nullptr;
+    ta.xs16 = narrow ? (uint16_t *)(ws + o_xs16) : nullptr;
     ta.err = (int *)(ctrl + 16);
     ta.T = T; ta.E = E; ta.H = H;
     hipLaunchKernelGGL(pf_token_kernel, dim3((T + 3) / 4), dim3(256), 0, R.stream, ta);
@@ -740,12 +786,15 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     const int q6 = LG.q6[0];
     const bool gu_one = LG.q6[1] == q6 && LG.sh_q6[0] == q6 && LG.sh_q6[1] == q6;
     const int gu_pers = op == PF_F16 && gu_one && (H / 256) % 2 == 0 && H / 256 >= 8 ? 1 + q6 : 0;
-    const bool fused = gu_pers && I <= 2 * GK && R.n_xcd == 8 && R.n_cu % 8 == 0 && pf_fused_enabled();
+    const bool fused = gu_pers && !nw_f16 && I <= 2 * GK && R.n_xcd == 8 && R.n_cu % 8 == 0 && pf_fused_enabled();
     pa.fx = fused ? (int *)(ws + o_fx) : nullptr;
     pa.n_wg = R.n_cu;
     pa.nt_out = H / PF_DN_ROWS;
     pa.T = T; pa.E = E;
     pa.chunk = chunk;
+    pa.nw_tiles = narrow ? (PfTile *)(ws + o_nwt) : nullptr;
+    pa.nw_ntiles = narrow ? (int *)(ws + o_nwn) : nullptr;
+    pa.nw_rows = nw_rows;
     hipLaunchKernelGGL(pf_plan_kernel, dim3(1), dim3(256), 0, R.stream, pa);
     if (rt_check(hipGetLastError(), "prefill plan launch")) return ROASTER_EDEVICE;
 
@@ -755,11 +804,15 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     ga.ntiles = pa.ntiles;
     ga.X = X;
     ga.X16 = ta.x16;
+    ga.X16l = ta.x16l;
+    ga.xs16 = ta.xs16;
+    ga.gu_tiles = pa.nw_tiles;
+    ga.gu_ntiles = pa.nw_ntiles;
     ga.xinv = ta.xinv;
     ga.xfwd = ta.xfwd;
     ga.act = (float *)(ws + o_act);
     ga.act16 = (uint16_t *)(ws + o_act);
-    ga.pmax = op == PF_F16 ? (float *)(ws + o_pmax) : nullptr;
+    ga.pmax = op == PF_F16 || nw_split ? (float *)(ws + o_pmax) : nullptr;
     /* fp16 mode: per-(token, expert) products in fp16, each row scaled by a
      * power of two of its bound (half the bytes of f32 rows, written by the
      * down GEMM and read back by the combine) */
@@ -782,7 +835,7 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     ga.dn_ctr = fused ? pa.fx + 16 : nullptr;
     ga.tile_done = fused ? pa.fx + 32 : nullptr;
     ga.err = (int *)(ctrl + 16);
-    if (int rc = pf_gemm_launch(ga, max_tiles, op)) return rc;
+    if (int rc = nw_split ? pf_narrow_launch(ga, max_nw) : pf_gemm_launch(ga, max_tiles, op, nw_f16 ? max_nw : 0)) return rc;
 
     if (op == PF_F16)
         hipLaunchKernelGGL(pf_combine16_kernel, dim3(T), dim3(256), 0, R.stream, (const uint16_t *)ga.out16,

@@ -1,0 +1,63 @@
+"""GPU parity of the prefill GEMMs on narrow tiles (pf_narrow.hip) against the
+oracle, where their tiles, K loops and operands can go wrong.
+
+Eight experts, so every expert gets every token: T = 1 .. 65 covers a tile's
+first and last row and one row past it (16 rows in split mode, 32 in fp16
+mode; fp16 mode leaves the narrow tiles past T = 28 with Q6_K and 36 with Q4_K
+gate matrices), hidden 256 / 768 / 2048 one, an odd and an even number of super-blocks,
+inter 256 / 512 one and two in the down product.  Q6_K scales take the whole
+int8 range: sc (q - 32) then exceeds 2048, where split mode's second weight
+operand holds what fp16 rounds off.  Routed and shared types are opposite, so
+each call runs both weight types.
+
+Bars: fp16 operands 2e-3 of max|y| as every fp16 prefill test; split mode
+1e-5 -- activations of 22 bits (2^-22 per product, random in sign) against
+f32 sums of up to 2048 terms on both sides, about 1e-6 each, through two
+products."""
+import numpy as np
+import pytest
+
+import roaster_amd as R
+from gpu_util import SynthTable, log, prefill, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def wide_scales(mat, rng):
+    """Q6_K bytes with scales over all of int8, d reduced to keep the weights' size."""
+    b = mat.reshape(-1, R.Q6K_BYTES).copy()
+    b[:, 192:208] = rng.integers(0, 256, (len(b), 16), dtype=np.uint8)
+    d = b[:, 208:210].copy().view(np.float16)
+    b[:, 208:210] = (d / np.float16(4)).view(np.uint8)
+    return b.reshape(-1)
+
+
+@pytest.fixture(scope="module", params=[(256, 256, 0, 1), (768, 512, 1, 0), (2048, 512, 0, 1), (2048, 512, 1, 0)],
+                ids=lambda p: "H%d-I%d-gu%d-dn%d" % p)
+def table(request):
+    H, I, gu, dn = request.param
+    q6, sq6 = (gu, gu, dn), (1 - gu, 1 - gu, 1 - dn)
+    t = SynthTable(11, n_experts=8, hidden=H, inter=I, q6=q6, sh_q6=sq6)
+    rng = np.random.default_rng(5)
+    for e in range(9):
+        types = sq6 if e == 8 else q6
+        m = [wide_scales(w, rng) if q else w for w, q in zip(t.expert(0, e), types)]
+        t._experts[(0, e)] = tuple(m)
+        R.check(R.lib().roaster_table_set_expert(t.t, 0, e, *(w.ctypes.data for w in m)), "set_expert")
+    yield t
+    t.destroy()
+
+
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33, 65])
+@pytest.mark.parametrize("prec,tol", [(R.PREC_F16, 2e-3), (R.PREC_SPLIT, 1e-5)], ids=["f16", "split"])
+def test_narrow_tiles(table, T, prec, tol):
+    H = table.desc.hidden
+    X = np.stack([R.synth_normal(9, R.synth_stream(0, t, 5), H) for t in range(T)])
+    X[T // 2] *= 2.0 ** 10                        # a row's scale is its own
+    Y, lg, ids, w, counts = prefill(table, X, precision=prec)
+    assert counts.tolist() == [T] * 8
+    rc, Y_ref, ids_ref, _, _ = table.oracle_layer(0).prefill(X, logits_in=lg)
+    assert rc == 0 and np.array_equal(ids_ref, ids)
+    err = max(rel_err(Y[t], Y_ref[t]) for t in range(T))
+    log(f"T {T} precision {prec}: max|d|/max|y| over rows = {err:.2e}")
+    assert err <= tol
