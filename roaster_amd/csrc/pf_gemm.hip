@@ -1688,10 +1688,15 @@ int pf_matmul_launch(const PfGemmArgs &A, int max_tiles)
  * the register budget of two waves per SIMD). */
 int pf_gemm_chunk(int op, bool mixed_gate_up) { return op == PF_F16 ? (mixed_gate_up ? 64 : V2_MC) : GM; }
 
-int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op, int max_nw)
+int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op, int max_nw, bool nw_down)
 {
     if (max_tiles <= 0) return 0;
-    if (op == PF_SPLIT) return launch_v1<PF_SPLIT>(A, max_tiles);
+    if (max_nw > 0) {
+        if (int rc = pf_narrow_gu_launch(A, max_nw, op == PF_SPLIT)) return rc;
+        if (nw_down) return pf_narrow_down_launch(A, max_nw, op == PF_SPLIT);
+    } else if (op == PF_SPLIT) {
+        return launch_v1<PF_SPLIT>(A, max_tiles);
+    }
     if (op == PF_BF16) return launch_v1<PF_BF16>(A, max_tiles);
     RtState &R = rt();
     const size_t lds_gu = 2 * (size_t)V3_XBUF * 2, lds_dn = lds_gu;
@@ -1700,13 +1705,13 @@ int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op, int max_nw)
         hipLaunchKernelGGL(pf2_fused_kernel, dim3(R.n_cu), dim3(V2_T), (size_t)GP_LDS, R.stream, A);
         return rt_check(hipGetLastError(), "prefill fused GEMM launch") ? ROASTER_EDEVICE : 0;
     }
-    if (max_nw > 0) {
-        if (int rc = pf_narrow_gu_launch(A, max_nw, false)) return rc;
-    } else if (A.gu_pers && g_pf_gu_pers)
-        hipLaunchKernelGGL(pf2_gu_pers_kernel, dim3(R.n_cu), dim3(V2_T), (size_t)GP_LDS, R.stream, A);
-    else
-        hipLaunchKernelGGL(pf2_gu_kernel, dim3(max_tiles * (A.I / V2_GU_J)), dim3(V2_T), lds_gu, R.stream, A);
-    if (rt_check(hipGetLastError(), "prefill gate/up launch")) return ROASTER_EDEVICE;
+    if (max_nw <= 0) {
+        if (A.gu_pers && g_pf_gu_pers)
+            hipLaunchKernelGGL(pf2_gu_pers_kernel, dim3(R.n_cu), dim3(V2_T), (size_t)GP_LDS, R.stream, A);
+        else
+            hipLaunchKernelGGL(pf2_gu_kernel, dim3(max_tiles * (A.I / V2_GU_J)), dim3(V2_T), lds_gu, R.stream, A);
+        if (rt_check(hipGetLastError(), "prefill gate/up launch")) return ROASTER_EDEVICE;
+    }
     PfGemmArgs D = A;
     if (A.I <= 2 * GK && g_pf_dn_bal && A.dn_bnd && A.dn_tiles && A.out16) {
         /* every K step's activations fit in LDS: one workgroup per CU over an

@@ -349,74 +349,115 @@ __global__ void __launch_bounds__(64 * NWV, 3) pfn_gu_kernel(PfGemmArgs A)
     else nw_gu_body<NWV, false, SPLIT>(A, G, meta, tile.m0, mlen, j0, (_Float16 *)nw_lds);
 }
 
-/* ---- down, split mode (inter <= 512) -----------------------------------------
- * A workgroup (4 waves) stages its tile's activations once -- every super-block
- * of the f32 SiLU*up rows, scaled by the row's power of two (from its part
- * maxima) and split into fp16 hi + lo, with their sub-block sums -- and walks
- * dn_nt blocks of 128 output rows, the next block's weights loaded as each
- * super-block's registers come free.  256 tokens, Q6_K: 386 -> 60 us against
- * the 64 x 64 tiles of gemm.h; 8-wave workgroups 65 us. */
+/* ---- down (inter <= 512) -----------------------------------------------------
+ * A workgroup (4 waves) stages its tile's activations once, every super-block
+ * of the SiLU*up rows with their sub-block sums, and walks dn_nt blocks of 128
+ * output rows, the next block's weights loaded as each super-block's registers
+ * come free.  Split mode: the f32 rows, scaled by the row's power of two (from
+ * its part maxima) and split into fp16 hi + lo; f32 products.  fp16 mode: the
+ * fp16 rows, each 16-column part moved from its own power of two onto the
+ * row's; the products leave in fp16, scaled by 2^-e, e the exponent of the
+ * bound max|act| * dbnd, as the wide down GEMMs store them (pf_gemm.hip).
+ * 256 tokens split, Q6_K: 386 -> 60 us against the 64 x 64 tiles of gemm.h;
+ * 8-wave workgroups 65 us. */
 #define NWD_T 256
 #define NWD_N (NWD_T / 2)         /* output rows per block: 32 a wave */
 
-template <bool Q6, int NKB>
-__device__ __forceinline__ void nw_dn_body(const PfGemmArgs &A, const PfGroup &G, float *fwd, int m0, int mlen, int n0,
+struct NwDnMeta {
+    float inv[NW_ROWS], fwd[NW_ROWS];
+    int8_t psh[NW_ROWS][32];      /* fp16 mode: part scale exponent - row scale exponent (<= 0) */
+};
+
+template <bool Q6, bool SPLIT, int NKB>
+__device__ __forceinline__ void nw_dn_body(const PfGemmArgs &A, const PfGroup &G, NwDnMeta &meta, int m0, int mlen, int n0,
                                            int nt_count, _Float16 *Xb)
 {
-    constexpr int ROWS = NwTile<true>::ROWS, TB = TL_BYTES(Q6), NP = ROWS * NKB * 32 / NWD_T;
+    constexpr int ROWS = NwTile<SPLIT>::ROWS, TB = TL_BYTES(Q6), NP = ROWS * NKB * 32 / NWD_T, NR = ROWS * 16 / NWD_T;
     const int t = threadIdx.x, l = t & 63, h = l >> 5, w = t >> 6, n = l & 31;
     const size_t slot0 = (size_t)(G.slot0 + m0);
     /* part maxima: 16 lanes per row, NKB of its 16 NKB parts each */
-    const int prow = (t >> 4) % ROWS;
-    const float *pp = A.pmax + (slot0 + min(prow, mlen - 1)) * (16 * NKB) + (t & 15) * NKB;
-    float pm[NKB];
+    float pm[NR][NKB];
 #pragma unroll
-    for (int k = 0; k < NKB; k++) pm[k] = pp[k];
+    for (int i = 0; i < NR; i++) {
+        const float *pp = A.pmax + (slot0 + min((t >> 4) + i * (NWD_T / 16), mlen - 1)) * (16 * NKB) + (t & 15) * NKB;
+#pragma unroll
+        for (int k = 0; k < NKB; k++) pm[i][k] = pp[k];
+    }
     /* activations: piece i of a thread is 8 columns of row idx / (32 NKB) */
     float4 xa[NP][2];
+    uint4 xh[NP];
 #pragma unroll
     for (int i = 0; i < NP; i++) {
         const int idx = t + i * NWD_T, row = min(idx / (32 * NKB), mlen - 1), c = idx % (32 * NKB);
-        const float *p = A.act + (slot0 + row) * (GK * NKB) + 8 * c;
-        xa[i][0] = gld_f4(p);
-        xa[i][1] = gld_f4(p + 4);
+        const size_t at = (slot0 + row) * (GK * NKB) + 8 * c;
+        if (SPLIT) {
+            xa[i][0] = gld_f4(A.act + at);
+            xa[i][1] = gld_f4(A.act + at + 4);
+        } else {
+            xh[i] = gld_u4(A.act16 + at);
+        }
     }
     typename RawOf<Q6>::T r[NKB];
     const uint8_t *wt = G.td + (size_t)((n0 + 32 * w) / TL_ROWS) * NKB * TB;
     constexpr size_t TN = (size_t)(NWD_N / TL_ROWS) * NKB * TB;          /* one block of output rows on */
 #pragma unroll
-    for (int k = 0; k < NKB; k++) tile_load(r[k], wt + (size_t)k * TB, l);
-    float mx = pm[0];
+    for (int k = 0; k < NKB; k++) nw_load(r[k], wt + (size_t)k * TB, 16 * l);
 #pragma unroll
-    for (int k = 1; k < NKB; k++) mx = fmaxf(mx, pm[k]);
-    mx = fmaxf(mx, dpp_f<DPP_XOR1>(mx));
-    mx = fmaxf(mx, dpp_f<DPP_XOR2>(mx));
-    mx = fmaxf(mx, dpp_f<DPP_HALF_MIRROR>(mx));
-    mx = fmaxf(mx, dpp_f<DPP_MIRROR>(mx));
-    float inv0, fwd0;
-    row_scale_wide(mx, inv0, fwd0);
-    float *inv = fwd + ROWS;
-    if ((t & 15) == 0 && t < 16 * ROWS) {
-        fwd[prow] = fwd0;
-        inv[prow] = inv0;
+    for (int i = 0; i < NR; i++) {
+        const int row = (t >> 4) + i * (NWD_T / 16);
+        float mx = pm[i][0];
+#pragma unroll
+        for (int k = 1; k < NKB; k++) mx = fmaxf(mx, pm[i][k]);
+        mx = fmaxf(mx, dpp_f<DPP_XOR1>(mx));
+        mx = fmaxf(mx, dpp_f<DPP_XOR2>(mx));
+        mx = fmaxf(mx, dpp_f<DPP_HALF_MIRROR>(mx));
+        mx = fmaxf(mx, dpp_f<DPP_MIRROR>(mx));
+        float inv, fwd;
+        if (SPLIT) {
+            row_scale_wide(mx, inv, fwd);
+        } else {
+            row_scale(mx, inv, fwd);
+            const int er = pf_scale_exp(mx), sp = pf_scale_exp(mx * G.dbnd);
+            fwd = __builtin_bit_cast(float, (uint32_t)(127 + max(-126, min(126, er - sp))) << 23);
+            if ((t & 15) == 0 && row < mlen && n0 == 0) A.oexp[slot0 + row] = (int8_t)sp;
+#pragma unroll
+            for (int k = 0; k < NKB; k++)
+                meta.psh[row][(t & 15) * NKB + k] = (int8_t)max(pf_scale_exp(pm[i][k]) - er, -64);
+        }
+        if ((t & 15) == 0) {
+            meta.inv[row] = inv;
+            meta.fwd[row] = fwd;
+        }
     }
     lds_barrier();
 #pragma unroll
     for (int i = 0; i < NP; i++) {
         const int idx = t + i * NWD_T, row = idx / (32 * NKB), c = idx % (32 * NKB), kb = c >> 5, c8 = 8 * (c & 31);
-        _Float16 *dh = Xb + kb * NW_BUF + row * NW_LD, *dl = dh + ROWS * NW_LD;
-        const float s = inv[row];
-        const f32x8 e = { xa[i][0].x * s, xa[i][0].y * s, xa[i][0].z * s, xa[i][0].w * s,
-                          xa[i][1].x * s, xa[i][1].y * s, xa[i][1].z * s, xa[i][1].w * s };
-        const f16x8 hi = __builtin_convertvector(e, f16x8);
-        const f32x8 back = __builtin_convertvector(hi, f32x8);
-        const f16x8 lo = __builtin_convertvector(e - back, f16x8);
-        const uint4 hu = __builtin_bit_cast(uint4, hi), lu = __builtin_bit_cast(uint4, lo);
+        if (i * NWD_T / (32 * NKB) >= mlen) break;                       /* workgroup-uniform */
+        _Float16 *dh = Xb + kb * NW_BUF + row * NW_LD;
         const int s0 = perm_slot4(c8), s1 = perm_slot4(c8 + 4);
+        f32x8 e;
+        if (SPLIT) {
+            const float s = meta.inv[row];
+            e = (f32x8){ xa[i][0].x, xa[i][0].y, xa[i][0].z, xa[i][0].w, xa[i][1].x, xa[i][1].y, xa[i][1].z, xa[i][1].w } * s;
+        } else {
+            const int sh = (int)meta.psh[row][c >> 1];
+            const f16x8 hv = __builtin_bit_cast(f16x8, xh[i]);
+#pragma unroll
+            for (int k = 0; k < 8; k++) e[k] = __builtin_ldexpf((float)hv[k], sh);
+        }
+        const f16x8 hi = __builtin_convertvector(e, f16x8);
+        const uint4 hu = __builtin_bit_cast(uint4, hi);
         *(uint2 *)(dh + s0) = make_uint2(hu.x, hu.y);
         *(uint2 *)(dh + s1) = make_uint2(hu.z, hu.w);
-        *(uint2 *)(dl + s0) = make_uint2(lu.x, lu.y);
-        *(uint2 *)(dl + s1) = make_uint2(lu.z, lu.w);
+        if (SPLIT) {
+            const f32x8 back = __builtin_convertvector(hi, f32x8);
+            const uint4 lu = __builtin_bit_cast(uint4, __builtin_convertvector(e - back, f16x8));
+            *(uint2 *)(dh + ROWS * NW_LD + s0) = make_uint2(lu.x, lu.y);
+            *(uint2 *)(dh + ROWS * NW_LD + s1) = make_uint2(lu.z, lu.w);
+        } else {
+            e = __builtin_convertvector(hi, f32x8);                      /* the sums of what the products see */
+        }
         if (!Q6) {
             /* a sub-block is four neighbouring lanes' pieces */
             float sum = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
@@ -433,53 +474,83 @@ __device__ __forceinline__ void nw_dn_body(const PfGemmArgs &A, const PfGroup &G
         /* the last block reloads its own weights: a fixed number of loads per
          * block, so that each wait counts only the loads it needs */
         wt += nt + 1 < nt_count ? TN : 0;
-        NwAcc<NwTile<true>::ACC> acc = {};
+        NwAcc<NwTile<SPLIT>::ACC> acc = {};
 #pragma unroll
         for (int k = 0; k < NKB; k++) {
             __builtin_amdgcn_sched_barrier(0);
-            nw_block<Q6, true>(acc, Xb + k * NW_BUF, r[k], l);
+            nw_block<Q6, SPLIT>(acc, Xb + k * NW_BUF, r[k], l);
             __builtin_amdgcn_sched_barrier(0);
-            tile_load(r[k], wt + (size_t)k * TB, l);
+            nw_load(r[k], wt + (size_t)k * TB, 16 * l);
         }
         /* addresses and scales are formed here, not kept over the blocks */
         int hh = h;
         asm volatile("" : "+v"(hh));
-        float *ob = A.out + slot0 * A.H + n0 + nt * NWD_N;
-        const uint32_t oo = (uint32_t)(4 * hh * A.H + 32 * w + n);
+        const size_t o0 = slot0 * A.H + n0 + nt * NWD_N;
+        if (SPLIT) {
+            float *ob = A.out + o0;
+            const uint32_t oo = (uint32_t)(4 * hh * A.H + 32 * w + n);
 #pragma unroll
-        for (int q = 0; q < ROWS / 8; q++) {
-            if (8 * q >= mlen) break;                                    /* wave-uniform */
-            const float4 f = *(const float4 *)(fwd + 8 * q + 4 * hh);
-            const float v[4] = { acc.v[4 * q] * f.x, acc.v[4 * q + 1] * f.y, acc.v[4 * q + 2] * f.z, acc.v[4 * q + 3] * f.w };
+            for (int q = 0; q < ROWS / 8; q++) {
+                if (8 * q >= mlen) break;                                /* wave-uniform */
+                const float4 f = *(const float4 *)(meta.fwd + 8 * q + 4 * hh);
+                const float v[4] = { acc.v[4 * q] * f.x, acc.v[4 * q + 1] * f.y, acc.v[4 * q + 2] * f.z, acc.v[4 * q + 3] * f.w };
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (8 * q + 4 * hh + i < mlen) ob[oo + (uint32_t)((8 * q + i) * A.H)] = v[i];
+                for (int i = 0; i < 4; i++)
+                    if (8 * q + 4 * hh + i < mlen) ob[oo + (uint32_t)((8 * q + i) * A.H)] = v[i];
+            }
+        } else {
+            /* lanes n and n ^ 1 swap one value of each row pair: the even lane
+             * stores the first row's two columns, the odd lane the second's */
+            const bool odd = (n & 1) != 0;
+            uint16_t *ob = A.out16 + o0;
+            const uint32_t oo = (uint32_t)((4 * hh + (odd ? 1 : 0)) * A.H + 32 * w + (n & ~1));
+#pragma unroll
+            for (int q = 0; q < ROWS / 8; q++) {
+                if (8 * q >= mlen) break;                                /* wave-uniform */
+                const float4 f = *(const float4 *)(meta.fwd + 8 * q + 4 * hh);
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                    const float v0 = acc.v[4 * q + i] * (i ? f.z : f.x), v1 = acc.v[4 * q + i + 1] * (i ? f.w : f.y);
+                    const float got = dpp_f<DPP_XOR1>(odd ? v0 : v1);
+                    const f16x2 pk = { (_Float16)(odd ? got : v0), (_Float16)(odd ? v1 : got) };
+                    if (8 * q + 4 * hh + i + (odd ? 1 : 0) < mlen)
+                        *(uint32_t *)(ob + oo + (uint32_t)((8 * q + i) * A.H)) = __builtin_bit_cast(uint32_t, pk);
+                }
+            }
         }
     }
 }
 
-extern "C" __global__ void __launch_bounds__(NWD_T, 3) pfn_down_kernel(PfGemmArgs A)
+template <bool SPLIT>
+__global__ void __launch_bounds__(NWD_T, 3) pfn_down_kernel(PfGemmArgs A)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t nw_lds[];
-    __shared__ __attribute__((aligned(16))) float fwd[2 * NW_ROWS];
+    __shared__ __attribute__((aligned(16))) NwDnMeta meta;
     const int nt = A.dn_nt, nblk = A.H / NWD_N / nt, R = *A.gu_ntiles * nblk;
     if ((int)blockIdx.x >= R) return;
     const int v = pf_virtual_block(blockIdx.x, R);
     const PfTile tile = A.gu_tiles[v / nblk];
     const PfGroup &G = A.groups[tile.grp];
-    const int mlen = min(NwTile<true>::ROWS, G.n - tile.m0), n0 = (v % nblk) * nt * NWD_N;
+    const int mlen = min(NwTile<SPLIT>::ROWS, G.n - tile.m0), n0 = (v % nblk) * nt * NWD_N;
     _Float16 *Xb = (_Float16 *)nw_lds;
     if (A.I > GK) {
-        if (G.dq6) nw_dn_body<true, 2>(A, G, fwd, tile.m0, mlen, n0, nt, Xb);
-        else nw_dn_body<false, 2>(A, G, fwd, tile.m0, mlen, n0, nt, Xb);
+        if (G.dq6) nw_dn_body<true, SPLIT, 2>(A, G, meta, tile.m0, mlen, n0, nt, Xb);
+        else nw_dn_body<false, SPLIT, 2>(A, G, meta, tile.m0, mlen, n0, nt, Xb);
     } else {
-        if (G.dq6) nw_dn_body<true, 1>(A, G, fwd, tile.m0, mlen, n0, nt, Xb);
-        else nw_dn_body<false, 1>(A, G, fwd, tile.m0, mlen, n0, nt, Xb);
+        if (G.dq6) nw_dn_body<true, SPLIT, 1>(A, G, meta, tile.m0, mlen, n0, nt, Xb);
+        else nw_dn_body<false, SPLIT, 1>(A, G, meta, tile.m0, mlen, n0, nt, Xb);
     }
 }
 
 /* ---- host ----------------------------------------------------------------- */
 int pf_narrow_rows(bool split) { return split ? NwTile<true>::ROWS : NwTile<false>::ROWS; }
+
+/* The down GEMM beside it: the wide one is level with this on Q6_K from 45
+ * tokens on (45 tokens 129.5 us a layer, here 131.9; 512 skewed 180, here 184;
+ * 4 tokens 55.4, here 52.8), and slower on Q4_K, whose dequantisation there
+ * costs twice the instructions (200 tokens 157 us, here 149; 512 skewed 175,
+ * here 170). */
+bool pf_narrow_f16_down(int T, int E, int q6) { return !q6 || 8 * (long long)T <= E; }
 
 int pf_narrow_gu_launch(const PfGemmArgs &A, int max_tiles, bool split)
 {
@@ -499,13 +570,14 @@ int pf_narrow_gu_launch(const PfGemmArgs &A, int max_tiles, bool split)
  * 211 -> 200, 768 233 -> 217, 1024 239 -> 240, 2048 301 -> 347. */
 bool pf_narrow_f16(int T, int E, int q6) { return 8 * (long long)T <= (long long)E * (q6 ? 28 : 36); }
 
-int pf_narrow_launch(const PfGemmArgs &A, int max_tiles)
+int pf_narrow_down_launch(const PfGemmArgs &A, int max_tiles, bool split)
 {
-    if (int rc = pf_narrow_gu_launch(A, max_tiles, true)) return rc;
     PfGemmArgs D = A;
     const int nb = A.H / NWD_N;                      /* even: H is a multiple of 256 */
     D.dn_nt = 2;                                     /* 1 / 2 / 4 / 8 blocks: 256 tokens 2 and 4 within 1%, 8 +3% */
+    const dim3 g((unsigned)(max_tiles * (nb / D.dn_nt))), b(NWD_T);
     const size_t lds = (size_t)(A.I / GK) * NW_BUF * 2;
-    hipLaunchKernelGGL(pfn_down_kernel, dim3((unsigned)(max_tiles * (nb / D.dn_nt))), dim3(NWD_T), lds, rt().stream, D);
+    if (split) hipLaunchKernelGGL(pfn_down_kernel<true>, g, b, lds, rt().stream, D);
+    else hipLaunchKernelGGL(pfn_down_kernel<false>, g, b, lds, rt().stream, D);
     return rt_check(hipGetLastError(), "prefill down launch") ? ROASTER_EDEVICE : 0;
 }

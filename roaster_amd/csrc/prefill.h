@@ -107,18 +107,20 @@ bool pf_fused_enabled();
 int pf_gemm_chunk(int op, bool mixed_gate_up);
 
 /* Launch the gate/up and down GEMMs over up to max_tiles tiles.  op: PF_F16,
- * PF_SPLIT or PF_BF16 (gemm.h).  max_nw > 0 (PF_F16): gate/up on up to max_nw
- * narrow tiles (pf_narrow.hip).  0 or ROASTER_EDEVICE. */
-int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op, int max_nw = 0);
+ * PF_SPLIT or PF_BF16 (gemm.h).  max_nw > 0 (PF_F16, PF_SPLIT): gate/up, and
+ * down with nw_down, on up to max_nw narrow tiles (pf_narrow.hip).  0 or
+ * ROASTER_EDEVICE. */
+int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op, int max_nw = 0, bool nw_down = false);
 
 /* The GEMMs on narrow tiles (pf_narrow_rows rows) with exact integer weights
- * (pf_narrow.hip): gate/up in fp16 or split mode, down in split mode.  They
- * read gu_tiles and xs16, the matrices' tile layout, gate and up matrices of
- * one type per group; down needs inter <= 512.  0 or ROASTER_EDEVICE. */
+ * (pf_narrow.hip), in fp16 or split mode.  They read gu_tiles, xs16 and the
+ * matrices' tile layout; gate/up takes gate and up matrices of one type per
+ * group, down inter <= 512.  0 or ROASTER_EDEVICE. */
 int pf_narrow_rows(bool split);
-bool pf_narrow_f16(int T, int E, int q6);                        /* whether fp16 mode's gate/up GEMM runs on them */
+bool pf_narrow_f16(int T, int E, int q6);      /* whether fp16 mode's gate/up GEMM runs on them, q6: gate type */
+bool pf_narrow_f16_down(int T, int E, int q6); /* and its down GEMM, q6: down type */
 int pf_narrow_gu_launch(const PfGemmArgs &A, int max_tiles, bool split);
-int pf_narrow_launch(const PfGemmArgs &A, int max_tiles);        /* both GEMMs, split mode */
+int pf_narrow_down_launch(const PfGemmArgs &A, int max_tiles, bool split);
 
 /* The down GEMM alone in split mode as a plain product: out[slot][r] =
  * act[slot] . W[r] over A.I columns for A.H (a multiple of 64) rows of each

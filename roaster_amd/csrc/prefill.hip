@@ -703,6 +703,7 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     const bool nw_split = op == PF_SPLIT && one_type && I <= 2 * GK;
     const bool nw_f16 = op == PF_F16 && one_type && pf_narrow_f16(T, E, LG.q6[0]);
     const bool narrow = nw_split || nw_f16;
+    const bool nw_down = nw_split || (nw_f16 && I <= 2 * GK && pf_narrow_f16_down(T, E, LG.q6[2]));
     const int nw_rows = pf_narrow_rows(nw_split);
     const int max_nw = (int)((8 * TT + nw_rows - 1) / nw_rows + E + (TT + nw_rows - 1) / nw_rows);
 
@@ -835,7 +836,7 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     ga.dn_ctr = fused ? pa.fx + 16 : nullptr;
     ga.tile_done = fused ? pa.fx + 32 : nullptr;
     ga.err = (int *)(ctrl + 16);
-    if (int rc = nw_split ? pf_narrow_launch(ga, max_nw) : pf_gemm_launch(ga, max_tiles, op, nw_f16 ? max_nw : 0)) return rc;
+    if (int rc = pf_gemm_launch(ga, max_tiles, op, narrow ? max_nw : 0, nw_down)) return rc;
 
     if (op == PF_F16)
         hipLaunchKernelGGL(pf_combine16_kernel, dim3(T), dim3(256), 0, R.stream, (const uint16_t *)ga.out16,
