@@ -1191,6 +1191,30 @@ __device__ __forceinline__ QChunk q_load_t(int q6, const uint8_t *m, size_t row,
     return q6 ? q_load<true>(m + (row * nb + lbc) * RQ6K_BYTES, c) : q_load<false>(m + (row * nb + lbc) * RQ4K_BYTES, c);
 }
 
+/* q_load_t without a branch: the same four loads for both types, at the
+ * type's offsets (Q4_K's last two repeat header bytes, unused), so that the
+ * number of loads in flight does not depend on the type and every wait behind
+ * them counts exactly. */
+__device__ __forceinline__ QChunk q_load_u(int q6, const uint8_t *m, size_t row, int nb, int lb, int c)
+{
+    const int lbc = lb < nb ? lb : nb - 1;
+    const uint8_t *blk = m + (row * nb + lbc) * (q6 ? RQ6K_BYTES : RQ4K_BYTES);
+    const int n = c >> 2, p = c & 3;
+    QChunk ch;
+    ch.q = gld_u4a2(blk + (q6 ? 0 : 16) + 16 * c);
+    ch.h = gld_u4a2(blk + (q6 ? 128 + 32 * n + 16 * (p & 1) : 0));
+    ch.s = gld_u2a2(blk + (q6 ? 192 + 8 * n : 0));
+    ch.dd = gld_u16(blk + (q6 ? 208 : 0));
+    return ch;
+}
+
+/* Down rows of type D (0 = Q4_K, 1 = Q6_K), or of q6's at run time (D < 0). */
+template <int D>
+__device__ __forceinline__ QChunk q_load_d(int q6, const uint8_t *m, size_t row, int nb, int lb, int c)
+{
+    return D < 0 ? q_load_u(q6, m, row, nb, lb, c) : q_load_t(D, m, row, nb, lb, c);
+}
+
 __device__ __forceinline__ int q_run_a_t(int q6, int c) { return q6 ? q_run_a<true>(c) : q_run_a<false>(c); }
 
 /* silu(gate_j . x) * (up_j . x) from the lane's chunks of one gate/up row
@@ -1808,8 +1832,8 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1_kernel(DecArgs 
 extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1_2x2_kernel(DecArgs A) { stack1_body<2, 2, 0x24>(A); }
 
 /* ---- one token, the router folded into the combine (dec_stack1r_kernel) ----
- * 256 experts, hidden 2048, inter 512, gate/up Q4_K and down Q6_K (routed and
- * shared).  Groups and slots as in dec_stack1_kernel (XCD k serves routed
+ * 256 experts, hidden 2048, inter 512, matrix types as in stack_types.  Groups
+ * and slots as in dec_stack1_kernel (XCD k serves routed
  * slot k; workgroup gi of every XCD combines rows [64 gi, 64 gi + 64)), but
  * each layer's router logits come from the rows the workgroups have just
  * combined, by linearity of the norm once 1/rms is known:
@@ -1898,13 +1922,15 @@ __device__ __forceinline__ float r1_gather_run(const uint64_t *base, int I, int 
 }
 
 /* k1_down_row's arithmetic on a rotated SiLU*up vector. */
-__device__ __forceinline__ float r1_down_row(const QChunk &ch, const float *eh, const float *ehs, bool live, int lane)
+__device__ __forceinline__ float r1_down_row(int d6, const QChunk &ch, const float *eh, const float *ehs, bool live,
+                                             int lane)
 {
     const int lr = lane & 15, c = lr & 7, lb = lr >> 3;
     float part = 0.0f;
     if (live) {
-        const int ca = lb * RQK + q_run_a<true>(c), cb = ca + 64;
-        part = q_chunk_dot<true>(ch, c, eh + r1_ehpos(ca), eh + r1_ehpos(cb), ehs[ca >> 4], ehs[cb >> 4]);
+        const int ca = lb * RQK + q_run_a_t(d6, c), cb = ca + (d6 ? 64 : 32);
+        part = d6 ? q_chunk_dot<true>(ch, c, eh + r1_ehpos(ca), eh + r1_ehpos(cb), ehs[ca >> 4], ehs[cb >> 4])
+                  : q_chunk_dot<false>(ch, c, eh + r1_ehpos(ca), eh + r1_ehpos(cb), ehs[ca >> 4], ehs[cb >> 4]);
     }
     return group_sum<16>(part);
 }
@@ -1964,7 +1990,10 @@ __device__ __forceinline__ void r1_prefetch_rs(const DecArgs &A, const DecLayer 
     }
 }
 
-extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs A)
+/* G: type of the gate and up matrices; D: of the down matrices, < 0 = each
+ * layer's own. */
+template <int G, int D>
+__device__ __forceinline__ void stack1r_body(const DecArgs &A)
 {
     constexpr int H = R1_H, I = R1_I, E = R1_E, HU = H / 4, nbh = H / RQK, nbi = I / RQK;
     constexpr int RD = R1_RD, SP = I / 256, RO = H / 256, RGP = I / K1_GW;
@@ -2042,11 +2071,11 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs
         if (wv >= K1_W - SP) {
             const size_t j = (size_t)gw * SP + (wv - (K1_W - SP));
             QChunk2 ch;
-            ch.g = q_load_t(0, L.sgate, j, nbh, lb, c);
-            ch.u = q_load_t(0, L.sup, j, nbh, lb, c);
+            ch.g = q_load_t(G, L.sgate, j, nbh, lb, c);
+            ch.u = q_load_t(G, L.sup, j, nbh, lb, c);
             shc_s[wv - (K1_W - SP)][lane] = ch;
             const int sdt = wv - (K1_W - nsd);
-            sdc_s[sdt][lane] = q_load_t(1, L.sdown, (size_t)min(gw * RO + sdt * rpw + rw_, H - 1), nbi, lr >> 3, lr & 7);
+            sdc_s[sdt][lane] = q_load_d<D>(L.sq6[2], L.sdown, (size_t)min(gw * RO + sdt * rpw + rw_, H - 1), nbi, lr >> 3, lr & 7);
         }
     }
     __syncthreads();
@@ -2199,7 +2228,7 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs
             k1_flag_wait(&s_xn, 4 * (li + 1));
             R1_TSW(6, 1);
             const int pr = wv - (K1_W - SP);
-            const float eh = k1_gu_pair(0, 0, shc_s[pr][lane], xn, xsum, swz, nbh, lane);
+            const float eh = k1_gu_pair(G, G, shc_s[pr][lane], xn, xsum, swz, nbh, lane);
             if (lane == 0) xch_put(xehs + (size_t)gw * XCH_LN + pr, eh, ep);
             R1_TSW(6, 2);
         }
@@ -2217,9 +2246,9 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs
         QChunk dch[2];
         R1_TSW(0, 15);
 #pragma unroll
-        for (int f = 0; f < 2; f++) gch[f].g = q_load_t(0, ge, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
+        for (int f = 0; f < 2; f++) gch[f].g = q_load_t(G, ge, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
 #pragma unroll
-        for (int f = 0; f < 2; f++) gch[f].u = q_load_t(0, ue, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
+        for (int f = 0; f < 2; f++) gch[f].u = q_load_t(G, ue, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
         const int sdt = wv - (K1_W - nsd);
         asm volatile("; R1MARK before xn wait" ::: "memory");
         R1_TSW(0, 12);
@@ -2227,17 +2256,17 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs
         R1_TS(5);
         float pgs[2];
 #pragma unroll
-        for (int f = 0; f < 2; f++) pgs[f] = k1_q_row(0, gch[f].g, xn, xsum, swz, nbh, lane);
+        for (int f = 0; f < 2; f++) pgs[f] = k1_q_row(G, gch[f].g, xn, xsum, swz, nbh, lane);
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("; gate rows dotted" ::"v"(pgs[0]) : "memory");
         R1_TSW(0, 13);
 #pragma unroll
         for (int f = 0; f < 2; f++)
-            dch[f] = q_load_t(1, de, (size_t)(gi * RD + (wv + f * K1_W) * rpw + rw_), nbi, lbd, lr & 7);
+            dch[f] = q_load_d<D>(L.q6[2], de, (size_t)(gi * RD + (wv + f * K1_W) * rpw + rw_), nbi, lbd, lr & 7);
 #pragma unroll
         for (int f = 0; f < 2; f++) {
             const int pj = wv + f * K1_W;
-            const float eh = silu_mul(pgs[f], k1_q_row(0, gch[f].u, xn, xsum, swz, nbh, lane));
+            const float eh = silu_mul(pgs[f], k1_q_row(G, gch[f].u, xn, xsum, swz, nbh, lane));
             if (lane == 0) xch_put_xcd(lehx + k1_run_slot(gi * RGP + pj, I), live_slot ? eh : 0.0f, ep, l2);
         }
         R1_TSW(6, 6);
@@ -2270,13 +2299,13 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs
              * down outputs (their SiLU*up values came in before the barrier) */
             const int rl = sdt * rpw + rw_;
             const bool live = rl < RO && lbd < nbi;
-            const float part = r1_down_row(sdc_s[sdt][lane], ehsh, ehshs, live, lane);
+            const float part = r1_down_row(D < 0 ? L.sq6[2] : D, sdc_s[sdt][lane], ehsh, ehshs, live, lane);
             if (live && lr == 0) xch_put(xdsh + (size_t)gw * XCH_LN + rl, part, ep);
         }
 #pragma unroll
         for (int f = 0; f < 2; f++) {
             const int rl = (wv + f * K1_W) * rpw + rw_, row = gi * RD + rl;
-            const float part = r1_down_row(dch[f], ehk, ehks, true, lane);
+            const float part = r1_down_row(D < 0 ? L.q6[2] : D, dch[f], ehk, ehks, true, lane);
             if (lr == 0) xch_put(xdx + (size_t)grp * H + row, live_slot ? part : 0.0f, ep);
         }
 
@@ -2292,9 +2321,9 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs
             } else if (wv >= K1_W - SP) {
                 const size_t j = (size_t)gw * SP + (wv - (K1_W - SP));
                 QChunk2 ch;
-                ch.g = q_load_t(0, L.sgate, j, nbh, lb, c);
-                ch.u = q_load_t(0, L.sup, j, nbh, lb, c);
-                const QChunk sd = q_load_t(1, L.sdown, (size_t)min(gw * RO + sdt * rpw + rw_, H - 1), nbi, lbd, lr & 7);
+                ch.g = q_load_t(G, L.sgate, j, nbh, lb, c);
+                ch.u = q_load_t(G, L.sup, j, nbh, lb, c);
+                const QChunk sd = q_load_d<D>(L.sq6[2], L.sdown, (size_t)min(gw * RO + sdt * rpw + rw_, H - 1), nbi, lbd, lr & 7);
                 shc_s[wv - (K1_W - SP)][lane] = ch;
                 sdc_s[sdt][lane] = sd;
             }
@@ -2333,6 +2362,10 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs
 #undef R1_TSW
 }
 
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs A) { stack1r_body<0, 1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_q4_kernel(DecArgs A) { stack1r_body<0, -1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_q6_kernel(DecArgs A) { stack1r_body<1, -1>(A); }
+
 /* ---- the batched one-launch stack: 2..8 tokens --------------------------------
  * The one-token stack's groups and exchanges with a token index: group k (an
  * XCD) serves slot k of every token (the token's k-th expert), so the chain
@@ -2364,9 +2397,8 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs
  * layer parity.
  * Every dot, sum, softmax and combine is the one-token kernel's, in its order,
  * so each token's results equal its one-token results bit for bit.  Shapes:
- * inter 512, hidden 512..2048 in whole 256-row blocks, at most 256 experts;
- * gate/up Q4_K and down Q6_K, routed and shared (dec_layerB_ok and the launch
- * check the rest). */
+ * inter 512, hidden 512..2048 in whole 256-row blocks, at most 256 experts
+ * (dec_layerB_ok); matrix types as in stack_types. */
 template <int NB>
 __device__ __forceinline__ void k1b_gather_h(const uint64_t *lh, int H, int HU, int u, int b0, int B, uint32_t ep,
                                              int &dead, uint32_t spin, float (*xn)[K1_MAXH])
@@ -2407,7 +2439,8 @@ __device__ __forceinline__ void k1b_gather_h(const uint64_t *lh, int H, int HU, 
     }
 }
 
-template <int NB>
+/* G, D: the matrix types as in stack1r_body. */
+template <int NB, int G, int D>
 __device__ __forceinline__ void stackB_body(const DecArgs &A)
 {
     __shared__ __align__(16) float xn[NB][K1_MAXH];
@@ -2510,10 +2543,10 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
             }
             if (wv >= K1_W - SP) {
                 const size_t j = (size_t)gw * SP + (wv - (K1_W - SP));
-                shc.g = q_load_t(0, Lx.sgate, j, nbh, lb, c);
-                shc.u = q_load_t(0, Lx.sup, j, nbh, lb, c);
+                shc.g = q_load_t(G, Lx.sgate, j, nbh, lb, c);
+                shc.u = q_load_t(G, Lx.sup, j, nbh, lb, c);
             }
-            if (sdt >= 0) sdc = q_load_t(1, Lx.sdown, (size_t)min(gw * RO + sdt * rpw + rw_, H - 1), nbi, lr >> 3, lr & 7);
+            if (sdt >= 0) sdc = q_load_d<D>(Lx.sq6[2], Lx.sdown, (size_t)min(gw * RO + sdt * rpw + rw_, H - 1), nbi, lr >> 3, lr & 7);
         };
         if (!EARLY || li == 0) wload(L);
         const int u = tid;
@@ -2614,7 +2647,7 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
         }
         for (int t = wv - 1; wv > 0 && t < SP * B; t += K1_W - 1) {
             const int pr = t % SP, b = t / SP;
-            const float eh = k1_gu_pair(0, 0, shc_s[pr][lane], xn[b], xsum[b], swz, nbh, lane);
+            const float eh = k1_gu_pair(G, G, shc_s[pr][lane], xn[b], xsum[b], swz, nbh, lane);
             if (lane == 0) xch_put(xehs + ((size_t)b * 256 + gw) * XCH_LN + pr, eh, ep);
         }
 
@@ -2677,9 +2710,9 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
                 const size_t ee = e >= 0 ? (size_t)e : 0;
                 const uint8_t *ge = L.gate + ee * L.eb[0], *ue = L.up + ee * L.eb[1];
 #pragma unroll
-                for (int f = 0; f < 2; f++) ch[f].g = q_load_t(0, ge, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
+                for (int f = 0; f < 2; f++) ch[f].g = q_load_t(G, ge, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
 #pragma unroll
-                for (int f = 0; f < 2; f++) ch[f].u = q_load_t(0, ue, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
+                for (int f = 0; f < 2; f++) ch[f].u = q_load_t(G, ue, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
             };
 #pragma unroll
             for (int b = 0; b < DG - 1; b++) gu_load(b, st[b]);
@@ -2704,15 +2737,15 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
                  * (k1_q_row's arithmetic per row) */
                 float pg[2] = {0.0f, 0.0f}, pu[2] = {0.0f, 0.0f};
                 if (lb < nbh) {
-                    const int xa = lb * RQK + q_run_a_t(0, c), xb = xa + 32;
+                    const int xa = lb * RQK + q_run_a_t(G, c), xb = xa + (G ? 64 : 32);
                     float4 x0[4], x1[4];
                     load_x16(xn[b], xa, x0, swz);
                     load_x16(xn[b], xb, x1, swz);
                     const float sa = xsum[b][xa >> 4], sb = xsum[b][xb >> 4];
 #pragma unroll
                     for (int f = 0; f < 2; f++) {
-                        pg[f] = q_chunk_dot_r<false>(cur[f].g, c, x0, x1, sa, sb);
-                        pu[f] = q_chunk_dot_r<false>(cur[f].u, c, x0, x1, sa, sb);
+                        pg[f] = q_chunk_dot_r<G != 0>(cur[f].g, c, x0, x1, sa, sb);
+                        pu[f] = q_chunk_dot_r<G != 0>(cur[f].u, c, x0, x1, sa, sb);
                     }
                 }
                 if constexpr (NB <= 4) {
@@ -2747,7 +2780,7 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
 #pragma unroll
                 for (int f = 0; f < 2; f++) {
                     const int task = min(wv + f * K1_W, ndt - 1);
-                    ch[f] = q_load_t(1, de, (size_t)min(gi * RD + task * rpw + rw_, H - 1), nbi, lbd, lr & 7);
+                    ch[f] = q_load_d<D>(L.q6[2], de, (size_t)min(gi * RD + task * rpw + rw_, H - 1), nbi, lbd, lr & 7);
                 }
             };
             /* 2 slots: the first token's down rows in flight through the
@@ -2780,7 +2813,7 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
                 const int rl = k * rpw + rw_;
                 const bool live = rl < RO && lbd < nbi;
                 k1_flag_wait(&s_eh_rdy[b], li + 1);
-                const float part = k1_down_row(1, sdc_s[li & 1][k][lane], ehsh[b], ehshs[b], live, lpr, lane);
+                const float part = k1_down_row(D < 0 ? L.sq6[2] : D, sdc_s[li & 1][k][lane], ehsh[b], ehshs[b], live, lpr, lane);
                 if (live && lr == 0) xch_put(xdsh + ((size_t)b * 256 + gw) * XCH_LN + rl, part, ep);
             }
 #pragma unroll
@@ -2796,7 +2829,7 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
                     if (task < ndt) {
                         const int rl = task * rpw + rw_, row = gi * RD + rl;
                         const bool live = rl < RD && lbd < nbi;
-                        const float part = k1_down_row(1, cur[f], ehk[b], ehks[b], live, lpr, lane);
+                        const float part = k1_down_row(D < 0 ? L.q6[2] : D, cur[f], ehk[b], ehks[b], live, lpr, lane);
                         if (live && lr == 0) xch_put(xdx + ((size_t)b * 8 + grp) * H + row, live_slot ? part : 0.0f, ep);
                     }
                 }
@@ -2846,9 +2879,16 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
 #undef K1_TS
 }
 
-extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB2_kernel(DecArgs A) { stackB_body<2>(A); }
-extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB4_kernel(DecArgs A) { stackB_body<4>(A); }
-extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB8_kernel(DecArgs A) { stackB_body<8>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB2_kernel(DecArgs A) { stackB_body<2, 0, 1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB4_kernel(DecArgs A) { stackB_body<4, 0, 1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB8_kernel(DecArgs A) { stackB_body<8, 0, 1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB2_q4_kernel(DecArgs A) { stackB_body<2, 0, -1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB4_q4_kernel(DecArgs A) { stackB_body<4, 0, -1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB8_q4_kernel(DecArgs A) { stackB_body<8, 0, -1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB2_q6_kernel(DecArgs A) { stackB_body<2, 1, -1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB4_q6_kernel(DecArgs A) { stackB_body<4, 1, -1>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB8_q6_kernel(DecArgs A) { stackB_body<8, 1, -1>(A); }
+
 
 /* Every workgroup's XCC_ID, in a grid of the stack kernel's shape. */
 extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_xcd_probe_kernel(unsigned *out)
@@ -2915,8 +2955,12 @@ static bool k1_fits()
 {
     if (g_k1_fits >= 0) return g_k1_fits == 1;
     const void *fns[] = {(const void *)dec_stack1_kernel, (const void *)dec_stack1_2x2_kernel,
-                         (const void *)dec_stack1r_kernel, (const void *)dec_stackB2_kernel,
-                         (const void *)dec_stackB4_kernel, (const void *)dec_stackB8_kernel};
+                         (const void *)dec_stack1r_kernel, (const void *)dec_stack1r_q4_kernel,
+                         (const void *)dec_stack1r_q6_kernel, (const void *)dec_stackB2_kernel,
+                         (const void *)dec_stackB4_kernel, (const void *)dec_stackB8_kernel,
+                         (const void *)dec_stackB2_q4_kernel, (const void *)dec_stackB4_q4_kernel,
+                         (const void *)dec_stackB8_q4_kernel, (const void *)dec_stackB2_q6_kernel,
+                         (const void *)dec_stackB4_q6_kernel, (const void *)dec_stackB8_q6_kernel};
     bool ok = rt().n_cu >= K1_NWG;
     for (const void *f : fns) {
         int nb = 0;
@@ -3051,20 +3095,64 @@ int dec_probe_placement()
 
 void dec_placement_failed() { g_xl2 = 0; }
 
-/* Which one-token kernel runs layers [c0, c0 + cn) of A on an exchange
- * buffer of xn slots: 0 dec_stack1r_kernel, 1 dec_stack1_2x2_kernel, 2
- * dec_stack1_kernel. */
-static int stack1_choice(const DecArgs &A, int c0, int cn, size_t xn)
+/* The matrix types of layers [l0, l0 + n) as the kernels are compiled for
+ * them: 0 = gate/up Q4_K and down Q6_K in every layer, 1 = gate/up Q4_K, down
+ * of either type, 2 = gate/up Q6_K, down of either type (routed and shared
+ * matrices alike), -1 = anything else. */
+static int stack_types(const DecArgs &A, int l0, int n)
+{
+    if (!A.layers_h) return -1;
+    const int g = A.layers_h[l0].q6[0] ? 1 : 0;
+    bool d6 = true;
+    for (int l = l0; l < l0 + n; l++) {
+        const DecLayer *Lh = A.layers_h + l;
+        for (int k = 0; k < 2; k++)
+            if ((Lh->q6[k] != 0) != g || (Lh->sq6[k] != 0) != g) return -1;
+        d6 = d6 && Lh->q6[2] && Lh->sq6[2];
+    }
+    return g ? 2 : d6 ? 0 : 1;
+}
+
+/* A one-launch kernel and its name. */
+struct StackKernel { const void *fn; const char *name; };
+#define STACK_KERNEL(f) StackKernel{ (const void *)f, #f }
+
+/* The one-token kernel of layers [c0, c0 + cn) of A on an exchange buffer of
+ * xn slots: the folded router at the model's shape wherever the types are one
+ * of stack_types' (16 layers with down types mixed by layer: 18.3 us per layer
+ * on the general kernel, 12.5 here; one all-Q6_K layer 25.2 and 17.1), else
+ * the general kernel. */
+static StackKernel stack1_choice(const DecArgs &A, int c0, int cn, size_t xn)
 {
     const int nbi = A.I / RQK, rpw = 64 / lanes_per_row(nbi);
     const int npg = (A.I / K1_GW + K1_W - 1) / K1_W, nd = ((A.H / K1_GW + rpw - 1) / rpw + K1_W - 1) / K1_W;
-    bool ty = A.layers_h != nullptr;
-    for (int l = c0; ty && l < c0 + cn; l++) {
-        const DecLayer *Lh = A.layers_h + l;
-        ty = !Lh->q6[0] && !Lh->q6[1] && Lh->q6[2] && !Lh->sq6[0] && !Lh->sq6[1] && Lh->sq6[2];
+    const int ty = stack_types(A, c0, cn);
+    if (ty >= 0 && A.cnt && dec_r1_shape(A.E, A.H, A.I) && xn >= (size_t)XR_U64(A.E, A.H, A.I))
+        return ty == 0 ? STACK_KERNEL(dec_stack1r_kernel)
+                       : ty == 1 ? STACK_KERNEL(dec_stack1r_q4_kernel) : STACK_KERNEL(dec_stack1r_q6_kernel);
+    return npg == 2 && nd == 2 && ty == 0 ? STACK_KERNEL(dec_stack1_2x2_kernel) : STACK_KERNEL(dec_stack1_kernel);
+}
+
+/* The kernel of B = 2..8 tokens (the smallest of 2, 4, 8 slots that holds B)
+ * for layers [l0, l0 + n) of A, or NULL (three kernels per layer).  Measured
+ * against those, us per layer of 16 with down types mixed by layer: 2 tokens
+ * 34.2 -> 20.2, 3 41.2 -> 26.5, 8 74.3 -> 51.4 (the run-time down type costs
+ * the 8-slot kernel 2.7 over the fixed one); one all-Q6_K layer of 4 tokens
+ * 46.4 -> 35.9. */
+static StackKernel stackB_choice(const DecArgs &A, int l0, int n)
+{
+    const int B = A.B;
+    switch (stack_types(A, l0, n)) {
+    case 0:
+        return B <= 2 ? STACK_KERNEL(dec_stackB2_kernel) : B <= 4 ? STACK_KERNEL(dec_stackB4_kernel) : STACK_KERNEL(dec_stackB8_kernel);
+    case 1:
+        return B <= 2 ? STACK_KERNEL(dec_stackB2_q4_kernel)
+                      : B <= 4 ? STACK_KERNEL(dec_stackB4_q4_kernel) : STACK_KERNEL(dec_stackB8_q4_kernel);
+    case 2:
+        return B <= 2 ? STACK_KERNEL(dec_stackB2_q6_kernel)
+                      : B <= 4 ? STACK_KERNEL(dec_stackB4_q6_kernel) : STACK_KERNEL(dec_stackB8_q6_kernel);
     }
-    if (ty && A.cnt && dec_r1_shape(A.E, A.H, A.I) && xn >= (size_t)XR_U64(A.E, A.H, A.I)) return 0;
-    return npg == 2 && nd == 2 && ty ? 1 : 2;
+    return StackKernel{ NULL, NULL };
 }
 
 /* One launch per run of up to K1_MAXL layers (dec_stack1_kernel) on the
@@ -3090,25 +3178,18 @@ static int launch_stack1(DecArgs &A0)
         X.epoch += (uint32_t)cn;
         A.spin = g_spin;
         A.xl2 = g_xl2 == 1;
-        const int ch = stack1_choice(A, c0, cn, X.n);
-        const void *fn = ch == 0 ? (const void *)dec_stack1r_kernel
-                         : ch == 1 ? (const void *)dec_stack1_2x2_kernel : (const void *)dec_stack1_kernel;
-        if (int rc = launch_k1(fn, A)) return rc;
+        if (int rc = launch_k1(stack1_choice(A, c0, cn, X.n).fn, A)) return rc;
     }
     return 0;
 }
 
-/* One launch per run of up to K1_MAXL layers of B = 2..8 tokens
- * (dec_stackB*_kernel, the smallest of 2, 4, 8 slots that holds B), when
- * every layer has Q4_K gate/up and Q6_K down matrices, routed and shared;
- * else 1 (the caller runs the three-kernel path). */
+/* One launch per run of up to K1_MAXL layers of B = 2..8 tokens on one kernel
+ * for all of the call's layers; 1 where there is none for their types (the
+ * caller runs the three-kernel path). */
 static int launch_stackB(DecArgs &A0)
 {
-    if (!A0.layers_h) return 1;
-    for (int l = A0.layer0; l < A0.layer0 + A0.nlayers; l++) {
-        const DecLayer *Lh = A0.layers_h + l;
-        if (Lh->q6[0] || Lh->q6[1] || !Lh->q6[2] || Lh->sq6[0] || Lh->sq6[1] || !Lh->sq6[2]) return 1;
-    }
+    const void *fn = stackB_choice(A0, A0.layer0, A0.nlayers).fn;
+    if (!fn) return 1;
     DecXch &X = *A0.xbuf;
     if (X.n < (size_t)XCHB_U64(K1B_MAXB, A0.E, A0.H, A0.I)) return 1;
     for (int c0 = A0.layer0; c0 < A0.layer0 + A0.nlayers; c0 += K1_MAXL) {
@@ -3129,8 +3210,6 @@ static int launch_stackB(DecArgs &A0)
         X.epoch += (uint32_t)cn;
         A.spin = g_spin;
         A.xl2 = g_xl2 == 1;
-        const void *fn = A.B <= 2 ? (const void *)dec_stackB2_kernel
-                         : A.B <= 4 ? (const void *)dec_stackB4_kernel : (const void *)dec_stackB8_kernel;
         if (int rc = launch_k1(fn, A)) return rc;
     }
     return 0;
@@ -3143,16 +3222,10 @@ const char *dec_kernel_names(const DecArgs &A)
     if (dec_layer1_ok(A.E, A.H, A.I, A.B)) {
         DecArgs C = A;
         if (!C.cnt) C.cnt = (uint32_t *)&C;               /* only its presence matters here */
-        const int ch = stack1_choice(C, A.layer0, std::min(A.nlayers, K1_MAXL), dec_xch_need1(A.E, A.H, A.I));
-        return ch == 0 ? "dec_stack1r_kernel" : ch == 1 ? "dec_stack1_2x2_kernel" : "dec_stack1_kernel";
+        return stack1_choice(C, A.layer0, std::min(A.nlayers, K1_MAXL), dec_xch_need1(A.E, A.H, A.I)).name;
     }
-    bool tyB = A.layers_h != nullptr;
-    for (int l = A.layer0; tyB && l < A.layer0 + A.nlayers; l++) {
-        const DecLayer *Lh = A.layers_h + l;
-        tyB = !Lh->q6[0] && !Lh->q6[1] && Lh->q6[2] && !Lh->sq6[0] && !Lh->sq6[1] && Lh->sq6[2];
-    }
-    if (tyB && dec_layerB_ok(A.E, A.H, A.I, A.B))
-        return A.B <= 2 ? "dec_stackB2_kernel" : A.B <= 4 ? "dec_stackB4_kernel" : "dec_stackB8_kernel";
+    if (dec_layerB_ok(A.E, A.H, A.I, A.B))
+        if (const char *name = stackB_choice(A, A.layer0, A.nlayers).name) return name;
     return A.B == 1 ? "dec_router1_kernel + dec_gu1_kernel + dec_down_kernel per layer"
                     : "dec_router_kernel + dec_gu_kernel + dec_down_kernel per layer";
 }
