@@ -71,6 +71,7 @@ struct DecArgs {
     /* kernel_ffn_fused mode */
     const DecActive *ffn_ex;    /* [n] device */
     int ffn_n;
+    int ffn_d;                  /* 1 = every down matrix Q4_K, 2 = every one Q6_K, 0 = mixed */
     float *ffn_out;             /* [n x H] or NULL */
     /* one-launch stack (dec_stack1_kernel): exchange slots, u64 = (epoch << 32) | f32 bits */
     uint64_t *xch;              /* [XCH_U64(E, H, I)] or NULL (then the three-kernel path runs) */
@@ -165,6 +166,10 @@ struct DecXch { uint64_t *p; size_t n; uint32_t epoch; };
  * the library's own scratch and control words are used. */
 int dec_launch(DecArgs &A);
 int dec_ffn_launch(DecArgs &A);      /* kernel_ffn_fused: gate/up + down kernels */
+/* Its input: n bytes (whole 16-byte units readable) of pinned host memory at
+ * src to device memory at dst on the library stream; *eout (pinned) gets the
+ * error bits of the calls before it. */
+int dec_ffn_stage(const void *src, void *dst, size_t n, int *eout);
 /* Whether one token's layers can run as one launch (dec_stack1_kernel) for
  * these shapes on this device. */
 bool dec_layer1_ok(int E, int H, int I, int B);

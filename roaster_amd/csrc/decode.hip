@@ -540,22 +540,25 @@ __device__ void build_plan(const DecArgs &A, const DecLayer &L, DecPlan &P, cons
     plan_from_ids(A, L, P, sg, emask);
 }
 
+/* kernel_ffn_fused's plan: thread k takes expert k (one round trip for the
+ * table; one thread walking it took nine). */
 __device__ void ffn_plan(const DecArgs &A, DecPlan &P)
 {
-    if (threadIdx.x == 0) {
+    const int k = threadIdx.x;
+    if (k == 0) {
         P.nact = A.ffn_n;
         P.nroute = A.ffn_n;
         P.err = 0;
-        for (int k = 0; k < A.ffn_n; k++) {
-            P.a[k] = A.ffn_ex[k];
-            P.a[k].ntok = 1;
-            P.a[k].tk[0] = k;
-        }
-        for (int k = 0; k < 9; k++) {
-            P.dsl[0][k] = k < A.ffn_n ? A.ffn_ex[k].d : NULL;
-            P.dq6k[k] = k < A.ffn_n ? A.ffn_ex[k].dq6 : 0;
-            P.w[0][k] = 0.0f;
-        }
+    }
+    if (k < 9) {
+        const bool in = k < A.ffn_n;
+        DecActive X = A.ffn_ex[in ? k : 0];
+        X.ntok = 1;
+        X.tk[0] = k;
+        if (in) P.a[k] = X;
+        P.dsl[0][k] = in ? X.d : NULL;
+        P.dq6k[k] = in ? X.dq6 : 0;
+        P.w[0][k] = 0.0f;
     }
     __syncthreads();
 }
@@ -902,11 +905,11 @@ __device__ __forceinline__ void down_one_token(const DecArgs &A, int dr, float *
     const int ca = lb * RQK + q_run_a<D6>(c), cb = ca + q_run_b_off<D6>();
     const DecPlan *PG = A.plan_g;
     /* the residual of this thread's output row (stack mode), read first */
-    const float hv = A.y ? 0.0f : A.h[min(r0 + min(tid, dr - 1), H - 1)];
+    const float hv = A.y || A.ffn_out ? 0.0f : A.h[min(r0 + min(tid, dr - 1), H - 1)];
     const uint8_t *mp[D_PF];
 #pragma unroll
     for (int f = 0; f < D_PF; f++) mp[f] = PG->dsl[0][min(wv + f * DW, ntask - 1) / ngroups];
-    const uint8_t *fb = PG->dsl[0][8];
+    const uint8_t *fb = PG->dsl[0][A.ffn_out ? 0 : 8];   /* always set */
     const float wk = PG->w[0][min(tid, 8)];
     /* the SiLU*up rows: 9 x I / 4 16-byte units, 5 per thread (I <= 568), in
      * named registers (an array here is not kept in registers across the
@@ -954,6 +957,13 @@ __device__ __forceinline__ void down_one_token(const DecArgs &A, int dr, float *
     }
     __syncthreads();
     PHASE_TS(2, 2);
+    if (A.ffn_out) {                    /* kernel_ffn_fused: per-expert outputs */
+        for (int idx = tid; idx < A.ffn_n * dr; idx += DT) {
+            const int k = idx / dr, rl = idx % dr, row = r0 + rl;
+            if (row < H) A.ffn_out[(size_t)k * H + row] = dbuf[k * D_MAXR + rl];
+        }
+        return;
+    }
     for (int rl = tid; rl < dr; rl += DT) {
         const int row = r0 + rl;
         if (row >= H) continue;
@@ -2916,9 +2926,10 @@ static int launch_layer(const DecArgs &A0, int l, bool with_router)
     const DecLayer *Lh = A.layers_h ? A.layers_h + l : nullptr;
     const int rpw1 = 64 / lanes_per_row(A.I / RQK);
     A.d1 = 0;
-    if (A.B == 1 && !A.ffn_out && Lh && Lh->q6[2] == Lh->sq6[2] && 9 * ((D_ROWS + rpw1 - 1) / rpw1) <= DW * D_PF &&
-        9 * A.I / 4 <= 5 * DT)
-        A.d1 = Lh->q6[2] ? 2 : 1;
+    if (A.B == 1 && 9 * ((D_ROWS + rpw1 - 1) / rpw1) <= DW * D_PF && 9 * A.I / 4 <= 5 * DT) {
+        if (A.ffn_out) A.d1 = A.ffn_d;
+        else if (Lh && Lh->q6[2] == Lh->sq6[2]) A.d1 = Lh->q6[2] ? 2 : 1;
+    }
     const size_t lds = norm_lds(A.B, A.H);
     if (with_router) {
         const int ntask = (A.logits_in ? 0 : A.E) + 1 + A.I;
@@ -3252,6 +3263,27 @@ int dec_launch(DecArgs &A)
     for (int l = A.layer0; l < A.layer0 + A.nlayers; l++)
         if (int rc = launch_layer(A, l, true)) return rc;
     return 0;
+}
+
+/* kernel_ffn_fused's input staging: n16 16-byte units of pinned host memory
+ * into device memory, and the library's error words (either may be NULL) as
+ * they stand before the call's kernels, into pinned host memory. */
+extern "C" __global__ void __launch_bounds__(1024) ffn_stage_kernel(const uint4 *src, uint4 *dst, int n16, const int *e0,
+                                                                    const int *e1, int *eout)
+{
+    const int t = (int)(blockIdx.x * 1024 + threadIdx.x);
+    if (t < n16) dst[t] = src[t];
+    if (t == 0) *eout = (e0 ? *e0 : 0) | (e1 ? *e1 : 0);
+}
+
+int dec_ffn_stage(const void *src, void *dst, size_t n, int *eout)
+{
+    const int n16 = (int)((n + 15) / 16);
+    int *w[2];
+    rt_err_words(w);
+    hipLaunchKernelGGL(ffn_stage_kernel, dim3((n16 + 1023) / 1024), dim3(1024), 0, rt().stream, (const uint4 *)src,
+                       (uint4 *)dst, n16, (const int *)w[0], (const int *)w[1], eout);
+    return rt_check(hipGetLastError(), "input staging launch") ? ROASTER_EDEVICE : 0;
 }
 
 int dec_ffn_launch(DecArgs &A)

@@ -109,12 +109,19 @@ unsigned *rt_ctrl()
     return g_ctrl;
 }
 
+void rt_err_words(int *(&w)[2])
+{
+    w[0] = g_ctrl ? (int *)(g_ctrl + 16) : NULL;
+    w[1] = g_aux_used ? g_aux_err : NULL;
+}
+
 int rt_take_err()
 {
     /* the error words come back with the stream's last work: copies queued
      * behind it into pinned memory, then one synchronisation (two blocking
      * copies cost about 20 us per call) */
-    int *words[2] = { g_ctrl ? (int *)(g_ctrl + 16) : NULL, g_aux_used ? g_aux_err : NULL };
+    int *words[2];
+    rt_err_words(words);
     g_aux_used = false;
     if (!g_err_pin && (words[0] || words[1]) &&
         rt_check(hipHostMalloc((void **)&g_err_pin, 64, hipHostMallocDefault), "error word hipHostMalloc")) {
