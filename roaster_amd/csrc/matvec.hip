@@ -14,6 +14,7 @@
 #include "internal.h"
 #include "qdot.h"
 #include "matvec.h"
+#include "pf_tile.h"
 
 #include <type_traits>
 
@@ -64,15 +65,65 @@ __global__ void __launch_bounds__(MV_THREADS) matvec_jobs_kernel(const MvJob *jo
  * super-block, lanes_per_row(blocks) lanes per row, 64 / lpr rows per wave pass).
  * Each lane's activation runs are fixed for every row it serves: with one
  * token they sit in registers for the whole kernel, with more in LDS.  Every
- * wave keeps DMV_PF row passes' loads in flight before it computes them. */
-#ifndef DMV_PF
-#define DMV_PF 2                           /* row passes in flight per wave */
-#endif
-#ifndef DMV_GRID
-#define DMV_GRID 8                         /* workgroups per CU at most */
-#endif
-
+ * wave keeps the next row pass's loads in flight while it computes one. */
 static int g_dense_mfma_t = 2;             /* tokens from which dense_mm8_kernel serves a call */
+
+/* 16 (8) bytes at a 2-byte aligned address as the aligned dwords around them;
+ * shift 0 or 16 brings them back.  A vector load that is not 4-byte aligned
+ * is split by the memory pipe: the LM head (Q6_K [248320 x 2048], one token)
+ * took 109 us with 2-byte aligned loads and takes 104 with these. */
+struct U5 { uint4 v; uint32_t w; };
+
+__device__ __forceinline__ U5 gld_5(const uint8_t *p)    /* p 4-byte aligned */
+{
+    typedef gu32x4 __attribute__((aligned(4))) gu32x4_a4;
+    const gu32x4 v = *(const GAS gu32x4_a4 *)p;
+    U5 r;
+    r.v = make_uint4(v.x, v.y, v.z, v.w);
+    r.w = gld_u32(p + 16);
+    return r;
+}
+
+__device__ __forceinline__ uint4 u5_fix(const U5 &a, uint32_t sh)
+{
+    return make_uint4(__builtin_amdgcn_alignbit(a.v.y, a.v.x, sh), __builtin_amdgcn_alignbit(a.v.z, a.v.y, sh),
+                      __builtin_amdgcn_alignbit(a.v.w, a.v.z, sh), __builtin_amdgcn_alignbit(a.w, a.v.w, sh));
+}
+
+/* A lane's chunk as loaded (q_load's bytes) and the QChunk it stands for. */
+template <bool Q6> struct QRaw;
+template <> struct QRaw<false> {
+    QChunk ch;
+    __device__ __forceinline__ void load(const uint8_t *blk, int c) { ch = q_load<false>(blk, c); }
+    __device__ __forceinline__ QChunk chunk() const { return ch; }
+};
+template <> struct QRaw<true> {
+    U5 q, h;
+    uint32_t s[3], dd, sh;
+    __device__ __forceinline__ void load(const uint8_t *blk, int c)
+    {
+        const uint8_t *al = (const uint8_t *)((uintptr_t)blk & ~(uintptr_t)3);
+        const int n = c >> 2, p = c & 3;
+        sh = ((uint32_t)(uintptr_t)blk & 2u) * 8u;
+        q = gld_5(al + 16 * c);
+        h = gld_5(al + 128 + 32 * n + 16 * (p & 1));
+        typedef gu32x2 __attribute__((aligned(4))) gu32x2_a4;
+        const gu32x2 v = *(const GAS gu32x2_a4 *)(al + 192 + 8 * n);
+        s[0] = v.x;
+        s[1] = v.y;
+        s[2] = gld_u32(al + 192 + 8 * n + (sh ? 8 : 4));    /* not past the block's end */
+        dd = gld_u16(blk + 208);
+    }
+    __device__ __forceinline__ QChunk chunk() const
+    {
+        QChunk ch;
+        ch.q = u5_fix(q, sh);
+        ch.h = u5_fix(h, sh);
+        ch.s = make_uint2(__builtin_amdgcn_alignbit(s[1], s[0], sh), __builtin_amdgcn_alignbit(s[2], s[1], sh));
+        ch.dd = dd;
+        return ch;
+    }
+};
 
 template <bool Q6, bool ONE, int KB>
 __global__ void __launch_bounds__(MV_THREADS) dense_mv_kernel(const uint8_t *W, const float *X, float *Y, int rows,
@@ -116,346 +167,363 @@ __global__ void __launch_bounds__(MV_THREADS) dense_mv_kernel(const uint8_t *W, 
     }
     const int gw = blockIdx.x * (MV_THREADS / 64) + (threadIdx.x >> 6), nw = gridDim.x * (MV_THREADS / 64);
     const int npass = (rows + rpw - 1) / rpw;
-    for (int p0 = gw; p0 < npass; p0 += nw * DMV_PF) {
-        QChunk ch[DMV_PF][KB];
+    /* the next pass's chunks are in flight while the current one's are dotted;
+     * rows and blocks past the end read the last one, unused, so that the loads
+     * carry no branches and each wait counts its own loads only */
+    QRaw<Q6> cur[KB], nxt[KB];
+    auto load = [&](QRaw<Q6> (&ch)[KB], int pass) {
+        const int row = min(min(pass, npass - 1) * rpw + rw, rows - 1);
 #pragma unroll
-        for (int f = 0; f < DMV_PF; f++) {
-            const int row = (p0 + f * nw) * rpw + rw;
+        for (int k = 0; k < KB; k++)
+            ch[k].load(W + (size_t)row * row_bytes + (size_t)min(lb + 8 * k, nb - 1) * bs, c);
+    };
+    auto compute = [&](const QRaw<Q6> (&ch)[KB], int pass) {
+        const int row = pass * rpw + rw;
+        const bool live = row < rows;
+        QChunk qc[KB];
 #pragma unroll
-            for (int k = 0; k < KB; k++)
-                if (blk_live[k] && row < rows)
-                    ch[f][k] = q_load<Q6>(W + (size_t)row * row_bytes + (size_t)(lb + 8 * k) * bs, c);
-        }
+        for (int k = 0; k < KB; k++) qc[k] = ch[k].chunk();
+        for (int t = 0; t < (ONE ? 1 : T); t++) {
+            float part = 0.0f;
 #pragma unroll
-        for (int f = 0; f < DMV_PF; f++) {
-            const int pass = p0 + f * nw;
-            if (pass >= npass) break;
-            const int row = pass * rpw + rw;
-            const bool live = row < rows;
-            for (int t = 0; t < (ONE ? 1 : T); t++) {
-                float part = 0.0f;
-#pragma unroll
-                for (int k = 0; k < KB; k++) {
-                    if (live && blk_live[k]) {
-                        if (ONE) {
-                            part += q_chunk_dot_r<Q6>(ch[f][k], c, xa[k], xb[k], sxa[k], sxb[k]);
-                        } else {
-                            const float *x = xs + (size_t)t * cols, *sx = xsum + (size_t)t * (cols / 16);
-                            part += q_chunk_dot<Q6>(ch[f][k], c, x + ca[k], x + cb[k], sx[ca[k] >> 4], sx[cb[k] >> 4]);
-                        }
+            for (int k = 0; k < KB; k++) {
+                if (live && blk_live[k]) {
+                    if (ONE) {
+                        part += q_chunk_dot_r<Q6>(qc[k], c, xa[k], xb[k], sxa[k], sxb[k]);
+                    } else {
+                        const float *x = xs + (size_t)t * cols, *sx = xsum + (size_t)t * (cols / 16);
+                        part += q_chunk_dot<Q6>(qc[k], c, x + ca[k], x + cb[k], sx[ca[k] >> 4], sx[cb[k] >> 4]);
                     }
                 }
-                part = group_sum_w(part, lpr);
-                if (live && lr == 0) Y[(size_t)t * rows + row] = part;
             }
+            part = group_sum_w(part, lpr);
+            if (live && lr == 0) Y[(size_t)t * rows + row] = part;
         }
+    };
+    if (gw >= npass) return;
+    load(cur, gw);
+    if (gw + nw >= npass) {                              /* this wave's only pass */
+        compute(cur, gw);
+        return;
+    }
+    for (int p = gw; p < npass; p += 2 * nw) {
+        load(nxt, p + nw);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(cur, p);
+        if (p + nw >= npass) break;
+        load(cur, p + 2 * nw);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(nxt, p + nw);
     }
 }
 
-/* ---- 2..8 tokens on MFMA -----------------------------------------------------
- * y[t][r] = W[r] . x[t] with the quants as MFMA operands and the block scales
- * applied in f32 per scale sub-block (the reference's fold, kernels.c:
- * 1844-1874: d sc sum(q x) - dmin m sum(x) for Q4_K, d sc sum(q x) -
- * 32 d sc sum(x) for Q6_K):
- *   B = 16 weight rows x one scale sub-block (Q4_K: 32 weights on
- *       v_mfma_f32_16x16x32_f16, Q6_K: 16 on v_mfma_f32_16x16x16f16); each
- *       quant q enters as the fp16 bit pattern q, i.e. q * 2^-24 (a
- *       denormal, exact), one mask per pair;
- *   A = the tokens' activations of the super-block, scaled per (token,
- *       super-block) by a power of two (max |x| in [2^14, 2^15)) and split
- *       into fp16 hi + lo, row m = 2t + (lo);
- *   C = per-sub-block sums p: lane l holds weight row l % 16 and tokens
- *       2(l / 16), 2(l / 16) + 1 (hi and lo rows) and accumulates
- *       z += (2^24 d sc)(p_hi + p_lo) - (dmin m) X_s over the super-block's
- *       sub-blocks (X_s: the sub-block's scaled activation sum, f32), then
- *       y += 2^-e z.
- * x = hi + lo keeps 22 of the 24 bits of an f32 activation; products and
- * sums are f32.  mm8_prep_kernel builds the A operands once per call, in
- * fragment order (lane l's 8 / 4 halves contiguous; inside a sub-block the
- * K order follows the quant pairs the masks produce, bytes 0, 2, 1, 3 of each
- * dword); every workgroup of dense_mm8_kernel copies them into LDS, and each
- * wave streams 16-row groups, the next super-block's raw quants in flight
- * while the current one computes. */
+/* ---- tokens on MFMA -----------------------------------------------------------
+ * y[t][r] = W[r] . x[t] with 16 weight rows per wave on
+ * v_mfma_f32_16x16x32_f16 and the block's integer part as the operand, which
+ * fp16 holds exactly:
+ *   B = 16 rows x 32 columns: Q4_K sc q (at most 945), Q6_K sc (q - 32) with
+ *       what its rounding to 11 bits drops (above 2048 in magnitude) as a
+ *       second operand; lane l holds row l % 16 and 8 columns of its run;
+ *   A = the tokens' activations, scaled per (token, super-block) by a power of
+ *       two (max |x| in [2^14, 2^15)) and split into fp16 parts: up to 4 tokens
+ *       three parts (every bit of an f32), rows 4 t + part, 5..8 tokens two
+ *       (22 bits), rows 2 t + part, so that the accumulators of lane l are the
+ *       parts of token l / 16 (of tokens 2 (l / 16), + 1) and add up in the
+ *       lane;
+ *   d, the scale's inverse and (Q4_K) dmin times the sub-block minima's
+ *       product with the sub-block sums (one more MFMA: minima 2 g, 2 g + 1 in
+ *       lane group g) are applied in f32 once per super-block
+ * (the reference's fold, kernels.c:1844-1874: d sc sum(q x) - dmin m sum(x),
+ * d sc sum((q - 32) x)).  Every workgroup prepares A in LDS itself while its
+ * first weights are on the way; each wave streams 16-row groups, the next
+ * super-block's quants in flight while one computes. */
 #define MM8_T 512
 #define MM8_W (MM8_T / 64)
 
-typedef _Float16 mm_f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 mm_f16x4 __attribute__((ext_vector_type(4)));
-typedef float mm_f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uint32_t gld_u32a2(const void *p)
-{
-    typedef uint32_t __attribute__((aligned(2))) u32_a2;
-    return *(const GAS u32_a2 *)p;
-}
-
-/* Operand buffer of one call: A fragments [cols / SB][64 lanes] (cols * 32
- * bytes), sub-block sums xs [cols / SB][8 tokens], super-block scales
- * ge [cols / 256][8 tokens] (2^-e). */
+/* LDS of one call: A fragments [cols / 256][8][64 lanes] (16 bytes), sub-block
+ * sums [cols / 256][64 lanes] (2 fp16), scales [cols / 256][8 tokens] (2^-e). */
 __host__ __device__ static inline size_t mm8_frag_bytes(size_t cols) { return cols * 32; }
-__host__ __device__ static inline size_t mm8_xs_bytes(size_t cols, int q6) { return cols / (q6 ? 16 : 32) * 8 * 4; }
-__host__ __device__ static inline size_t mm8_buf_bytes(size_t cols, int q6) { return mm8_frag_bytes(cols) + mm8_xs_bytes(cols, q6) + cols / RQK * 8 * 4; }
+__host__ __device__ static inline size_t mm8_sum_bytes(size_t cols) { return cols; }
+__host__ __device__ static inline size_t mm8_lds_bytes(size_t cols) { return mm8_frag_bytes(cols) + mm8_sum_bytes(cols) + cols / RQK * 8 * 4; }
 
-/* Workgroup kb (256 threads): thread (t = tid / 32, c = tid % 32) holds
- * columns 256 kb + 8c .. + 7 of token t; it writes both halves (hi, lo) of
- * every fragment slot those columns fill, and sub-block sums are reduced
- * over the 4 (Q4_K) or 2 (Q6_K) threads of a sub-block. */
-template <bool Q6>
-__global__ void __launch_bounds__(256) mm8_prep_kernel(const float *X, int cols, int T, uint8_t *buf)
+/* Super-block kb of the activations into LDS (one wave): lane (t = l / 8, c =
+ * l % 8) takes columns 32 c .. + 31 of token t. */
+template <bool Q6, int PARTS>
+__device__ __forceinline__ void mm8_prep(const float *X, int cols, int T, int kb, uint8_t *lds, int lane)
 {
-    constexpr int SB = Q6 ? 16 : 32, FB = Q6 ? 512 : 1024;
-    const int kb = blockIdx.x, tid = threadIdx.x, t = tid >> 5, c = tid & 31;
-    const int ns = cols / SB;
-    uint8_t *frag = buf;
-    float *xs = (float *)(buf + mm8_frag_bytes(cols));
-    float *ge = xs + (size_t)ns * 8;
-    float4 v0 = make_float4(0.f, 0.f, 0.f, 0.f), v1 = v0;
-    if (t < T) {
-        const float *xp = X + (size_t)t * cols + RQK * kb + 8 * c;
-        v0 = gld_f4(xp);
-        v1 = gld_f4(xp + 4);
-    }
-    float mx = fmaxf(fmaxf(fmaxf(fabsf(v0.x), fabsf(v0.y)), fmaxf(fabsf(v0.z), fabsf(v0.w))),
-                     fmaxf(fmaxf(fabsf(v1.x), fabsf(v1.y)), fmaxf(fabsf(v1.z), fabsf(v1.w))));
+    const int t = lane >> 3, c = lane & 7;
+    /* lane group g's columns in slice f follow its 16-byte runs of quants
+     * (mm8_load): Q6_K 64 (f / 2) + 16 g + 8 (f % 2) .. + 7, Q4_K 128 (f / 4) +
+     * 64 (g / 2) + 32 ((f / 2) % 2) + 16 (g % 2) + 8 (f % 2) .. + 7 */
+    f16x8 *frag = (f16x8 *)lds + (size_t)kb * 512 +
+                  (Q6 ? 128 * (c >> 1) + 32 * (c & 1) : 256 * (c >> 2) + 128 * (c & 1) + 32 * ((c >> 1) & 1));
+    f16x2 *sums = (f16x2 *)(lds + mm8_frag_bytes(cols)) + kb * 64;
+    float *ge = (float *)(lds + mm8_frag_bytes(cols) + mm8_sum_bytes(cols)) + kb * 8;
+    if (t >= T) return;
+    const float *xp = X + (size_t)t * cols + RQK * kb + 32 * c;
+    float4 v[8];
 #pragma unroll
-    for (int o = 16; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 32));
+    for (int i = 0; i < 8; i++) v[i] = gld_f4(xp + 4 * i);
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
+    mx = fmaxf(mx, dpp_f<DPP_XOR1>(mx));
+    mx = fmaxf(mx, dpp_f<DPP_XOR2>(mx));
+    mx = fmaxf(mx, dpp_f<DPP_HALF_MIRROR>(mx));
     int e = 0;
     if (mx > 0.0f && mx <= 3.0e38f) {
         int E;
         (void)frexpf(mx, &E);
         e = min(max(15 - E, -100), 100);
     }
-    if (c == 0) ge[kb * 8 + t] = ldexpf(1.0f, -e);
-    const float w8[8] = {ldexpf(v0.x, e), ldexpf(v0.y, e), ldexpf(v0.z, e), ldexpf(v0.w, e),
-                         ldexpf(v1.x, e), ldexpf(v1.y, e), ldexpf(v1.z, e), ldexpf(v1.w, e)};
-    _Float16 hi[8], lo[8];
+    const float up = ldexpf(1.0f, e);
+    if (c == 0) ge[t] = ldexpf(1.0f, -e);
+    const int row = PARTS == 3 ? 4 * t : 2 * t;
+    float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        hi[i] = (_Float16)w8[i];
-        lo[i] = (_Float16)(w8[i] - (float)hi[i]);
+    for (int g = 0; g < 4; g++) {
+        f32x8 w = { v[2 * g].x, v[2 * g].y, v[2 * g].z, v[2 * g].w, v[2 * g + 1].x, v[2 * g + 1].y, v[2 * g + 1].z, v[2 * g + 1].w };
+        w = w * up;
+        sum += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+#pragma unroll
+        for (int p = 0; p < PARTS; p++) {
+            const f16x8 h = __builtin_convertvector(w, f16x8);
+            frag[64 * (g & 1) + 16 * (g >> 1) + row + p] = h;
+            w = w - __builtin_convertvector(h, f32x8);
+        }
     }
-    float sum = ((w8[0] + w8[1]) + (w8[2] + w8[3])) + ((w8[4] + w8[5]) + (w8[6] + w8[7]));
-    if (!Q6) {
-        /* sub-block s = c / 4 of this super-block, lane group j = c % 4: slots
-         * 0..7 = columns 0, 2, 1, 3, 4, 6, 5, 7 */
-        const int f = kb * 8 + (c >> 2), j = c & 3;
-        const mm_f16x8 h8 = {hi[0], hi[2], hi[1], hi[3], hi[4], hi[6], hi[5], hi[7]};
-        const mm_f16x8 l8 = {lo[0], lo[2], lo[1], lo[3], lo[4], lo[6], lo[5], lo[7]};
-        if (t < 8) {
-            *(mm_f16x8 *)(frag + (size_t)f * FB + (16 * j + 2 * t) * 16) = h8;
-            *(mm_f16x8 *)(frag + (size_t)f * FB + (16 * j + 2 * t + 1) * 16) = l8;
-        }
-        sum += __shfl_xor(sum, 1, 32);
-        sum += __shfl_xor(sum, 2, 32);
-        if (j == 0) xs[f * 8 + t] = sum;
-    } else {
-        /* sub-block s = c / 2, lane groups j = 2 (c % 2) and + 1, 4 columns
-         * each: slots 0..3 = columns 0, 2, 1, 3 */
-        const int f = kb * 16 + (c >> 1), j0 = 2 * (c & 1);
+    /* sub-block c's sum, in lane group c / 2's slot c % 2 */
+    sum *= 0.015625f;
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const mm_f16x4 h4 = {hi[4 * u], hi[4 * u + 2], hi[4 * u + 1], hi[4 * u + 3]};
-            const mm_f16x4 l4 = {lo[4 * u], lo[4 * u + 2], lo[4 * u + 1], lo[4 * u + 3]};
-            *(mm_f16x4 *)(frag + (size_t)f * FB + (16 * (j0 + u) + 2 * t) * 8) = h4;
-            *(mm_f16x4 *)(frag + (size_t)f * FB + (16 * (j0 + u) + 2 * t + 1) * 8) = l4;
-        }
-        sum += __shfl_xor(sum, 1, 32);
-        if ((c & 1) == 0) xs[f * 8 + t] = sum;
+    for (int p = 0; p < PARTS; p++) {
+        const _Float16 h = (_Float16)sum;
+        ((_Float16 *)(sums + 16 * (c >> 1) + row + p))[c & 1] = h;
+        sum -= (float)h;
     }
 }
 
-struct Mm8Q4 { uint4 hd; uint2 p[4]; };              /* header; qs bytes 32g + 8j .. + 7 */
-struct Mm8Q6 { uint32_t L[8], Hq[4]; uint4 sc; uint32_t d; };
+/* Lane group g's share of a super-block: 16-byte runs, so that the four lanes
+ * of a row read 64 contiguous bytes a load (8-byte runs, 32 bytes a load,
+ * measured 121 us on the LM head with five tokens where these take XXX).
+ * Q4_K: qs bytes 64 k + 16 g (sub-blocks 4 k + 2 (g / 2), + 1); Q6_K, by half n:
+ * ql bytes 64 n + 16 g (scales 8 n + g, + 4) and the qh bytes under them. */
+struct Mm8Q4 { uint4 hd, p[2]; };
+struct Mm8Q6 { U5 l[2], h[2], sc; uint32_t d, sh; };
 
-__device__ __forceinline__ void mm8_load(Mm8Q4 &r, const uint8_t *blk, int j)
+__device__ __forceinline__ void mm8_load(Mm8Q4 &r, const uint8_t *blk, int g)
 {
     r.hd = gld_u4(blk);
 #pragma unroll
-    for (int g = 0; g < 4; g++) r.p[g] = gld_u2(blk + 16 + 32 * g + 8 * j);
+    for (int k = 0; k < 2; k++) r.p[k] = gld_u4(blk + 16 + 64 * k + 16 * g);
 }
 
-/* Q6_K sub-block s (weights 16 s .. 16 s + 15; n = s / 8, q = (s % 8) / 2,
- * hb = s % 2, kernels.c:449-468): lane j's 4 quants are the nibble q / 2 of
- * ql dword L[4 n + 2 (q % 2) + hb] (bytes 64 n + 32 (q % 2) + 16 hb + 4 j ..)
- * with bits 2 q of qh dword Hq[2 n + hb] (bytes 128 + 32 n + 16 hb + 4 j ..). */
-__device__ __forceinline__ void mm8_load(Mm8Q6 &r, const uint8_t *blk, int j)
+__device__ __forceinline__ void mm8_load(Mm8Q6 &r, const uint8_t *blk, int g)
 {
+    const uint8_t *al = (const uint8_t *)((uintptr_t)blk & ~(uintptr_t)3);
+    r.sh = ((uint32_t)(uintptr_t)blk & 2u) * 8u;
 #pragma unroll
-    for (int n = 0; n < 2; n++)
-#pragma unroll
-        for (int q = 0; q < 2; q++)
-#pragma unroll
-            for (int hb = 0; hb < 2; hb++) r.L[4 * n + 2 * q + hb] = gld_u32a2(blk + 64 * n + 32 * q + 16 * hb + 4 * j);
-#pragma unroll
-    for (int n = 0; n < 2; n++)
-#pragma unroll
-        for (int hb = 0; hb < 2; hb++) r.Hq[2 * n + hb] = gld_u32a2(blk + 128 + 32 * n + 16 * hb + 4 * j);
-    r.sc = gld_u4a2(blk + 192);
+    for (int n = 0; n < 2; n++) {
+        r.l[n] = gld_5(al + 64 * n + 16 * g);
+        r.h[n] = gld_5(al + 128 + 32 * n + 16 * (g & 1));
+    }
+    typedef gu32x4 __attribute__((aligned(4))) gu32x4_a4;
+    const gu32x4 v = *(const GAS gu32x4_a4 *)(al + 192);
+    r.sc.v = make_uint4(v.x, v.y, v.z, v.w);
+    r.sc.w = gld_u32(al + (r.sh ? 208 : 204));
     r.d = gld_u16(blk + 208);
 }
 
-/* Super-block kb of one 16-row group: 8 (Q4_K) or 16 (Q6_K) MFMAs; z0 / z1
- * accumulate tokens 2 (l / 16) and + 1 of row l % 16.  frag: this
- * super-block's A fragments, xs: its sub-block sums [sub][8 tokens]. */
-__device__ __forceinline__ void mm8_block(const Mm8Q4 &r, const uint8_t *frag, const float *xs, int lane, float &z0,
-                                          float &z1)
+__device__ __forceinline__ uint32_t u4_word(const uint4 &v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+
+/* Scale / minimum j (a byte offset of 0..2 with j + 1 in the same half) and
+ * the next of a lane group whose sub-blocks lie in the header's lower (lo) or
+ * upper half; sh = 8 j. */
+__device__ __forceinline__ uint32_t q4_pair6(uint32_t own, uint32_t s811, int nib, int sh, bool lo)
 {
-    const float d = f16_bits_to_f32(r.hd.x & 0xFFFFu) * 16777216.0f, dmin = f16_bits_to_f32(r.hd.x >> 16);
+    const uint32_t a = own >> sh, b = s811 >> (sh + nib);
+    const uint32_t x = a & 0x3F3Fu, y = (b & 0x0F0Fu) | ((a >> 2) & 0x3030u);
+    return lo ? x : y;                                   /* bytes 0 and 1 */
+}
+
+/* z: the integer products of one super-block; zm: the minima's (Q4_K). */
+__device__ __forceinline__ void mm8_block(const Mm8Q4 &r, const uint8_t *frag, const uint8_t *sums, int lane, f32x4 (&z)[2],
+                                          f32x4 &zm)
+{
     const uint32_t s03 = r.hd.y, s47 = r.hd.z, s811 = r.hd.w;
-    const int t0 = 2 * (lane >> 4);
+    const int g = lane >> 4;
+    {
+        /* minima 2 g, 2 g + 1 of lane group g against the sums of those sub-blocks */
+        const uint32_t m = q4_pair6(s47, s811, 4, 16 * (g & 1), g < 2);
+        const _Float16 o = (_Float16)0.0f;
+        const f16x8 mb = { (_Float16)(int)(m & 0xFF), (_Float16)(int)(m >> 8), o, o, o, o, o, o };
+        const f16x2 xs = *(const f16x2 *)(sums + 4 * lane);
+        const f16x8 xa = { xs[0], xs[1], o, o, o, o, o, o };
+        zm = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa, mb, (f32x4){}, 0, 0, 0);
+    }
+    z[0] = z[1] = (f32x4){};
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const int g = s >> 1, hi = s & 1;
-        int sc, m;
-        if (s < 4) {
-            sc = byte_of(s03, s) & 63;
-            m = byte_of(s47, s) & 63;
-        } else {
-            sc = (byte_of(s811, s - 4) & 15) | ((byte_of(s03, s - 4) >> 6) << 4);
-            m = (byte_of(s811, s - 4) >> 4) | ((byte_of(s47, s - 4) >> 6) << 4);
+    for (int k = 0; k < 2; k++) {
+        /* sub-blocks 4 k + 2 (g / 2) (low nibbles) and + 1 (high) */
+        const uint32_t scs = q4_pair6(s03, s811, 0, 16 * (g >> 1), k == 0);
+#pragma unroll
+        for (int hi = 0; hi < 2; hi++) {
+            const _Float16 sf = (_Float16)(int)(hi ? scs >> 8 : scs & 0xFF);
+            const f16x2 scv = { sf, sf };
+            const f16x2 bias = scv * (f16x2){ (_Float16)-1024.0f, (_Float16)-1024.0f };   /* exact: 63 * 1024 < 65504 */
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const uint32_t p = u4_word(r.p[k], 2 * i), q = u4_word(r.p[k], 2 * i + 1);
+                const uint32_t x = (hi ? p >> 4 : p) & 0x0F0F0F0Fu, y = (hi ? q >> 4 : q) & 0x0F0F0F0Fu;
+                const f16x2 w0 = __builtin_elementwise_fma(magic_lo(x), scv, bias), w1 = __builtin_elementwise_fma(magic_hi(x), scv, bias);
+                const f16x2 w2 = __builtin_elementwise_fma(magic_lo(y), scv, bias), w3 = __builtin_elementwise_fma(magic_hi(y), scv, bias);
+                const f16x8 b = { w0[0], w0[1], w1[0], w1[1], w2[0], w2[1], w3[0], w3[1] };
+                const f16x8 a = *(const f16x8 *)(frag + (4 * k + 2 * hi + i) * 1024 + lane * 16);
+                z[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, z[i], 0, 0, 0);
+            }
         }
-        const uint32_t x = r.p[g].x >> (4 * hi), y = r.p[g].y >> (4 * hi);
-        const uint4 bq = make_uint4(x & 0x000F000Fu, (x >> 8) & 0x000F000Fu, y & 0x000F000Fu, (y >> 8) & 0x000F000Fu);
-        const mm_f16x8 b = __builtin_bit_cast(mm_f16x8, bq);
-        const mm_f16x8 a = *(const mm_f16x8 *)(frag + s * 1024 + lane * 16);
-        const mm_f32x4 cc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, (mm_f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-        const float2 xm = *(const float2 *)(xs + s * 8 + t0);
-        const float sa = d * (float)sc, ma = dmin * (float)m;
-        z0 = fmaf(sa, cc[0] + cc[1], z0);
-        z0 = fmaf(-ma, xm.x, z0);
-        z1 = fmaf(sa, cc[2] + cc[3], z1);
-        z1 = fmaf(-ma, xm.y, z1);
     }
 }
 
-__device__ __forceinline__ void mm8_block(const Mm8Q6 &r, const uint8_t *frag, const float *xs, int lane, float &z0,
-                                          float &z1)
+__device__ __forceinline__ void mm8_block(const Mm8Q6 &r, const uint8_t *frag, const uint8_t *, int lane, f32x4 (&z)[2], f32x4 &)
 {
-    const float d = f16_bits_to_f32(r.d) * 16777216.0f;
-    const int t0 = 2 * (lane >> 4);
+    const int g = lane >> 4, qs = 2 * (g >> 1);             /* qh bits of the low nibbles' columns */
+    const f16x2 off = { (_Float16)-1056.0f, (_Float16)-1056.0f };
+    z[0] = z[1] = (f32x4){};
+    const uint4 scv = u5_fix(r.sc, r.sh);
 #pragma unroll
-    for (int s = 0; s < 16; s++) {
-        const int n = s >> 3, q = (s & 7) >> 1, hb = s & 1;
-        const uint32_t lw = r.L[4 * n + 2 * (q & 1) + hb], hw = r.Hq[2 * n + hb];
-        const uint32_t v = ((lw >> (4 * (q >> 1))) & 0x0F0F0F0Fu) | (((hw >> (2 * q)) & 0x03030303u) << 4);
-        const uint2 bq = make_uint2(v & 0x00FF00FFu, (v >> 8) & 0x00FF00FFu);
-        const mm_f16x4 b = __builtin_bit_cast(mm_f16x4, bq);
-        const mm_f16x4 a = *(const mm_f16x4 *)(frag + s * 512 + lane * 8);
-        const mm_f32x4 cc = __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, (mm_f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-        const float2 xm = *(const float2 *)(xs + s * 8 + t0);
-        const uint32_t sw = s < 4 ? r.sc.x : s < 8 ? r.sc.y : s < 12 ? r.sc.z : r.sc.w;
-        /* sa carries the quants' 2^24; the 32 d sc of the offset does not */
-        const float sa = d * (float)(int)(int8_t)byte_of(sw, s & 3), ma = sa * 1.9073486328125e-06f;
-        z0 = fmaf(sa, cc[0] + cc[1], z0);
-        z0 = fmaf(-ma, xm.x, z0);
-        z1 = fmaf(sa, cc[2] + cc[3], z1);
-        z1 = fmaf(-ma, xm.y, z1);
+    for (int n = 0; n < 2; n++) {
+        const uint4 rl = u5_fix(r.l[n], r.sh), rh = u5_fix(r.h[n], r.sh);
+        uint32_t hs[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) hs[i] = u4_word(rh, i) >> qs;
+#pragma unroll
+        for (int hi = 0; hi < 2; hi++) {
+            const uint32_t sw = u4_word(scv, 2 * n + hi);
+            const _Float16 sf = (_Float16)(short)__builtin_amdgcn_sbfe((int)sw, 8 * g, 8);
+            const f16x2 sc = { sf, sf };
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                f16x2 w[4], e[4];
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const uint32_t lw = u4_word(rl, 2 * i + k), hw = hs[2 * i + k];
+                    const uint32_t q = hi ? ((lw >> 4) & 0x0F0F0F0Fu) | (hw & 0x30303030u) : (lw & 0x0F0F0F0Fu) | ((hw << 4) & 0x30303030u);
+                    const f16x2 u = magic_lo(q) + off, v = magic_hi(q) + off;    /* q - 32 */
+                    w[2 * k] = u * sc;
+                    w[2 * k + 1] = v * sc;
+                    e[2 * k] = __builtin_elementwise_fma(u, sc, -w[2 * k]);
+                    e[2 * k + 1] = __builtin_elementwise_fma(v, sc, -w[2 * k + 1]);
+                }
+                const f16x8 b = { w[0][0], w[0][1], w[1][0], w[1][1], w[2][0], w[2][1], w[3][0], w[3][1] };
+                const f16x8 be = { e[0][0], e[0][1], e[1][0], e[1][1], e[2][0], e[2][1], e[3][0], e[3][1] };
+                const f16x8 a = *(const f16x8 *)(frag + (4 * n + 2 * hi + i) * 1024 + lane * 16);
+                z[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, z[0], 0, 0, 0);
+                z[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, be, z[1], 0, 0, 0);
+            }
+        }
     }
 }
 
-template <bool Q6>
-__global__ void __launch_bounds__(MM8_T) dense_mm8_kernel(const uint8_t *W, const uint8_t *buf, float *Y, int rows,
-                                                          int cols, int T, int ksplit)
+/* One super-block of a 16-row group: its products added (live) to y, the sums
+ * of this lane's tokens (PARTS == 3: token l / 16; 2: tokens 2 (l / 16), + 1). */
+template <bool Q6, int PARTS, class Raw>
+__device__ __forceinline__ void mm8_add(const Raw &raw, const uint8_t *lds, int cols, int kb, bool live, int lane,
+                                        float (&y)[2])
+{
+    f32x4 z[2], zm;
+    mm8_block(raw, lds + (size_t)kb * 8192, lds + mm8_frag_bytes(cols) + kb * 256, lane, z, zm);
+    const float *ge = (const float *)(lds + mm8_frag_bytes(cols) + mm8_sum_bytes(cols)) + kb * 8;
+    const int g = lane >> 4;
+    float d, dm;
+    if constexpr (Q6) {
+        d = f16_bits_to_f32(raw.d);
+        dm = 0.0f;
+    } else {
+        d = f16_bits_to_f32(raw.hd.x & 0xFFFFu);
+        dm = f16_bits_to_f32(raw.hd.x >> 16) * -64.0f;   /* the sums carry 2^-6 */
+    }
+    const f32x4 s = z[0] + z[1];
+    if (PARTS == 3) {
+        float v = d * ((s[0] + s[1]) + s[2]);
+        if (!Q6) v = fmaf(dm, (zm[0] + zm[1]) + zm[2], v);
+        y[0] = live ? fmaf(v, ge[g], y[0]) : y[0];
+    } else {
+        float v0 = d * (s[0] + s[1]), v1 = d * (s[2] + s[3]);
+        if (!Q6) {
+            v0 = fmaf(dm, zm[0] + zm[1], v0);
+            v1 = fmaf(dm, zm[2] + zm[3], v1);
+        }
+        const float2 g2 = *(const float2 *)(ge + 2 * g);
+        y[0] = live ? fmaf(v0, g2.x, y[0]) : y[0];
+        y[1] = live ? fmaf(v1, g2.y, y[1]) : y[1];
+    }
+}
+
+template <int PARTS>
+__device__ __forceinline__ void mm8_store(float *Y, int rows, int T, int r, int lane, const float (&y)[2])
+{
+    if (r >= rows) return;
+    const int t0 = PARTS == 3 ? lane >> 4 : 2 * (lane >> 4);
+    if (t0 < T) Y[(size_t)t0 * rows + r] = y[0];
+    if (PARTS == 2 && t0 + 1 < T) Y[(size_t)(t0 + 1) * rows + r] = y[1];
+}
+
+template <bool Q6, int PARTS>
+__global__ void __launch_bounds__(MM8_T, 4) dense_mm8_kernel(const uint8_t *W, const float *X, float *Y, int rows, int cols,
+                                                             int T, int split)
 {
     extern __shared__ __align__(16) uint8_t mm8_lds[];
-    constexpr int SB = Q6 ? 16 : 32;                  /* weights per scale sub-block */
-    constexpr int FB = Q6 ? 512 : 1024;               /* bytes per A fragment (64 lanes) */
     constexpr size_t BS = Q6 ? RQ6K_BYTES : RQ4K_BYTES;
     typedef typename std::conditional<Q6, Mm8Q6, Mm8Q4>::type Raw;
-    const int ns = cols / SB, nb = cols / RQK;
-    /* the call's operands: fragments, sub-block sums and super-block scales */
-    const int n16 = (int)(mm8_buf_bytes(cols, Q6) / 16);
-    for (int i = threadIdx.x; i < n16; i += MM8_T) ((uint4 *)mm8_lds)[i] = gld_u4(buf + 16 * (size_t)i);
-    const uint8_t *frag = mm8_lds;
-    const float *xs = (const float *)(mm8_lds + mm8_frag_bytes(cols));
-    const float *ge = xs + (size_t)ns * 8;
-    __syncthreads();
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int nb = cols / RQK;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g4 = lane >> 4;
     const int ngroups = (rows + 15) >> 4;
-    if (ksplit) {
-        /* few groups (nb <= 16): a workgroup per group, wave w takes super-
-         * blocks w and w + 8, the 8 partial sums added by wave 0 in wave order */
-        __shared__ float2 red[MM8_W][64];
-        const int j = lane >> 4, t0 = 2 * j;
-        for (int g = blockIdx.x; g < ngroups; g += gridDim.x) {
-            const int r = min(16 * g + (lane & 15), rows - 1);
-            const uint8_t *wr = W + (size_t)r * nb * BS;
-            Raw r0, r1;
-            const int k0 = min(wv, nb - 1), k1 = min(wv + MM8_W, nb - 1);
-            mm8_load(r0, wr + (size_t)k0 * BS, j);
-            mm8_load(r1, wr + (size_t)k1 * BS, j);
-            float y0 = 0.0f, y1 = 0.0f;
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const int kb = wv + u * MM8_W;
-                if (kb < nb) {
-                    float z0 = 0.0f, z1 = 0.0f;
-                    mm8_block(u ? r1 : r0, frag + (size_t)kb * (RQK / SB) * FB, xs + (size_t)kb * (RQK / SB) * 8, lane,
-                              z0, z1);
-                    const float2 g2 = *(const float2 *)(ge + kb * 8 + t0);
-                    y0 = fmaf(z0, g2.x, y0);
-                    y1 = fmaf(z1, g2.y, y1);
-                }
-            }
-            red[wv][lane] = make_float2(y0, y1);
-            __syncthreads();
-            if (wv == 0) {
-                float2 a = red[0][lane];
-#pragma unroll
-                for (int w = 1; w < MM8_W; w++) {
-                    const float2 b = red[w][lane];
-                    a.x += b.x;
-                    a.y += b.y;
-                }
-                const int rr = 16 * g + (lane & 15);
-                if (rr < rows) {
-                    if (t0 < T) Y[(size_t)t0 * rows + rr] = a.x;
-                    if (t0 + 1 < T) Y[(size_t)(t0 + 1) * rows + rr] = a.y;
-                }
-            }
-            __syncthreads();
-        }
-        return;
-    }
-    /* many groups: 16-row groups, wave-strided; items (group, kb) with the
-     * next item's raw quants loaded while the current computes */
-    const int gw = blockIdx.x * MM8_W + wv, nw = gridDim.x * MM8_W;
-    const int mine = gw < ngroups ? (ngroups - 1 - gw) / nw + 1 : 0;
-    const int total = mine * nb;
-    if (total == 0) return;
-    const int j = lane >> 4, t0 = 2 * j;
+    /* a workgroup is 8 / split teams of split waves; a team takes a 16-row
+     * group, its member m the super-blocks m, m + split, ..., and member 0 adds
+     * the members' sums in their order */
+    const int member = wv & (split - 1), tpw = MM8_W / split;
+    const int team = blockIdx.x * tpw + wv / split, nteam = gridDim.x * tpw;
+    const int iters = (ngroups + nteam - 1) / nteam, per = (nb + split - 1) / split, total = iters * per;
+    __shared__ float2 red[2][MM8_W][64];
+    /* item i: super-block member + (i % per) split of group team + (i / per)
+     * nteam; past either end the last one again, so that every wave runs the
+     * same items and barriers */
     auto blk = [&](int item) {
-        const int g = gw + (item / nb) * nw, kb = item % nb;
+        const int g = min(team + (item / per) * nteam, ngroups - 1), kb = min(member + (item % per) * split, nb - 1);
         const int r = min(16 * g + (lane & 15), rows - 1);
         return W + ((size_t)r * nb + kb) * BS;
     };
-    float y0 = 0.0f, y1 = 0.0f;
-    auto compute = [&](const Raw &raw, int item) {
-        const int kb = item % nb;
-        float z0 = 0.0f, z1 = 0.0f;
-        mm8_block(raw, frag + (size_t)kb * (RQK / SB) * FB, xs + (size_t)kb * (RQK / SB) * 8, lane, z0, z1);
-        const float2 g2 = *(const float2 *)(ge + kb * 8 + t0);
-        y0 = fmaf(z0, g2.x, y0);
-        y1 = fmaf(z1, g2.y, y1);
-        if (kb == nb - 1) {
-            const int g = gw + (item / nb) * nw, r = 16 * g + (lane & 15);
-            if (r < rows) {
-                if (t0 < T) Y[(size_t)t0 * rows + r] = y0;
-                if (t0 + 1 < T) Y[(size_t)(t0 + 1) * rows + r] = y1;
-            }
-            y0 = y1 = 0.0f;
-        }
-    };
-    /* the loads are unconditional (past the last item: the last item again),
-     * so that the wait before a computation counts only its own loads, not
-     * the next item's behind them */
     Raw ra, rb;
-    mm8_load(ra, blk(0), j);
+    mm8_load(ra, blk(0), g4);
+    for (int kb = wv; kb < nb; kb += MM8_W) mm8_prep<Q6, PARTS>(X, cols, T, kb, mm8_lds, lane);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   /* LDS only: the weights stay in flight */
+    float y[2] = { 0.0f, 0.0f };
+    auto compute = [&](const Raw &raw, int item) {
+        const int it = item / per, j = item - it * per, kb = member + j * split;
+        mm8_add<Q6, PARTS>(raw, mm8_lds, cols, min(kb, nb - 1), kb < nb, lane, y);   /* no branch: the loads stay ahead */
+        if (j != per - 1) return;
+        const int g = team + it * nteam;
+        if (split > 1) {
+            red[it & 1][wv][lane] = make_float2(y[0], y[1]);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (member == 0)
+                for (int w = 1; w < split; w++) {
+                    const float2 b = red[it & 1][wv + w][lane];
+                    y[0] += b.x;
+                    y[1] += b.y;
+                }
+        }
+        if (member == 0 && g < ngroups) mm8_store<PARTS>(Y, rows, T, 16 * g + (lane & 15), lane, y);
+        y[0] = y[1] = 0.0f;
+    };
+    /* the loads are unconditional, so that the wait before a computation counts
+     * only its own loads, not the next item's behind them */
     for (int it = 0;; it += 2) {
-        mm8_load(rb, blk(min(it + 1, total - 1)), j);
+        mm8_load(rb, blk(min(it + 1, total - 1)), g4);
         compute(ra, it);
         if (it + 1 >= total) break;
-        mm8_load(ra, blk(min(it + 2, total - 1)), j);
+        mm8_load(ra, blk(min(it + 2, total - 1)), g4);
         compute(rb, it + 1);
         if (it + 2 >= total) break;
     }
@@ -465,26 +533,30 @@ int dense_mfma_min_tokens() { return g_dense_mfma_t; }
 
 int dense_mm8_launch(const uint8_t *W, int q6, const float *X, float *Y, size_t rows, size_t cols, int T)
 {
-    const size_t bytes = mm8_buf_bytes(cols, q6);
-    uint8_t *buf = (uint8_t *)rt_scratch(SCR_MM, bytes);
-    if (!buf) return ROASTER_EDEVICE;
+    const size_t lds = mm8_lds_bytes(cols);
     const size_t ng = (rows + 15) / 16;
-    const size_t cap = (size_t)(bytes <= 80 * 1024 ? 2 : 1) * rt().n_cu;
+    const size_t cap = (size_t)(lds <= 78 * 1024 ? 2 : 1) * rt().n_cu;
     const int nb = (int)(cols / RQK);
-    /* fewer groups than waves in a full grid (and at most 16 super-blocks):
-     * the super-blocks of a group split over a workgroup's waves */
-    const int ksplit = ng < MM8_W * cap && nb <= 2 * MM8_W;
-    size_t blocks = ksplit ? ng : (ng + MM8_W - 1) / MM8_W;
-    if (blocks > cap) blocks = cap;
-    if (q6) {
-        hipLaunchKernelGGL(mm8_prep_kernel<true>, dim3(nb), dim3(256), 0, rt().stream, X, (int)cols, T, buf);
-        hipLaunchKernelGGL(dense_mm8_kernel<true>, dim3((unsigned)blocks), dim3(MM8_T), bytes, rt().stream, W, buf, Y,
-                           (int)rows, (int)cols, T, ksplit);
-    } else {
-        hipLaunchKernelGGL(mm8_prep_kernel<false>, dim3(nb), dim3(256), 0, rt().stream, X, (int)cols, T, buf);
-        hipLaunchKernelGGL(dense_mm8_kernel<false>, dim3((unsigned)blocks), dim3(MM8_T), bytes, rt().stream, W, buf, Y,
-                           (int)rows, (int)cols, T, ksplit);
+    /* waves per group: the split whose waves run the fewest super-blocks one
+     * after the other (a few groups need several waves each to fill the CUs) */
+    int split = 1;
+    size_t best = 0;
+    for (int sp = 1; sp <= MM8_W && sp <= nb; sp *= 2) {
+        const size_t teams = cap * (MM8_W / sp), cost = (ng + teams - 1) / teams * ((nb + sp - 1) / sp);
+        if (!best || cost < best) best = cost, split = sp;
     }
+    size_t blocks = (ng + MM8_W / split - 1) / (MM8_W / split);
+    if (blocks > cap) blocks = cap;
+    const dim3 gd((unsigned)blocks), bd(MM8_T);
+#define MM8(Q6_, P_) hipLaunchKernelGGL((dense_mm8_kernel<Q6_, P_>), gd, bd, lds, rt().stream, W, X, Y, (int)rows, (int)cols, T, split)
+    if (T <= 4) {
+        if (q6) MM8(true, 3);
+        else MM8(false, 3);
+    } else {
+        if (q6) MM8(true, 2);
+        else MM8(false, 2);
+    }
+#undef MM8
     return rt_check(hipGetLastError(), "dense MFMA launch") ? ROASTER_EDEVICE : 0;
 }
 
@@ -542,8 +614,13 @@ extern "C" int roaster_matvec_q(const void *W, int q6, const float *X, float *Y,
         return dense_mm8_launch((const uint8_t *)W, q6, X, Y, rows, cols, T);
     const int nb = (int)(cols / RQK), rpw = 64 / lanes_per_row(nb);
     const size_t npass = (rows + rpw - 1) / rpw;
-    size_t blocks = (npass + 3) / 4;
-    if (blocks > (size_t)DMV_GRID * rt().n_cu) blocks = (size_t)DMV_GRID * rt().n_cu;
+    /* a grid that is resident at once (registers: 5 workgroups per CU for Q6_K,
+     * 6 for Q4_K, 3 past 8 super-blocks), its waves with equal numbers of
+     * passes: the LM head with one token 104 us on 8 workgroups per CU, 99.5 on
+     * 5, 96 with the next pass's loads under the current one's dots; 8192 rows
+     * of 2048 7.8 -> 6.2 us */
+    const size_t per_cu = nb > 8 ? 3 : q6 ? 5 : 6, waves = 4 * per_cu * rt().n_cu;
+    const size_t iters = (npass + waves - 1) / waves, blocks = (npass + 4 * iters - 1) / (4 * iters);
     const size_t lds = T > 1 ? (size_t)T * cols * 4 + (size_t)T * (cols / 16) * 4 : 0;
     const dim3 gd((unsigned)blocks), bd(MV_THREADS);
     const uint8_t *w = (const uint8_t *)W;

@@ -1,5 +1,5 @@
 /*
- * pf_tile.h -- device helpers shared by the prefill GEMMs that read weights in
+ * pf_tile.h -- device helpers shared by the MFMA GEMMs, first those that read weights in
  * the MFMA tile layout (tile.h): raw lane records and their loads, the fp16
  * bit-pattern conversions of quants, the permuted K order of a super-block,
  * power-of-two scale exponents and the block numbering of a launch.
@@ -40,6 +40,7 @@ __device__ __forceinline__ int pf_virtual_block(int b, int R)
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 /* One lane's raw share of a super-block: half h (weights 128h .. 128h+127). */
 struct RawQ6 { uint32_t L[16], Hh[8], S[2], d; };

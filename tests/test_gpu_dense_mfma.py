@@ -1,0 +1,35 @@
+"""roaster_matvec_q of several tokens on MFMA (dense_mm8_kernel) where its splits
+and operands can go wrong, against the oracle: one row, a row past a 16-row
+group, groups that need every wave of a workgroup and groups that fill the
+grid with one wave each; one, three and nine super-blocks (a wave's members and
+items ragged); 4 tokens in three fp16 parts and 5 in two, and the ends; Q6_K
+scales over the whole int8 range (sc (q - 32) past 2048 needs the second weight
+operand).  One token runs the pipelined matvec on the same shapes.
+
+Bar 5e-6 of max|y|: 22-bit activations (2^-22 per product, random in sign) and
+f32 sums of up to 2304 terms on both sides, about 1e-6 each."""
+import numpy as np
+import pytest
+
+import roaster_amd as R
+from oracle import oracle as O
+from test_gpu_dense import run, weights
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("q6", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (17, 2304), (300, 768), (33000, 256), (70001, 768)])
+def test_splits(q6, rows, cols):
+    W = weights(q6, rows, cols, 70 + cols)
+    if q6:
+        b = W.reshape(-1, R.Q6K_BYTES)
+        b[:, 192:208] = np.random.default_rng(3).integers(0, 256, (len(b), 16), dtype=np.uint8)
+    X = np.stack([R.synth_normal(71, R.synth_stream(t, cols, 5), cols) for t in range(8)])
+    X[1, : cols // 2] *= 2.0 ** 12                # super-blocks of very different size
+    ref = [O.matvec(q6, W, x, rows, cols) for x in X]
+    for T in (1, 2, 4, 5, 8):
+        Y = run(q6, W, X[:T], rows, cols)
+        for t in range(T):
+            err = np.max(np.abs(Y[t] - ref[t])) / np.max(np.abs(ref[t]))
+            assert err <= 5e-6, (T, t, err)
