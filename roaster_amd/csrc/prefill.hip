@@ -68,87 +68,89 @@ __device__ int block_scan_256(int v, int *lds, int *total)
 }
 
 /* ---- router on MFMA: part[s][t][e] = sum over k in split s of X[t][k] W[e][k]
- * A workgroup (4 waves) takes 32 tokens x 128 experts of K split s; wave w
- * owns experts e0 + 32 w .. + 31 in one v_mfma_f32_32x32x2_f32 accumulator
+ * A workgroup (4 waves) takes 32 MT tokens x 128 experts of K split s; wave w
+ * owns experts e0 + 32 w .. + 31 in MT v_mfma_f32_32x32x2_f32 accumulators
  * (A = X rows, B = W rows, fp32 products and sums).  The tokens' K slice is
  * staged once in LDS (row stride klen + 4 floats: the 16 rows a ds_read_b128
- * pass reads fall in 16 different bank groups); each wave reads its weight
- * rows straight from global memory, one 32-wide K chunk ahead.  In a chunk,
- * lane half h supplies k = 16 h + j to MFMA j (j = 0..15), so 16 MFMAs cover
- * the chunk and every lane reads 16 consecutive floats of X and of W. */
+ * pass reads fall in 16 different bank groups); each wave reads its weights
+ * from the router's operand copy (TileLayer.router).  In a 32-wide chunk, lane
+ * half h supplies k = 8 (j / 4) + 4 h + j % 4 to MFMA j (j = 0..15).
+ * At few tokens the time is load latency, so every load of a wave is issued
+ * before its first wait; a staging loop with a bound and weights fetched a chunk
+ * ahead waited for one load after the other: 47 -> 31 us at 2048 tokens, 12.6 ->
+ * 11.1 at 512, 10.7 -> 8.5 at 45 (E 256, H 2048; sixteen waves with a fourth of
+ * the K slice each: 32, 12.0, 8.4).  64 tokens a workgroup halve the weight
+ * reads and give a wave two independent chains, but half the workgroups: 31
+ * against 35.6 us at 2048 tokens, 15.9 against 11.1 at 512. */
 #define RM_E 128                  /* experts per workgroup */
-#define RM_T 32                   /* tokens per workgroup */
-
-extern "C" __global__ void __launch_bounds__(256, 2) pf_router_mfma_kernel(const float *X, const float *W, float *part,
-                                                                           int T, int E, int H)
+#define RM_T2 1024                /* tokens from which a workgroup takes 64 */
+template <int MT>
+__global__ void __launch_bounds__(256, 2) pf_router_mfma_kernel(const float *X, const float *W, float *part,
+                                                                             int T, int E, int H)
 {
+    constexpr int RM_T = 32 * MT;                       /* tokens per workgroup */
     extern __shared__ __align__(16) float xs[];         /* [RM_T][klen + 4] */
     const int tid = threadIdx.x, l = tid & 63, h = l >> 5, n = l & 31;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t0 = blockIdx.x * RM_T, e0 = blockIdx.y * RM_E + 32 * w, s = blockIdx.z;
     const int klen = H / RT_KSPLIT, kbeg = s * klen, ld = klen + 4;
-    /* stage X[t0 .. t0 + 31][kbeg .. kbeg + klen) (klen <= 512: at most 16
-     * float4 per thread, all loaded before the first store; rows past T read
-     * row T - 1, pieces past the slice repeat its last one) */
+    /* stage X[t0 .. t0 + RM_T - 1][kbeg .. kbeg + klen) (klen <= 256: at most 8
+     * MT float4 per thread, all loaded before the first store; rows past T read
+     * row T - 1, pieces past the slice repeat its last one: a store under a
+     * condition takes its load with it) */
     const int q4 = klen / 4, nq = RM_T * q4;           /* float4 per row, in the slice */
-    float4 v[16];
+    float4 v[8 * MT];
 #pragma unroll
-    for (int k = 0; k < 16; k++) {
+    for (int k = 0; k < 8 * MT; k++) {
         const int i = min(tid + 256 * k, nq - 1), r = i / q4, c = i - r * q4;
         v[k] = *(const float4 *)(X + (size_t)min(t0 + r, T - 1) * H + kbeg + 4 * c);
     }
+    /* this lane's weights, every chunk at once (at most 8; chunks past nch
+     * repeat the last, unused; the last block again past E, not stored) */
+    const int nb = (E + 31) / 32, nch = klen / 32;
+    const float *wr = W + ((size_t)min(e0 >> 5, nb - 1) * (H / 32) + kbeg / 32) * 1024 + 4 * l;
+    float4 wb[8][4];
 #pragma unroll
-    for (int k = 0; k < 16; k++) {
+    for (int j = 0; j < 8; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) wb[j][q] = *(const float4 *)(wr + 1024 * min(j, nch - 1) + 256 * q);
+#pragma unroll
+    for (int k = 0; k < 8 * MT; k++) {
         const int i = min(tid + 256 * k, nq - 1), r = i / q4, c = i - r * q4;
         *(float4 *)(xs + r * ld + 4 * c) = v[k];
     }
-    __syncthreads();
-    /* this lane's weight row (clamped past E; those columns are not stored) */
-    const float *wr = W + (size_t)min(e0 + n, E - 1) * H + kbeg + 16 * h;
-    const float *xr = xs + n * ld + 16 * h;
-    f32x16 acc = (f32x16){};
-    /* weights in batches of RM_B chunks, the next batch loaded during the
-     * current one (chunk indices clamped; chunks past nch are not used) */
-    constexpr int RM_B = 4;
-    const int nch = klen / 32;
-    float4 wb[2][RM_B][4];
-    auto w_batch = [&](float4 (&dst)[RM_B][4], int c0) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   /* LDS only: the weights stay in flight */
+    const float *xr = xs + n * ld + 4 * h;
+    f32x16 acc[MT];
 #pragma unroll
-        for (int j = 0; j < RM_B; j++)
+    for (int m = 0; m < MT; m++) acc[m] = (f32x16){};
 #pragma unroll
-            for (int q = 0; q < 4; q++) dst[j][q] = *(const float4 *)(wr + 32 * min(c0 + j, nch - 1) + 4 * q);
-    };
-    auto compute = [&](const float4 (&src)[RM_B][4], int c0) {
+    for (int j = 0; j < 8; j++) {
+        if (j >= nch) break;
 #pragma unroll
-        for (int j = 0; j < RM_B; j++) {
-            if (c0 + j >= nch) break;
-            float4 xa[4];
+        for (int q = 0; q < 4; q++) {
+            float4 xa[MT];
 #pragma unroll
-            for (int q = 0; q < 4; q++) xa[q] = *(const float4 *)(xr + 32 * (c0 + j) + 4 * q);
+            for (int m = 0; m < MT; m++) xa[m] = *(const float4 *)(xr + 32 * m * ld + 32 * j + 8 * q);
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[q].x, src[j][q].x, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[q].y, src[j][q].y, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[q].z, src[j][q].z, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[q].w, src[j][q].w, acc, 0, 0, 0);
-            }
+            for (int m = 0; m < MT; m++) acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[m].x, wb[j][q].x, acc[m], 0, 0, 0);
+#pragma unroll
+            for (int m = 0; m < MT; m++) acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[m].y, wb[j][q].y, acc[m], 0, 0, 0);
+#pragma unroll
+            for (int m = 0; m < MT; m++) acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[m].z, wb[j][q].z, acc[m], 0, 0, 0);
+#pragma unroll
+            for (int m = 0; m < MT; m++) acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[m].w, wb[j][q].w, acc[m], 0, 0, 0);
         }
-    };
-    w_batch(wb[0], 0);
-    for (int c = 0; c < nch; c += 2 * RM_B) {
-        w_batch(wb[1], c + RM_B);
-        compute(wb[0], c);
-        if (c + RM_B >= nch) break;
-        w_batch(wb[0], c + 2 * RM_B);
-        compute(wb[1], c + RM_B);
     }
-    /* D item i: token t0 + 8 (i / 4) + 4 h + i % 4, expert e0 + n */
+    /* D item i: token t0 + 32 m + 8 (i / 4) + 4 h + i % 4, expert e0 + n */
     if (e0 + n < E) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int m = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
-            if (m < T) part[((size_t)s * T + m) * E + e0 + n] = acc[i];
-        }
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int t = t0 + 32 * m + 8 * (i >> 2) + 4 * h + (i & 3);
+                if (t < T) part[((size_t)s * T + t) * E + e0 + n] = acc[m][i];
+            }
     }
 }
 
@@ -732,10 +734,13 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     const DecLayer &L = t->layers_h[layer];
 
     if (!opt.logits_in) {
-        dim3 g((T + RM_T - 1) / RM_T, (E + RM_E - 1) / RM_E, RT_KSPLIT);
-        const size_t xlds = (size_t)RM_T * (H / RT_KSPLIT + 4) * 4;
-        hipLaunchKernelGGL(pf_router_mfma_kernel, g, dim3(256), xlds, R.stream, X, L.router, (float *)(ws + o_part), T,
-                           E, H);
+        const int mt = T >= RM_T2 ? 2 : 1;
+        dim3 g((T + 32 * mt - 1) / (32 * mt), (E + RM_E - 1) / RM_E, RT_KSPLIT);
+        const size_t xlds = (size_t)32 * mt * (H / RT_KSPLIT + 4) * 4;
+        if (mt == 2)
+            hipLaunchKernelGGL(pf_router_mfma_kernel<2>, g, dim3(256), xlds, R.stream, X, t->tlayers_h[layer].router, (float *)(ws + o_part), T, E, H);
+        else
+            hipLaunchKernelGGL(pf_router_mfma_kernel<1>, g, dim3(256), xlds, R.stream, X, t->tlayers_h[layer].router, (float *)(ws + o_part), T, E, H);
         if (rt_check(hipGetLastError(), "prefill router launch")) return ROASTER_EDEVICE;
     }
     PfTokArgs ta;

@@ -70,7 +70,8 @@ extern "C" RoasterTable *roaster_table_create_layers(const RoasterTableDesc *d, 
     }
     t->qbytes = qoff;
     t->tbytes = toff;
-    t->fbytes = (size_t)d->n_layers * (E * H + H) * sizeof(float);
+    const size_t EB = (E + 31) / 32 * 32;         /* experts of the router's operand copy */
+    t->fbytes = (size_t)d->n_layers * (E * H + H + EB * H) * sizeof(float);
     if (hipMalloc((void **)&t->qmem, t->qbytes + RT_TAIL_PAD) != hipSuccess ||
         hipMalloc((void **)&t->tmem, t->tbytes + RT_TAIL_PAD) != hipSuccess ||
         hipMalloc((void **)&t->fmem, t->fbytes) != hipSuccess ||
@@ -116,6 +117,7 @@ extern "C" RoasterTable *roaster_table_create_layers(const RoasterTableDesc *d, 
         TL.sgate = tbase + G.toff_sh[0];
         TL.sup = tbase + G.toff_sh[1];
         TL.sdown = tbase + G.toff_sh[2];
+        TL.router = t->fmem + (size_t)d->n_layers * (E * H + H) + (size_t)l * EB * H;
     }
     if (rt_check(hipMemcpy(t->layers_d, t->layers_h.data(), sizeof(DecLayer) * d->n_layers, hipMemcpyHostToDevice),
                  "layer table upload")) {
@@ -254,6 +256,26 @@ __global__ void __launch_bounds__(256) dbound_kernel(const uint8_t *src, size_t 
     if (threadIdx.x == 0) dst[blockIdx.x] = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
 }
 
+/* A router's operand copy (TileLayer.router), one thread per 16 bytes. */
+__global__ void router_tile_kernel(const float *src, float4 *dst, int E, int H)
+{
+    const size_t n = (size_t)(E + 31) / 32 * 32 * H / 4, id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (id >= n) return;
+    const int l = (int)(id & 63), q = (int)(id >> 6) & 3;
+    const size_t bc = id >> 8;
+    const int c = (int)(bc % (H / 32)), e = 32 * (int)(bc / (H / 32)) + (l & 31);
+    dst[id] = e < E ? *(const float4 *)(src + (size_t)e * H + 32 * c + 8 * q + 4 * (l >> 5)) : make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+static int router_tile(const RoasterTable *t, int layer)
+{
+    const int E = t->d.n_experts, H = (int)t->d.hidden;
+    const size_t n = (size_t)(E + 31) / 32 * 32 * H / 4;
+    hipLaunchKernelGGL(router_tile_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, rt().stream,
+                       t->layers_h[layer].router, (float4 *)t->tlayers_h[layer].router, E, H);
+    return rt_check(hipGetLastError(), "router repack launch") ? ROASTER_EDEVICE : 0;
+}
+
 /* Rebuild the tile copy of nmat consecutive matrices of one kind (routed
  * experts e0 .. e0 + nmat - 1, or the shared expert when e0 == E), and for
  * down matrices their row bounds. */
@@ -319,7 +341,8 @@ extern "C" int roaster_table_set_router(RoasterTable *t, int layer, const float 
     if (rt_check(hipMemcpy((void *)L.router, router, EH * 4, hipMemcpyHostToDevice), "router upload") ||
         rt_check(hipMemcpy((void *)L.gate_inp, gate_inp, t->d.hidden * 4, hipMemcpyHostToDevice), "gate upload"))
         return ROASTER_EDEVICE;
-    return 0;
+    if (int rc = router_tile(t, layer)) return rc;
+    return rt_check(hipStreamSynchronize(rt().stream), "router repack") ? ROASTER_EDEVICE : 0;
 }
 
 extern "C" int roaster_table_expert_ptrs(const RoasterTable *t, int layer, int expert, const void **gate,
@@ -423,9 +446,10 @@ extern "C" int roaster_table_synth(RoasterTable *t, uint64_t seed, const Roaster
         roaster_synth_normal(seed, roaster_synth_stream(l, 0, 4), H, s.gate_inp_sigma, gi.data());
         const DecLayer &L = t->layers_h[l];
         if (rt_check(hipMemcpyAsync((void *)L.router, router.data(), E * H * 4, hipMemcpyHostToDevice, st), "router") ||
-            rt_check(hipMemcpyAsync((void *)L.gate_inp, gi.data(), H * 4, hipMemcpyHostToDevice, st), "gate_inp") ||
-            rt_check(hipStreamSynchronize(st), "synth sync"))
+            rt_check(hipMemcpyAsync((void *)L.gate_inp, gi.data(), H * 4, hipMemcpyHostToDevice, st), "gate_inp"))
             return ROASTER_EDEVICE;
+        if (int rc = router_tile(t, l)) return rc;
+        if (rt_check(hipStreamSynchronize(st), "synth sync")) return ROASTER_EDEVICE;
     }
     return 0;
 }
