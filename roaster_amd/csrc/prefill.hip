@@ -13,7 +13,8 @@
  *                      of model.c:1713-1731
  *   pf_plan_kernel     offsets (prefix sums of the counts), groups and the
  *                      tile list; the shared expert is one more group over
- *                      all T tokens (model.c:1694-1711)
+ *                      all T tokens (model.c:1694-1711).  Up to PF_ONE_T
+ *                      tokens the token kernel does both (pf_bucket_plan)
  *   grouped GEMMs      gate/up with the SiLU(gate) * up epilogue, then down
  *                      (pf_gemm.hip)
  *   pf_combine_kernel  Y[t] = sigmoid(s_t) * shared(t), then += w * expert
@@ -155,153 +156,6 @@ __global__ void __launch_bounds__(256, 2) pf_router_mfma_kernel(const float *X, 
 }
 
 
-/* ---- per token: logits, top-8, shared gate, X row scale ------------------ */
-struct PfTokArgs {
-    const float *X;
-    const float *gate_inp;
-    const float *part;          /* router partial sums [KSPLIT][T][E], or NULL */
-    const float *logits_in;     /* [T x E] or NULL */
-    const float *bias;          /* [E] or NULL */
-    float *logits_out;          /* [T x E] or NULL */
-    int *ids;                   /* [T x 8] */
-    float *w;                   /* [T x 8] */
-    int *ids_out;
-    float *w_out;
-    float *sg;                  /* [T] */
-    float *xinv, *xfwd;         /* [T] (fp16 mode) or NULL */
-    uint16_t *x16;              /* [T x H] fp16 X * xinv in the GEMM's permuted K order, or NULL */
-    uint16_t *x16l;             /* [T x H] what x16 rounded off (split mode on narrow tiles), or NULL */
-    uint16_t *xs16;             /* [T][H / 256][16] sub-block sums of x16 + x16l, scaled by 2^-6 (hi, lo), or NULL */
-    int *err;
-    int T, E, H;
-};
-
-extern "C" __global__ void __launch_bounds__(256) pf_token_kernel(PfTokArgs A)
-{
-    __shared__ int bad[4];
-    __shared__ TopkScratch ts[4];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int t = blockIdx.x * 4 + wv;
-    if (t >= A.T) return;
-    /* The token's logits (or router partial sums) and biases are loaded
-     * first, then its X row (H <= 2048: at most 8 float4 per lane) and the
-     * gate vector, indices clamped.  A wave's loads complete in order, so
-     * the top 8 runs on the logits while the X row is still arriving; the
-     * row then stays in registers for the fp16 conversion. */
-    float v4[4], b4[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
-    /* the router's 4 x RT_KSPLIT partial sums (or the 4 logits) in one
-     * batch, summed in split order once the X row is on its way */
-    const size_t TE = (size_t)A.T * A.E;
-    float p[4][RT_KSPLIT];
-    if (A.logits_in) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) v4[i] = A.logits_in[(size_t)t * A.E + min(lane + 64 * i, A.E - 1)];
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int s = 0; s < RT_KSPLIT; s++) p[i][s] = A.part[s * TE + (size_t)t * A.E + min(lane + 64 * i, A.E - 1)];
-    }
-    if (A.bias) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) b4[i] = A.bias[min(lane + 64 * i, A.E - 1)];
-    }
-    const float *x = A.X + (size_t)t * A.H;
-    float4 xv[8], gv[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int k = min(4 * lane + 256 * i, A.H - 4);
-        xv[i] = *(const float4 *)(x + k);
-        gv[i] = *(const float4 *)(A.gate_inp + k);
-    }
-    if (!A.logits_in) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float sum = p[i][0];
-#pragma unroll
-            for (int s = 1; s < RT_KSPLIT; s++) sum += p[i][s];
-            v4[i] = sum;
-        }
-    }
-    /* logits (+ bias) and the top 8 */
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int e = lane + 64 * i;
-        float l = -INFINITY;
-        if (e < A.E) {
-            l = v4[i];
-            if (A.bias) l = l + b4[i];
-            if (A.logits_out) A.logits_out[(size_t)t * A.E + e] = l;
-        }
-        v4[i] = l;
-    }
-    if (lane == 0) bad[wv] = 0;
-    __builtin_amdgcn_wave_barrier();
-    topk8_fast(v4, A.E, A.ids + (size_t)t * 8, A.w + (size_t)t * 8, &bad[wv], &ts[wv]);
-    /* X row: max |x|, the shared-expert gate dot, the fp16 copy */
-    float mx = 0.0f, dot = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        if (4 * lane + 256 * i < A.H) {
-            const float4 v = xv[i], g = gv[i];
-            mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-            dot = fmaf(v.x, g.x, dot); dot = fmaf(v.y, g.y, dot);
-            dot = fmaf(v.z, g.z, dot); dot = fmaf(v.w, g.w, dot);
-        }
-    }
-    dot = group_sum<64>(dot);
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
-    if (A.xinv) {
-        float inv, fwd;
-        if (A.x16l) row_scale_wide(mx, inv, fwd);
-        else row_scale(mx, inv, fwd);
-        if (lane == 0) {
-            A.xinv[t] = inv;
-            A.xfwd[t] = fwd;
-        }
-        if (A.x16) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int k = 4 * lane + 256 * i;
-                if (k < A.H) {
-                    const float4 v = xv[i];
-                    const f32x8 e = { v.x * inv, v.y * inv, v.z * inv, v.w * inv, 0.f, 0.f, 0.f, 0.f };
-                    const f16x8 hi = __builtin_convertvector(e, f16x8);
-                    const uint4 c = __builtin_bit_cast(uint4, hi);
-                    const size_t at = (size_t)t * A.H + (k & ~255) + pf_perm_slot4(k & 255);
-                    *(uint2 *)(A.x16 + at) = make_uint2(c.x, c.y);
-                    f32x8 used = __builtin_convertvector(hi, f32x8);
-                    if (A.x16l) {
-                        const f16x8 lo = __builtin_convertvector(e - used, f16x8);
-                        const uint4 lc = __builtin_bit_cast(uint4, lo);
-                        *(uint2 *)(A.x16l + at) = make_uint2(lc.x, lc.y);
-                        used = used + __builtin_convertvector(lo, f32x8);
-                    }
-                    if (A.xs16) {
-                        /* a 32-column sub-block is 8 neighbouring lanes */
-                        const float sum = group_sum<8>((used[0] + used[1]) + (used[2] + used[3])) * 0.015625f;
-                        const _Float16 sh = (_Float16)sum, sl = (_Float16)(sum - (float)sh);
-                        uint16_t *o = A.xs16 + ((size_t)t * (A.H / 256) + i) * 16 + (lane >> 3);
-                        if ((lane & 7) == 0) {
-                            o[0] = __builtin_bit_cast(uint16_t, sh);
-                            o[8] = __builtin_bit_cast(uint16_t, sl);
-                        }
-                    }
-                }
-            }
-        }
-    }
-    if (lane == 0) A.sg[t] = 1.0f / (1.0f + expf(-dot));
-    if (lane < 8) {
-        if (A.ids_out) A.ids_out[(size_t)t * 8 + lane] = A.ids[(size_t)t * 8 + lane];
-        if (A.w_out) A.w_out[(size_t)t * 8 + lane] = A.w[(size_t)t * 8 + lane];
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-    if (lane == 0 && bad[wv]) atomicOr(A.err, 1);
-}
-
 /* ---- bucketing: list[e][r] = r-th token (ascending) that selected e ------- */
 extern "C" __global__ void __launch_bounds__(256) pf_bucket_kernel(const int *ids, int T, int *list, int *rank,
                                                                    int *cnt)
@@ -354,7 +208,8 @@ struct PfPlanArgs {
     size_t teb_g, teb_u, teb_d; /* per-expert tile-layout bytes */
     int q6g, q6u, q6d, sq6g, sq6u, sq6d;
     const int *cnt;
-    const int *list;
+    int *list;                  /* [E][T] */
+    int *rank;                  /* [T x 8] */
     int *off;                   /* [E] */
     int *counts_out;            /* [E] or NULL */
     PfGroup *groups;            /* [E + 1] */
@@ -413,15 +268,14 @@ __device__ int4 block_scan4_256(int4 v, int *lds, int4 *total)
     return make_int4(before.x + inc.x - v.x, before.y + inc.y - v.y, before.z + inc.z - v.z, before.w + inc.w - v.w);
 }
 
-extern "C" __global__ void __launch_bounds__(256) pf_plan_kernel(PfPlanArgs A)
+/* The plan by one 256-thread workgroup; thread e < E brings its expert's row
+ * count c and both down bounds (0 past E). */
+__device__ __forceinline__ void pf_plan(const PfPlanArgs &A, int c, float dbnd, float sdbnd)
 {
     __shared__ int wsum[16];
     __shared__ int s_gc[258], s_toff[257], s_c[257];
     const int e = threadIdx.x;
     if (e < 8) A.gu_ctr[e] = 0;
-    /* every global read first (their latencies overlap) */
-    const int c = e < A.E ? A.cnt[e] : 0;
-    const float dbnd = e < A.E ? A.dbound[e] : 0.0f, sdbnd = A.dbound[A.E];
     const int nt = (c + A.chunk - 1) / A.chunk;
     const int cost = A.dn_bnd && e < A.E ? pf_dn_group_cost(c, A.chunk, A.nt_out) : 0;
     const int nn = A.nw_tiles ? (c + A.nw_rows - 1) / A.nw_rows : 0;
@@ -551,6 +405,253 @@ extern "C" __global__ void __launch_bounds__(256) pf_plan_kernel(PfPlanArgs A)
             }
             A.dn_bnd[b] = u;
         }
+    }
+}
+
+extern "C" __global__ void __launch_bounds__(256) pf_plan_kernel(PfPlanArgs A)
+{
+    /* every global read first (their latencies overlap) */
+    const int e = threadIdx.x;
+    const int c = e < A.E ? A.cnt[e] : 0;
+    const float dbnd = e < A.E ? A.dbound[e] : 0.0f, sdbnd = A.dbound[A.E];
+    pf_plan(A, c, dbnd, sdbnd);
+}
+
+/* Bucketing and plan by one 256-thread workgroup (T <= PF_ONE_T, E <= 256):
+ * which expert has which tokens as a bit map in LDS; a pick's rank is the
+ * number of set bits before its token.  Run by the last workgroup of the token
+ * kernel it saves two launches of about 5 us each and costs a serial stretch
+ * that grows with T; the whole call (E 256, H 2048, inter 512) took, in place of
+ * the three launches, 40.7 for 44.1 us at 1 token, 123.5 for 127.1 at 45, 159.1
+ * for 161.3 at 256, 175.7 for 177.8 at 512, and 225.8 for 222.5 at 1024. */
+#define PF_ONE_T 512
+/* words per expert, odd: the experts' words of one token fall in different banks */
+__host__ __device__ static inline int pf_map_ld(int T) { return (T + 31) / 32 | 1; }
+static size_t pf_map_bytes(int T, int E) { return (size_t)E * pf_map_ld(T) * 6; }
+
+__device__ __forceinline__ void pf_bucket_plan(const PfPlanArgs &A, const int *ids, int *list, int *rank, uint32_t *map)
+{
+    const int tid = threadIdx.x, np = 8 * A.T, ld = pf_map_ld(A.T);
+    uint16_t *before = (uint16_t *)(map + A.E * ld);    /* [E][ld] set bits of the words before */
+    const float dbnd = tid < A.E ? A.dbound[tid] : 0.0f, sdbnd = A.dbound[A.E];
+    /* the picks, 2048 a batch (indices clamped) */
+    constexpr int NB = 8 * PF_ONE_T / 2048;
+    int id[NB][8];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        if (2048 * b >= np) break;
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            id[b][j] = __hip_atomic_load(ids + min(2048 * b + 256 * j + tid, np - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    for (int i = tid; i < A.E * ld; i += 256) map[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        if (2048 * b >= np) break;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int p = 2048 * b + 256 * j + tid, t = p >> 3;
+            if (p < np && id[b][j] >= 0) atomicOr(&map[id[b][j] * ld + (t >> 5)], 1u << (t & 31));
+        }
+    }
+    __syncthreads();
+    int c = 0;
+    if (tid < A.E)
+        for (int i = 0; i < ld; i++) {
+            before[tid * ld + i] = (uint16_t)c;
+            c += __popc(map[tid * ld + i]);
+        }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        if (2048 * b >= np) break;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int p = 2048 * b + 256 * j + tid, t = p >> 3;
+            if (p < np && id[b][j] >= 0) {
+                const int at = id[b][j] * ld + (t >> 5);
+                const int r = before[at] + __popc(map[at] & ((1u << (t & 31)) - 1u));
+                list[(size_t)id[b][j] * A.T + r] = t;
+                rank[p] = r;
+            }
+        }
+    }
+    pf_plan(A, c, dbnd, sdbnd);
+}
+
+/* ---- per token: logits, top-8, shared gate, X row scale ------------------ */
+struct PfTokArgs {
+    const float *X;
+    const float *gate_inp;
+    const float *part;          /* router partial sums [KSPLIT][T][E], or NULL */
+    const float *logits_in;     /* [T x E] or NULL */
+    const float *bias;          /* [E] or NULL */
+    float *logits_out;          /* [T x E] or NULL */
+    int *ids;                   /* [T x 8] */
+    float *w;                   /* [T x 8] */
+    int *ids_out;
+    float *w_out;
+    float *sg;                  /* [T] */
+    float *xinv, *xfwd;         /* [T] (fp16 mode) or NULL */
+    uint16_t *x16;              /* [T x H] fp16 X * xinv in the GEMM's permuted K order, or NULL */
+    uint16_t *x16l;             /* [T x H] what x16 rounded off (split mode on narrow tiles), or NULL */
+    uint16_t *xs16;             /* [T][H / 256][16] sub-block sums of x16 + x16l, scaled by 2^-6 (hi, lo), or NULL */
+    int *err;
+    int *done;                  /* PLAN: workgroups whose picks are written; 0 between calls */
+    int T, E, H;
+};
+
+/* PLAN: the workgroup that finds all others' picks written buckets and plans
+ * as well (pf_bucket_plan), in place of two more launches. */
+template <bool PLAN>
+__global__ void __launch_bounds__(256, 4) pf_token_kernel(PfTokArgs A, PfPlanArgs P)
+{
+    extern __shared__ __align__(16) uint32_t pf_map[];  /* PLAN: the bit map */
+    __shared__ int bad[4];
+    __shared__ TopkScratch ts[4];
+    __shared__ int s_ids[4][RTOPK];
+    __shared__ float s_w[4][RTOPK];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int t = min(blockIdx.x * 4 + wv, A.T - 1);    /* waves past T: token T - 1 again, the same values */
+    /* The token's logits (or router partial sums) and biases are loaded
+     * first, then its X row (H <= 2048: at most 8 float4 per lane) and the
+     * gate vector, indices clamped.  A wave's loads complete in order, so
+     * the top 8 runs on the logits while the X row is still arriving; the
+     * row then stays in registers for the fp16 conversion. */
+    float v4[4], b4[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+    /* the router's 4 x RT_KSPLIT partial sums (or the 4 logits) in one
+     * batch, summed in split order once the X row is on its way */
+    const size_t TE = (size_t)A.T * A.E;
+    float p[4][RT_KSPLIT];
+    if (A.logits_in) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v4[i] = A.logits_in[(size_t)t * A.E + min(lane + 64 * i, A.E - 1)];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int s = 0; s < RT_KSPLIT; s++) p[i][s] = A.part[s * TE + (size_t)t * A.E + min(lane + 64 * i, A.E - 1)];
+    }
+    if (A.bias) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) b4[i] = A.bias[min(lane + 64 * i, A.E - 1)];
+    }
+    const float *x = A.X + (size_t)t * A.H;
+    float4 xv[8], gv[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int k = min(4 * lane + 256 * i, A.H - 4);
+        xv[i] = *(const float4 *)(x + k);
+        gv[i] = *(const float4 *)(A.gate_inp + k);
+    }
+    if (!A.logits_in) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float sum = p[i][0];
+#pragma unroll
+            for (int s = 1; s < RT_KSPLIT; s++) sum += p[i][s];
+            v4[i] = sum;
+        }
+    }
+    /* logits (+ bias) and the top 8 */
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int e = lane + 64 * i;
+        float l = -INFINITY;
+        if (e < A.E) {
+            l = v4[i];
+            if (A.bias) l = l + b4[i];
+            if (A.logits_out) A.logits_out[(size_t)t * A.E + e] = l;
+        }
+        v4[i] = l;
+    }
+    if (lane == 0) bad[wv] = 0;
+    __builtin_amdgcn_wave_barrier();
+    topk8_fast(v4, A.E, s_ids[wv], s_w[wv], &bad[wv], &ts[wv]);
+    __builtin_amdgcn_wave_barrier();
+    if (lane < 8) {
+        const int id = s_ids[wv][lane];
+        const float w = s_w[wv][lane];
+        if constexpr (PLAN)
+            __hip_atomic_store(A.ids + (size_t)t * 8 + lane, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+            A.ids[(size_t)t * 8 + lane] = id;
+        A.w[(size_t)t * 8 + lane] = w;
+        if (A.ids_out) A.ids_out[(size_t)t * 8 + lane] = id;
+        if (A.w_out) A.w_out[(size_t)t * 8 + lane] = w;
+    }
+    int ndone = 0;
+    if constexpr (PLAN) {
+        /* the ids are agent-scope stores: once counted complete here they are
+         * in memory, where the planning workgroup's agent-scope loads find
+         * them (a release would also write back the XCD's L2, per workgroup) */
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (threadIdx.x == 0) ndone = __hip_atomic_fetch_add(A.done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    /* X row: max |x|, the shared-expert gate dot, the fp16 copy */
+    float mx = 0.0f, dot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        if (4 * lane + 256 * i < A.H) {
+            const float4 v = xv[i], g = gv[i];
+            mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+            dot = fmaf(v.x, g.x, dot); dot = fmaf(v.y, g.y, dot);
+            dot = fmaf(v.z, g.z, dot); dot = fmaf(v.w, g.w, dot);
+        }
+    }
+    dot = group_sum<64>(dot);
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+    if (A.xinv) {
+        float inv, fwd;
+        if (A.x16l) row_scale_wide(mx, inv, fwd);
+        else row_scale(mx, inv, fwd);
+        if (lane == 0) {
+            A.xinv[t] = inv;
+            A.xfwd[t] = fwd;
+        }
+        if (A.x16) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int k = 4 * lane + 256 * i;
+                if (k < A.H) {
+                    const float4 v = xv[i];
+                    const f32x8 e = { v.x * inv, v.y * inv, v.z * inv, v.w * inv, 0.f, 0.f, 0.f, 0.f };
+                    const f16x8 hi = __builtin_convertvector(e, f16x8);
+                    const uint4 c = __builtin_bit_cast(uint4, hi);
+                    const size_t at = (size_t)t * A.H + (k & ~255) + pf_perm_slot4(k & 255);
+                    *(uint2 *)(A.x16 + at) = make_uint2(c.x, c.y);
+                    f32x8 used = __builtin_convertvector(hi, f32x8);
+                    if (A.x16l) {
+                        const f16x8 lo = __builtin_convertvector(e - used, f16x8);
+                        const uint4 lc = __builtin_bit_cast(uint4, lo);
+                        *(uint2 *)(A.x16l + at) = make_uint2(lc.x, lc.y);
+                        used = used + __builtin_convertvector(lo, f32x8);
+                    }
+                    if (A.xs16) {
+                        /* a 32-column sub-block is 8 neighbouring lanes */
+                        const float sum = group_sum<8>((used[0] + used[1]) + (used[2] + used[3])) * 0.015625f;
+                        const _Float16 sh = (_Float16)sum, sl = (_Float16)(sum - (float)sh);
+                        uint16_t *o = A.xs16 + ((size_t)t * (A.H / 256) + i) * 16 + (lane >> 3);
+                        if ((lane & 7) == 0) {
+                            o[0] = __builtin_bit_cast(uint16_t, sh);
+                            o[8] = __builtin_bit_cast(uint16_t, sl);
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if (lane == 0) A.sg[t] = 1.0f / (1.0f + expf(-dot));
+    if (lane == 0 && bad[wv]) atomicOr(A.err, 1);
+    if constexpr (PLAN) {
+        __shared__ int last;
+        if (threadIdx.x == 0) last = ndone == (int)gridDim.x - 1;
+        __syncthreads();
+        if (!last) return;
+        if (threadIdx.x == 0) __hip_atomic_store(A.done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        pf_bucket_plan(P, A.ids, P.list, P.rank, pf_map);
     }
 }
 
@@ -761,14 +862,8 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     ta.x16l = nw_split ? (uint16_t *)(ws + o_x16l) : nullptr;
     ta.xs16 = narrow ? (uint16_t *)(ws + o_xs16) : nullptr;
     ta.err = (int *)(ctrl + 16);
+    ta.done = (int *)(ctrl + 48);
     ta.T = T; ta.E = E; ta.H = H;
-    hipLaunchKernelGGL(pf_token_kernel, dim3((T + 3) / 4), dim3(256), 0, R.stream, ta);
-    if (rt_check(hipGetLastError(), "prefill token launch")) return ROASTER_EDEVICE;
-
-    hipLaunchKernelGGL(pf_bucket_kernel, dim3(E), dim3(256), 0, R.stream, (const int *)(ws + o_ids), T,
-                       (int *)(ws + o_list), (int *)(ws + o_rank), (int *)(ws + o_cnt));
-    if (rt_check(hipGetLastError(), "prefill bucket launch")) return ROASTER_EDEVICE;
-
     PfPlanArgs pa;
     pa.L = L;
     pa.TL = t->tlayers_h[layer];
@@ -777,7 +872,8 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     pa.q6g = LG.q6[0]; pa.q6u = LG.q6[1]; pa.q6d = LG.q6[2];
     pa.sq6g = LG.sh_q6[0]; pa.sq6u = LG.sh_q6[1]; pa.sq6d = LG.sh_q6[2];
     pa.cnt = (const int *)(ws + o_cnt);
-    pa.list = (const int *)(ws + o_list);
+    pa.list = (int *)(ws + o_list);
+    pa.rank = (int *)(ws + o_rank);
     pa.off = (int *)(ws + o_off);
     pa.counts_out = opt.counts_out;
     pa.groups = (PfGroup *)(ws + o_grp);
@@ -801,8 +897,18 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     pa.nw_tiles = narrow ? (PfTile *)(ws + o_nwt) : nullptr;
     pa.nw_ntiles = narrow ? (int *)(ws + o_nwn) : nullptr;
     pa.nw_rows = nw_rows;
-    hipLaunchKernelGGL(pf_plan_kernel, dim3(1), dim3(256), 0, R.stream, pa);
-    if (rt_check(hipGetLastError(), "prefill plan launch")) return ROASTER_EDEVICE;
+    if (T <= PF_ONE_T) {
+        hipLaunchKernelGGL(pf_token_kernel<true>, dim3((T + 3) / 4), dim3(256), pf_map_bytes(T, E), R.stream, ta, pa);
+        if (rt_check(hipGetLastError(), "prefill token launch")) return ROASTER_EDEVICE;
+    } else {
+        hipLaunchKernelGGL(pf_token_kernel<false>, dim3((T + 3) / 4), dim3(256), 0, R.stream, ta, pa);
+        if (rt_check(hipGetLastError(), "prefill token launch")) return ROASTER_EDEVICE;
+        hipLaunchKernelGGL(pf_bucket_kernel, dim3(E), dim3(256), 0, R.stream, (const int *)(ws + o_ids), T, pa.list,
+                           pa.rank, (int *)(ws + o_cnt));
+        if (rt_check(hipGetLastError(), "prefill bucket launch")) return ROASTER_EDEVICE;
+        hipLaunchKernelGGL(pf_plan_kernel, dim3(1), dim3(256), 0, R.stream, pa);
+        if (rt_check(hipGetLastError(), "prefill plan launch")) return ROASTER_EDEVICE;
+    }
 
     PfGemmArgs ga;
     ga.groups = pa.groups;

@@ -88,7 +88,9 @@ extern "C" void *roaster_stream(void)
     return (void *)g_rt.stream;
 }
 
-/* Control words of the decode kernels: [16] sticky error bits (1 = routing
+/* Control words of the decode and prefill kernels: [32] counts the
+ * one-launch stack's workgroups (never reset) and [48] the prefill token
+ * kernel's (0 between calls); [16] sticky error bits (1 = routing
  * found fewer than 8 finite logits, 2 = an exchange wait of the one-launch
  * stack gave up, 4 = a workgroup of it read an XCC_ID out of range), cleared
  * when reported; 4 also sends later launches' exchanges through memory. */
