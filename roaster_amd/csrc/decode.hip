@@ -53,6 +53,7 @@
 
 #include <stdio.h>
 #include <string.h>
+#include <type_traits>
 
 #define DT 256                        /* threads per workgroup */
 #define DW (DT / 64)                  /* waves per workgroup */
@@ -1932,15 +1933,20 @@ __device__ __forceinline__ float r1_gather_run(const uint64_t *base, int I, int 
 }
 
 /* k1_down_row's arithmetic on a rotated SiLU*up vector. */
-__device__ __forceinline__ float r1_down_row(int d6, const QChunk &ch, const float *eh, const float *ehs, bool live,
+template <int D>
+__device__ __forceinline__ float r1_down_row(int q6, const QChunk &ch, const float *eh, const float *ehs, bool live,
                                              int lane)
 {
     const int lr = lane & 15, c = lr & 7, lb = lr >> 3;
     float part = 0.0f;
+    auto dot = [&](auto t6) {
+        constexpr bool T6 = decltype(t6)::value;
+        const int ca = lb * RQK + q_run_a<T6>(c), cb = ca + (T6 ? 64 : 32);
+        return q_chunk_dot<T6>(ch, c, eh + r1_ehpos(ca), eh + r1_ehpos(cb), ehs[ca >> 4], ehs[cb >> 4]);
+    };
     if (live) {
-        const int ca = lb * RQK + q_run_a_t(d6, c), cb = ca + (d6 ? 64 : 32);
-        part = d6 ? q_chunk_dot<true>(ch, c, eh + r1_ehpos(ca), eh + r1_ehpos(cb), ehs[ca >> 4], ehs[cb >> 4])
-                  : q_chunk_dot<false>(ch, c, eh + r1_ehpos(ca), eh + r1_ehpos(cb), ehs[ca >> 4], ehs[cb >> 4]);
+        if constexpr (D >= 0) part = dot(std::bool_constant<D != 0>());
+        else part = q6 ? dot(std::true_type()) : dot(std::false_type());
     }
     return group_sum<16>(part);
 }
@@ -2001,9 +2007,10 @@ __device__ __forceinline__ void r1_prefetch_rs(const DecArgs &A, const DecLayer 
 }
 
 /* G: type of the gate and up matrices; D: of the down matrices, < 0 = each
- * layer's own. */
+ * layer's own.  A kernel template: called from three kernels, the same body was
+ * scheduled 0.1 us per launch slower. */
 template <int G, int D>
-__device__ __forceinline__ void stack1r_body(const DecArgs &A)
+__global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs A)
 {
     constexpr int H = R1_H, I = R1_I, E = R1_E, HU = H / 4, nbh = H / RQK, nbi = I / RQK;
     constexpr int RD = R1_RD, SP = I / 256, RO = H / 256, RGP = I / K1_GW;
@@ -2309,13 +2316,13 @@ __device__ __forceinline__ void stack1r_body(const DecArgs &A)
              * down outputs (their SiLU*up values came in before the barrier) */
             const int rl = sdt * rpw + rw_;
             const bool live = rl < RO && lbd < nbi;
-            const float part = r1_down_row(D < 0 ? L.sq6[2] : D, sdc_s[sdt][lane], ehsh, ehshs, live, lane);
+            const float part = r1_down_row<D>(L.sq6[2], sdc_s[sdt][lane], ehsh, ehshs, live, lane);
             if (live && lr == 0) xch_put(xdsh + (size_t)gw * XCH_LN + rl, part, ep);
         }
 #pragma unroll
         for (int f = 0; f < 2; f++) {
             const int rl = (wv + f * K1_W) * rpw + rw_, row = gi * RD + rl;
-            const float part = r1_down_row(D < 0 ? L.q6[2] : D, dch[f], ehk, ehks, true, lane);
+            const float part = r1_down_row<D>(L.q6[2], dch[f], ehk, ehks, true, lane);
             if (lr == 0) xch_put(xdx + (size_t)grp * H + row, live_slot ? part : 0.0f, ep);
         }
 
@@ -2372,9 +2379,6 @@ __device__ __forceinline__ void stack1r_body(const DecArgs &A)
 #undef R1_TSW
 }
 
-extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs A) { stack1r_body<0, 1>(A); }
-extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_q4_kernel(DecArgs A) { stack1r_body<0, -1>(A); }
-extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_q6_kernel(DecArgs A) { stack1r_body<1, -1>(A); }
 
 /* ---- the batched one-launch stack: 2..8 tokens --------------------------------
  * The one-token stack's groups and exchanges with a token index: group k (an
@@ -2449,7 +2453,7 @@ __device__ __forceinline__ void k1b_gather_h(const uint64_t *lh, int H, int HU, 
     }
 }
 
-/* G, D: the matrix types as in stack1r_body. */
+/* G, D: the matrix types as in dec_stack1r_kernel. */
 template <int NB, int G, int D>
 __device__ __forceinline__ void stackB_body(const DecArgs &A)
 {
@@ -2966,8 +2970,8 @@ static bool k1_fits()
 {
     if (g_k1_fits >= 0) return g_k1_fits == 1;
     const void *fns[] = {(const void *)dec_stack1_kernel, (const void *)dec_stack1_2x2_kernel,
-                         (const void *)dec_stack1r_kernel, (const void *)dec_stack1r_q4_kernel,
-                         (const void *)dec_stack1r_q6_kernel, (const void *)dec_stackB2_kernel,
+                         (const void *)dec_stack1r_kernel<0, 1>, (const void *)dec_stack1r_kernel<0, -1>,
+                         (const void *)dec_stack1r_kernel<1, -1>, (const void *)dec_stackB2_kernel,
                          (const void *)dec_stackB4_kernel, (const void *)dec_stackB8_kernel,
                          (const void *)dec_stackB2_q4_kernel, (const void *)dec_stackB4_q4_kernel,
                          (const void *)dec_stackB8_q4_kernel, (const void *)dec_stackB2_q6_kernel,
@@ -3139,8 +3143,9 @@ static StackKernel stack1_choice(const DecArgs &A, int c0, int cn, size_t xn)
     const int npg = (A.I / K1_GW + K1_W - 1) / K1_W, nd = ((A.H / K1_GW + rpw - 1) / rpw + K1_W - 1) / K1_W;
     const int ty = stack_types(A, c0, cn);
     if (ty >= 0 && A.cnt && dec_r1_shape(A.E, A.H, A.I) && xn >= (size_t)XR_U64(A.E, A.H, A.I))
-        return ty == 0 ? STACK_KERNEL(dec_stack1r_kernel)
-                       : ty == 1 ? STACK_KERNEL(dec_stack1r_q4_kernel) : STACK_KERNEL(dec_stack1r_q6_kernel);
+        return ty == 0 ? StackKernel{ (const void *)dec_stack1r_kernel<0, 1>, "dec_stack1r_kernel" }
+             : ty == 1 ? StackKernel{ (const void *)dec_stack1r_kernel<0, -1>, "dec_stack1r_q4_kernel" }
+                       : StackKernel{ (const void *)dec_stack1r_kernel<1, -1>, "dec_stack1r_q6_kernel" };
     return npg == 2 && nd == 2 && ty == 0 ? STACK_KERNEL(dec_stack1_2x2_kernel) : STACK_KERNEL(dec_stack1_kernel);
 }
 
