@@ -304,9 +304,7 @@ __device__ __forceinline__ void mm8_prep(const float *X, int cols, int T, int kb
 }
 
 /* Lane group g's share of a super-block: 16-byte runs, so that the four lanes
- * of a row read 64 contiguous bytes a load (8-byte runs, 32 bytes a load,
- * measured 121 us on the LM head with five tokens where these take XXX).
- * Q4_K: qs bytes 64 k + 16 g (sub-blocks 4 k + 2 (g / 2), + 1); Q6_K, by half n:
+ * of a row read 64 contiguous bytes a load.  Q4_K: qs bytes 64 k + 16 g (sub-blocks 4 k + 2 (g / 2), + 1); Q6_K, by half n:
  * ql bytes 64 n + 16 g (scales 8 n + g, + 4) and the qh bytes under them. */
 struct Mm8Q4 { uint4 hd, p[2]; };
 struct Mm8Q6 { U5 l[2], h[2], sc; uint32_t d, sh; };
@@ -529,12 +527,151 @@ __global__ void __launch_bounds__(MM8_T, 4) dense_mm8_kernel(const uint8_t *W, c
     }
 }
 
+/* The same with the weights staged in LDS, for many rows: 16 waves, each on
+ * 16-row groups of its own.  Loaded where they are used, a Q6_K super-block's
+ * 16 x 210 bytes take a wave eleven loads of 64-byte pieces at 2-byte alignment,
+ * and a 128-byte line is fetched by several of them, after the CU's other waves
+ * have driven it out of its cache.  Here a wave takes them in order, 13 chunks of
+ * 16 bytes a row (Q4_K 9), with four loads and one for the last four bytes, two
+ * super-blocks in flight, and picks its quants up from its own slice of LDS.
+ * Groups go round the CUs before the waves of one.  LM head (Q6_K [248320 x
+ * 2048]), five tokens: 124.5 -> 100.4 us (4.15 TB/s); [60000 x 2048] 37.4 -> 27.9. */
+#define MM8S_T 1024
+#define MM8S_W (MM8S_T / 64)
+
+/* A lane's share of a staged super-block: its chunks; Q6_K: bytes 206..209 of
+ * the lane's own row and the shift of its bytes. */
+template <bool Q6>
+struct Mm8S {
+    static constexpr int CH = Q6 ? 13 : 9, N = 16 * CH, NL = (N + 63) / 64;   /* chunks a row (odd: 8 rows' 16-byte reads
+                                                                                  fall in different banks), a group, loads */
+    uint4 c[NL];
+    uint32_t t, sh;
+};
+
+template <bool Q6, int PARTS>
+__global__ void __launch_bounds__(MM8S_T, 1) dense_mm8s_kernel(const uint8_t *W, const float *X, float *Y, int rows, int cols,
+                                                               int T)
+{
+    extern __shared__ __align__(16) uint8_t mm8_lds[];
+    typedef Mm8S<Q6> Raw;
+    constexpr unsigned BS = Q6 ? RQ6K_BYTES : RQ4K_BYTES;
+    const int nb = cols / RQK;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g4 = lane >> 4;
+    const int ngroups = (rows + 15) >> 4, nw = gridDim.x * MM8S_W;
+    uint8_t *slice = mm8_lds + mm8_lds_bytes(cols) + wv * 16 * Raw::N;
+    /* load i of this lane: chunk ck of the group's row cr (past the last chunk
+     * that one again, to the same place) */
+    int cr[Raw::NL], ck[Raw::NL];
+#pragma unroll
+    for (int i = 0; i < Raw::NL; i++) {
+        const int idx = min(64 * i + lane, Raw::N - 1);
+        cr[i] = idx / Raw::CH;
+        ck[i] = 16 * (idx - Raw::CH * cr[i]);
+    }
+    const int g0 = wv * gridDim.x + blockIdx.x;
+    int lg = g0, lkb = 0;                               /* the next super-block to load */
+    auto rowp = [&](int r) { return W + (size_t)min(16 * min(lg, ngroups - 1) + r, rows - 1) * nb * BS; };
+    const uint8_t *wr[Raw::NL], *own;
+    auto rowset = [&]() {
+#pragma unroll
+        for (int i = 0; i < Raw::NL; i++) wr[i] = rowp(cr[i]);
+        own = rowp(lane & 15);
+    };
+    rowset();
+    auto load = [&](Raw &r) {                           /* past the last group that one again, unused */
+        typedef gu32x4 __attribute__((aligned(4))) gu32x4_a4;
+        const unsigned at = (unsigned)lkb * BS;
+#pragma unroll
+        for (int i = 0; i < Raw::NL; i++) {
+            const uint8_t *al = wr[i] + at;
+            if (Q6) al = (const uint8_t *)((uintptr_t)al & ~(uintptr_t)3);
+            const gu32x4 v = *(const GAS gu32x4_a4 *)(al + ck[i]);
+            r.c[i] = make_uint4(v.x, v.y, v.z, v.w);
+        }
+        if constexpr (Q6) {
+            typedef uint32_t __attribute__((aligned(2))) u32_a2;
+            const uint8_t *b = own + at;
+            r.t = *(const GAS u32_a2 *)(b + 206);
+            r.sh = ((uint32_t)(uintptr_t)b & 2u) * 8u;
+        }
+        if (++lkb == nb) {
+            lkb = 0;
+            lg += nw;
+            rowset();
+        }
+    };
+    Raw ra, rb;
+    load(ra);
+    load(rb);
+    for (int kb = wv; kb < nb; kb += MM8S_W) mm8_prep<Q6, PARTS>(X, cols, T, kb, mm8_lds, lane);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   /* LDS only: the weights stay in flight */
+    if (g0 >= ngroups) return;
+    float y[2] = { 0.0f, 0.0f };
+    int g = g0, kb = 0;                                 /* the super-block to compute */
+    auto step = [&](Raw &r) {                           /* whether it was the last */
+#pragma unroll
+        for (int i = 0; i < Raw::NL; i++) *(uint4 *)(slice + 16 * min(64 * i + lane, Raw::N - 1)) = r.c[i];
+        const uint32_t tail = r.t, sh = r.sh;
+        load(r);
+        const uint8_t *row = slice + (lane & 15) * (16 * Raw::CH);
+        if constexpr (Q6) {
+            auto u5 = [&](int at) { return U5{ *(const uint4 *)(row + at), *(const uint32_t *)(row + at + 16) }; };
+            Mm8Q6 q;
+#pragma unroll
+            for (int n = 0; n < 2; n++) {
+                q.l[n] = u5(64 * n + 16 * g4);
+                q.h[n] = u5(128 + 32 * n + 16 * (g4 & 1));
+            }
+            q.sc = U5{ *(const uint4 *)(row + 192), tail };
+            q.d = tail >> 16;
+            q.sh = sh;
+            mm8_add<true, PARTS>(q, mm8_lds, cols, kb, true, lane, y);
+        } else {
+            Mm8Q4 q;
+            q.hd = *(const uint4 *)row;
+#pragma unroll
+            for (int k = 0; k < 2; k++) q.p[k] = *(const uint4 *)(row + 16 + 64 * k + 16 * g4);
+            mm8_add<false, PARTS>(q, mm8_lds, cols, kb, true, lane, y);
+        }
+        if (++kb != nb) return false;
+        mm8_store<PARTS>(Y, rows, T, 16 * g + (lane & 15), lane, y);
+        y[0] = y[1] = 0.0f;
+        kb = 0;
+        g += nw;
+        return g >= ngroups;
+    };
+    for (;;) {
+        if (step(ra)) break;
+        if (step(rb)) break;
+    }
+}
+
 int dense_mfma_min_tokens() { return g_dense_mfma_t; }
 
 int dense_mm8_launch(const uint8_t *W, int q6, const float *X, float *Y, size_t rows, size_t cols, int T)
 {
     const size_t lds = mm8_lds_bytes(cols);
     const size_t ng = (rows + 15) / 16;
+    const size_t slds = lds + MM8S_W * 256 * (q6 ? Mm8S<true>::CH : Mm8S<false>::CH);
+    const dim3 gs((unsigned)rt().n_cu), bs(MM8S_T);
+#define MM8S(Q6_, P_) hipLaunchKernelGGL((dense_mm8s_kernel<Q6_, P_>), gs, bs, slds, rt().stream, W, X, Y, (int)rows, (int)cols, T)
+    /* staged from 4 groups per CU on (256 CUs: 16384 rows), where a wave with a
+     * group to itself is no longer short of others (Q6_K / Q4_K, five tokens:
+     * [16384 x 768] 7.3 / 5.7 us staged, 7.9 / 5.7 not; [8192 x 2048] 11.8 / 8.4
+     * and 11.0 / 8.4), while the slices fit beside the activations (Q6_K: 3328
+     * columns) */
+    if (ng >= 4 * (size_t)rt().n_cu && slds <= 160 * 1024) {
+        if (T <= 4) {
+            if (q6) MM8S(true, 3);
+            else MM8S(false, 3);
+        } else {
+            if (q6) MM8S(true, 2);
+            else MM8S(false, 2);
+        }
+#undef MM8S
+        return rt_check(hipGetLastError(), "dense MFMA launch") ? ROASTER_EDEVICE : 0;
+    }
     const size_t cap = (size_t)(lds <= 78 * 1024 ? 2 : 1) * rt().n_cu;
     const int nb = (int)(cols / RQK);
     /* waves per group: the split whose waves run the fewest super-blocks one

@@ -7,7 +7,7 @@ scales over the whole int8 range (sc (q - 32) past 2048 needs the second weight
 operand).  One token runs the pipelined matvec on the same shapes.
 
 Bar 5e-6 of max|y|: 22-bit activations (2^-22 per product, random in sign) and
-f32 sums of up to 2304 terms on both sides, about 1e-6 each."""
+f32 sums of up to 3584 terms on both sides, about 1e-6 each."""
 import numpy as np
 import pytest
 
@@ -31,5 +31,21 @@ def test_splits(q6, rows, cols):
     for T in (1, 2, 4, 5, 8):
         Y = run(q6, W, X[:T], rows, cols)
         for t in range(T):
+            err = np.max(np.abs(Y[t] - ref[t])) / np.max(np.abs(ref[t]))
+            assert err <= 5e-6, (T, t, err)
+
+
+@pytest.mark.parametrize("q6", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(16368, 256), (16369, 512), (16400, 3328), (16400, 3584)])
+def test_staged(q6, rows, cols):
+    """The weights staged in LDS (from 1024 16-row groups on 256 CUs): the last
+    size before and the first after, the widest that fits with Q6_K and one
+    past it."""
+    W = weights(q6, rows, cols, 90 + cols)
+    X = np.stack([R.synth_normal(91, R.synth_stream(t, cols, 5), cols) for t in range(6)])
+    ref = {t: O.matvec(q6, W, X[t], rows, cols) for t in (0, 1, 5)}
+    for T in (2, 6):
+        Y = run(q6, W, X[:T], rows, cols)
+        for t in (t for t in ref if t < T):
             err = np.max(np.abs(Y[t] - ref[t])) / np.max(np.abs(ref[t]))
             assert err <= 5e-6, (T, t, err)
