@@ -166,8 +166,8 @@ int roaster_moe_decode_stack(RoasterTable *t, float *h, int B, int layer0, int n
  * combine in 256 workgroups that exchange values through memory) wherever the
  * shapes allow it: a device with at least 256 CUs on which each one-launch
  * kernel fits one workgroup per CU, experts a multiple of 32 up to 256; for
- * one token hidden up to 2048 and inter up to 1024; for 2..8 tokens inter 512,
- * hidden 512..2048 in multiples of 256, and gate and up matrices, routed and
+ * one token hidden up to 2048 and inter up to 1024; for 2..8 tokens inter 512 or
+ * 256, hidden 512..2048 in multiples of 256, and gate and up matrices, routed and
  * shared, of one type in every layer of the call (down matrices of either).
  * Otherwise each layer runs as three launches.
  * One token at 256 experts, hidden 2048, inter 512 with gate and up matrices of

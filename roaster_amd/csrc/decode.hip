@@ -12,14 +12,15 @@
  * workgroups serve routed slot k of every token (the k-th selected expert);
  * the shared expert and the router are spread over all 256.
  *   dec_stack1r_kernel   one token, 256 experts / hidden 2048 / inter 512,
- *                        gate/up Q4_K and down Q6_K: the router folded into
+ *                        gate and up of one type: the router folded into
  *                        the previous layer's combine (partial logits over
  *                        each workgroup's combined rows, summed across XCDs);
  *   dec_stack1_kernel,   one token, any other shape the launch takes (2x2:
  *   dec_stack1_2x2_kernel  two gate/up pairs and two down tasks per wave),
  *                        with the three-kernel path's arithmetic;
- *   dec_stackB2/4/8_kernel  2..8 tokens, each token's results equal to its
- *                        one-token result on the three-kernel arithmetic.
+ *   dec_stackB2/4/8_*kernel  2..8 tokens, inter 512 or 256, gate and up of one
+ *                        type, each token's results equal to its one-token
+ *                        result on the three-kernel arithmetic.
  * A stack call's final h is staged and copied over the caller's only when no
  * wait gave up anywhere (k1_finish).
  *
@@ -2411,8 +2412,8 @@ __global__ void __launch_bounds__(K1_T, 1) dec_stack1r_kernel(DecArgs A)
  * layer parity.
  * Every dot, sum, softmax and combine is the one-token kernel's, in its order,
  * so each token's results equal its one-token results bit for bit.  Shapes:
- * inter 512, hidden 512..2048 in whole 256-row blocks, at most 256 experts
- * (dec_layerB_ok); matrix types as in stack_types. */
+ * inter 512 or 256, hidden 512..2048 in whole 256-row blocks, at most 256
+ * experts (dec_layerB_ok); matrix types as in stack_types. */
 template <int NB>
 __device__ __forceinline__ void k1b_gather_h(const uint64_t *lh, int H, int HU, int u, int b0, int B, uint32_t ep,
                                              int &dead, uint32_t spin, float (*xn)[K1_MAXH])
@@ -2453,17 +2454,17 @@ __device__ __forceinline__ void k1b_gather_h(const uint64_t *lh, int H, int HU, 
     }
 }
 
-/* G, D: the matrix types as in dec_stack1r_kernel. */
-template <int NB, int G, int D>
+/* G, D: the matrix types as in dec_stack1r_kernel; I: inter, 512 or 256. */
+template <int NB, int G, int D, int I = 512>
 __device__ __forceinline__ void stackB_body(const DecArgs &A)
 {
     __shared__ __align__(16) float xn[NB][K1_MAXH];
     __shared__ float xsum[NB][K1_MAXH / 16];
     __shared__ float hown[NB][64];                           /* the owned rows' residual */
-    __shared__ __align__(16) float ehk[NB][512];
-    __shared__ float ehks[NB][512 / 16];
-    __shared__ __align__(16) float ehsh[NB][512];
-    __shared__ float ehshs[NB][512 / 16];
+    __shared__ __align__(16) float ehk[NB][I];
+    __shared__ float ehks[NB][I / 16];
+    __shared__ __align__(16) float ehsh[NB][I];
+    __shared__ float ehshs[NB][I / 16];
     __shared__ TopkScratch tks[NB];
     __shared__ int ids_s[NB][RTOPK];
     __shared__ float w_s[NB][RTOPK + 1];
@@ -2480,7 +2481,9 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
     __shared__ int s_ids_rdy[NB];                             /* layer index + 1 once token b's ids are in */
     __shared__ int s_eh_rdy[NB];                              /* ... once its SiLU*up vectors are in */
 
-    constexpr int I = 512, nbi = 2, SP = 2, RGP = I / K1_GW;
+    /* per workgroup: SP shared pairs, RGP routed gate/up rows (F a wave), and at
+     * most FD down tasks a wave (H <= 2048) */
+    constexpr int nbi = I / RQK, SP = I / 256, RGP = I / K1_GW, F = RGP / K1_W, FD = I / 256;
     const int H = A.H, E = A.E, B = A.B, HU = H / 4, nbh = H / RQK;
     const int tid = threadIdx.x, wv = wave_id();
     unsigned xcc;
@@ -2717,16 +2720,16 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
         float sg = 0.0f;
         {
             constexpr int DG = 2;                            /* tokens' gate/up rows in flight */
-            QChunk2 st[DG][2];
-            auto gu_load = [&](int b, QChunk2 (&ch)[2]) {
+            QChunk2 st[DG][F];
+            auto gu_load = [&](int b, QChunk2 (&ch)[F]) {
                 k1_flag_wait(&s_ids_rdy[min(b, B - 1)], li + 1);
                 const int e = __builtin_amdgcn_readfirstlane(ids_s[min(b, B - 1)][grp]);   /* wave-uniform */
                 const size_t ee = e >= 0 ? (size_t)e : 0;
                 const uint8_t *ge = L.gate + ee * L.eb[0], *ue = L.up + ee * L.eb[1];
 #pragma unroll
-                for (int f = 0; f < 2; f++) ch[f].g = q_load_t(G, ge, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
+                for (int f = 0; f < F; f++) ch[f].g = q_load_t(G, ge, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
 #pragma unroll
-                for (int f = 0; f < 2; f++) ch[f].u = q_load_t(G, ue, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
+                for (int f = 0; f < F; f++) ch[f].u = q_load_t(G, ue, (size_t)gi * RGP + wv + f * K1_W, nbh, lb, c);
             };
 #pragma unroll
             for (int b = 0; b < DG - 1; b++) gu_load(b, st[b]);
@@ -2746,10 +2749,10 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
                 if (b >= B) break;
                 const bool live_slot = ids_s[b][grp] >= 0;
                 if (b + DG - 1 < NB) gu_load(b + DG - 1, st[(b + DG - 1) % DG]);   /* past the last token: unused */
-                QChunk2 (&cur)[2] = st[b % DG];
+                QChunk2 (&cur)[F] = st[b % DG];
                 /* the wave's four rows share one read of the token's x
                  * (k1_q_row's arithmetic per row) */
-                float pg[2] = {0.0f, 0.0f}, pu[2] = {0.0f, 0.0f};
+                float pg[F] = {}, pu[F] = {};
                 if (lb < nbh) {
                     const int xa = lb * RQK + q_run_a_t(G, c), xb = xa + (G ? 64 : 32);
                     float4 x0[4], x1[4];
@@ -2757,12 +2760,12 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
                     load_x16(xn[b], xb, x1, swz);
                     const float sa = xsum[b][xa >> 4], sb = xsum[b][xb >> 4];
 #pragma unroll
-                    for (int f = 0; f < 2; f++) {
+                    for (int f = 0; f < F; f++) {
                         pg[f] = q_chunk_dot_r<G != 0>(cur[f].g, c, x0, x1, sa, sb);
                         pu[f] = q_chunk_dot_r<G != 0>(cur[f].u, c, x0, x1, sa, sb);
                     }
                 }
-                if constexpr (NB <= 4) {
+                if constexpr (NB <= 4 && F == 2) {
                     /* both rows' SiLU*up in one pass: lane 0 row wv, lane 1 row
                      * wv + 8 (with 8 slots measured slower) */
                     const float g0 = group_sum<64>(pg[0]), u0 = group_sum<64>(pu[0]);
@@ -2774,7 +2777,7 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
                                     ep, l2);
                 } else {
 #pragma unroll
-                    for (int f = 0; f < 2; f++) {
+                    for (int f = 0; f < F; f++) {
                         const int pj = wv + f * K1_W;
                         const float eh = silu_mul(group_sum<64>(pg[f]), group_sum<64>(pu[f]));
                         if (lane == 0)
@@ -2786,13 +2789,13 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
         K1_TS(5);
         {
             constexpr int DD = 2;                            /* tokens' down rows in flight */
-            QChunk st[DD][2];
-            auto dn_load = [&](int b, QChunk (&ch)[2]) {
+            QChunk st[DD][FD];
+            auto dn_load = [&](int b, QChunk (&ch)[FD]) {
                 const int e = __builtin_amdgcn_readfirstlane(ids_s[min(b, B - 1)][grp]);   /* wave-uniform */
                 const size_t ee = e >= 0 ? (size_t)e : 0;
                 const uint8_t *de = L.down + ee * L.eb[2];
 #pragma unroll
-                for (int f = 0; f < 2; f++) {
+                for (int f = 0; f < FD; f++) {
                     const int task = min(wv + f * K1_W, ndt - 1);
                     ch[f] = q_load_d<D>(L.q6[2], de, (size_t)min(gi * RD + task * rpw + rw_, H - 1), nbi, lbd, lr & 7);
                 }
@@ -2835,10 +2838,10 @@ __device__ __forceinline__ void stackB_body(const DecArgs &A)
                 if (b >= B) break;
                 const bool live_slot = ids_s[b][grp] >= 0;
                 if (b + DD - 1 < NB) dn_load(b + DD - 1, st[(b + DD - 1) % DD]);
-                QChunk (&cur)[2] = st[b % DD];
+                QChunk (&cur)[FD] = st[b % DD];
                 k1_flag_wait(&s_eh_rdy[b], li + 1);
 #pragma unroll
-                for (int f = 0; f < 2; f++) {
+                for (int f = 0; f < FD; f++) {
                     const int task = wv + f * K1_W;
                     if (task < ndt) {
                         const int rl = task * rpw + rw_, row = gi * RD + rl;
@@ -2902,7 +2905,12 @@ extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB8_q4_kernel(DecA
 extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB2_q6_kernel(DecArgs A) { stackB_body<2, 1, -1>(A); }
 extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB4_q6_kernel(DecArgs A) { stackB_body<4, 1, -1>(A); }
 extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB8_q6_kernel(DecArgs A) { stackB_body<8, 1, -1>(A); }
-
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB2_i256_q4_kernel(DecArgs A) { stackB_body<2, 0, -1, 256>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB4_i256_q4_kernel(DecArgs A) { stackB_body<4, 0, -1, 256>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB8_i256_q4_kernel(DecArgs A) { stackB_body<8, 0, -1, 256>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB2_i256_q6_kernel(DecArgs A) { stackB_body<2, 1, -1, 256>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB4_i256_q6_kernel(DecArgs A) { stackB_body<4, 1, -1, 256>(A); }
+extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_stackB8_i256_q6_kernel(DecArgs A) { stackB_body<8, 1, -1, 256>(A); }
 
 /* Every workgroup's XCC_ID, in a grid of the stack kernel's shape. */
 extern "C" __global__ void __launch_bounds__(K1_T, 1) dec_xcd_probe_kernel(unsigned *out)
@@ -2975,7 +2983,10 @@ static bool k1_fits()
                          (const void *)dec_stackB4_kernel, (const void *)dec_stackB8_kernel,
                          (const void *)dec_stackB2_q4_kernel, (const void *)dec_stackB4_q4_kernel,
                          (const void *)dec_stackB8_q4_kernel, (const void *)dec_stackB2_q6_kernel,
-                         (const void *)dec_stackB4_q6_kernel, (const void *)dec_stackB8_q6_kernel};
+                         (const void *)dec_stackB4_q6_kernel, (const void *)dec_stackB8_q6_kernel,
+                         (const void *)dec_stackB2_i256_q4_kernel, (const void *)dec_stackB4_i256_q4_kernel,
+                         (const void *)dec_stackB8_i256_q4_kernel, (const void *)dec_stackB2_i256_q6_kernel,
+                         (const void *)dec_stackB4_i256_q6_kernel, (const void *)dec_stackB8_i256_q6_kernel};
     bool ok = rt().n_cu >= K1_NWG;
     for (const void *f : fns) {
         int nb = 0;
@@ -3035,13 +3046,13 @@ bool dec_layer1_ok(int E, int H, int I, int B)
            H <= K1_MAXH && I % RQK == 0 && I <= K1_MAXI;
 }
 
-/* The batched kernel's shapes: inter 512 (two gate/up rows and two down
- * tasks per wave), hidden 512..2048 in whole 256-row blocks, at most 256
+/* The batched kernels' shapes: inter 512 (two gate/up rows and two down
+ * tasks per wave) or 256 (one and one), hidden 512..2048 in whole 256-row blocks, at most 256
  * experts (one logit per lane of a wave's 64 for 8 tokens). */
 bool dec_layerB_ok(int E, int H, int I, int B)
 {
     return g_layer1 && B >= 2 && B <= K1B_MAXB && k1_fits() && E >= RTOPK && E <= 256 && E % K1_GW == 0 &&
-           I == 512 && H % 256 == 0 && H >= 512 && H <= K1_MAXH;
+           (I == 512 || I == 256) && H % 256 == 0 && H >= 512 && H <= K1_MAXH;
 }
 
 static DecXch g_xch;
@@ -3154,11 +3165,20 @@ static StackKernel stack1_choice(const DecArgs &A, int c0, int cn, size_t xn)
  * against those, us per layer of 16 with down types mixed by layer: 2 tokens
  * 34.2 -> 20.2, 3 41.2 -> 26.5, 8 74.3 -> 51.4 (the run-time down type costs
  * the 8-slot kernel 2.7 over the fixed one); one all-Q6_K layer of 4 tokens
- * 46.4 -> 35.9. */
+ * 46.4 -> 35.9.  Inter 256: 2 tokens 26.9 -> 15.3, 4 35.7 -> 21.6, 8 61.0 ->
+ * 34.4; one layer of 5 tokens 41.5 -> 27.7. */
 static StackKernel stackB_choice(const DecArgs &A, int l0, int n)
 {
-    const int B = A.B;
-    switch (stack_types(A, l0, n)) {
+    const int B = A.B, ty = stack_types(A, l0, n);
+    if (A.I == 256) {                     /* either down type at run time */
+        if (ty < 0) return StackKernel{ NULL, NULL };
+        if (ty == 2)
+            return B <= 2 ? STACK_KERNEL(dec_stackB2_i256_q6_kernel)
+                          : B <= 4 ? STACK_KERNEL(dec_stackB4_i256_q6_kernel) : STACK_KERNEL(dec_stackB8_i256_q6_kernel);
+        return B <= 2 ? STACK_KERNEL(dec_stackB2_i256_q4_kernel)
+                      : B <= 4 ? STACK_KERNEL(dec_stackB4_i256_q4_kernel) : STACK_KERNEL(dec_stackB8_i256_q4_kernel);
+    }
+    switch (ty) {
     case 0:
         return B <= 2 ? STACK_KERNEL(dec_stackB2_kernel) : B <= 4 ? STACK_KERNEL(dec_stackB4_kernel) : STACK_KERNEL(dec_stackB8_kernel);
     case 1:

@@ -86,3 +86,26 @@ def test_types(mix, shape, B):
         assert err <= 1e-4
     finally:
         t.destroy()
+
+
+@pytest.mark.parametrize("mix", sorted(MIXES))
+@pytest.mark.parametrize("shape", [(256, 2048), (64, 768), (32, 512)], ids=lambda s: "E%d-H%d" % s)
+@pytest.mark.parametrize("B", [2, 3, 8])
+def test_inter_256_in_one_launch(shape, mix, B):
+    """Inter 256 (one row per wave, one super-block per down row): bit for bit
+    the three kernels' results, ids equal to the oracle's."""
+    E, H = shape
+    NL = len(MIXES[mix])
+    t = LayerTable(61, MIXES[mix], n_experts=E, hidden=H, inter=256)
+    try:
+        name = R.lib().roaster_decode_stack_kernel(t.t, B, 0, NL).decode()
+        assert name.endswith("_i256_q6_kernel" if mix == "q6" else "_i256_q4_kernel"), name
+        h0 = np.stack([R.synth_normal(61, R.synth_stream(0, b, 5), H) for b in range(B)])
+        nw = np.stack([1.0 + 0.25 * R.synth_normal(62, R.synth_stream(l, 0, 6), H) for l in range(NL)]).astype(np.float32)
+        a = _stack(t, h0, NL, nw)
+        _same(a, _in_mode(0, lambda: _stack(t, h0, NL, nw)))
+        h_ref, ids_ref = oracle_stack(t, h0, NL, norm_w=nw)
+        assert np.array_equal(a[1], ids_ref)
+        assert rel_err(a[0] - h0, h_ref - h0) <= 1e-4
+    finally:
+        t.destroy()
