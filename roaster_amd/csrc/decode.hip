@@ -51,6 +51,7 @@
 #include "qdot.h"
 #include "topk.h"
 #include "decode.h"
+#include "down_lds.h"
 
 #include <stdio.h>
 #include <string.h>
@@ -887,20 +888,20 @@ __device__ void down_slots(const DecArgs &A, const uint8_t *const *sd, int k0, i
     }
 }
 
-/* Down rows and combine for one token when the 9 down matrices share one
- * type D6 (A.d1, set per launch): each wave reads its tasks' slot pointers
- * straight from the published plan and issues the weight-row loads as soon
- * as they arrive, before the SiLU*up rows are stored to LDS, so the rows'
+/* Down rows and combine for one token when the slots' down matrices (nine, or
+ * kernel_ffn_fused's experts) share one type D6 (A.d1, set per launch): each
+ * wave reads its tasks' slot pointers straight from the published plan and
+ * issues the weight-row loads as soon as they arrive, before the SiLU*up rows are stored to LDS, so the rows'
  * memory latency overlaps the copy, the barriers and the run sums.  Tasks as
  * in down_slots (q = k * ngroups + g, wave w takes q = w, w + 4, ...; the
  * host checks that D_PF tasks per wave cover them); loads are unconditional
  * (clamped task, row and block; an unselected slot reads the shared slot's
  * matrix) and the copy's stores wait for the copy's loads only. */
 template <bool D6>
-__device__ __forceinline__ void down_one_token(const DecArgs &A, int dr, float *ehl, float *ehs, float *dbuf, float *sw)
+__device__ __forceinline__ void down_one_token(const DecArgs &A, int dr, const DownLds S, float *ehl, float *dbuf, float *sw)
 {
     const int H = A.H, I = A.I, nb = I / RQK, tid = threadIdx.x, lane = tid & 63, wv = wave_id();
-    const int lpr = lanes_per_row(nb), rpw = 64 / lpr, ngroups = (dr + rpw - 1) / rpw, ntask = 9 * ngroups;
+    const int lpr = lanes_per_row(nb), rpw = 64 / lpr, ngroups = (dr + rpw - 1) / rpw, ntask = S.n * ngroups;
     const int rw = lane / lpr, lr = lane % lpr, c = lr & 7, lb = lr >> 3;
     const int r0 = blockIdx.x * dr;
     const size_t dbs = D6 ? RQ6K_BYTES : RQ4K_BYTES;
@@ -911,15 +912,15 @@ __device__ __forceinline__ void down_one_token(const DecArgs &A, int dr, float *
     const uint8_t *mp[D_PF];
 #pragma unroll
     for (int f = 0; f < D_PF; f++) mp[f] = PG->dsl[0][min(wv + f * DW, ntask - 1) / ngroups];
-    const uint8_t *fb = PG->dsl[0][A.ffn_out ? 0 : 8];   /* always set */
+    const uint8_t *fb = PG->dsl[0][S.n - 1];                /* always set */
     const float wk = PG->w[0][min(tid, 8)];
-    /* the SiLU*up rows: 9 x I / 4 16-byte units, 5 per thread (I <= 568), in
-     * named registers (an array here is not kept in registers across the
-     * scheduling fences) */
-    const int n16 = 9 * I / 4;
+    /* the SiLU*up rows: at most 9 x I / 4 16-byte units, 5 per thread (I <=
+     * 568), in named registers (an array here is not kept in registers across
+     * the scheduling fences) */
+    const int u0 = S.unit(tid), u1 = S.unit(tid + DT), u2 = S.unit(tid + 2 * DT), u3 = S.unit(tid + 3 * DT);
+    const int u4 = S.unit(tid + 4 * DT);
     const uint4 *eh4 = (const uint4 *)A.eh;
-    const uint4 e0 = eh4[min(tid, n16 - 1)], e1 = eh4[min(tid + DT, n16 - 1)], e2 = eh4[min(tid + 2 * DT, n16 - 1)];
-    const uint4 e3 = eh4[min(tid + 3 * DT, n16 - 1)], e4 = eh4[min(tid + 4 * DT, n16 - 1)];
+    const uint4 e0 = eh4[u0], e1 = eh4[u1], e2 = eh4[u2], e3 = eh4[u3], e4 = eh4[u4];
     __builtin_amdgcn_sched_barrier(0);
     QChunk ch[D_PF];
 #pragma unroll
@@ -931,15 +932,16 @@ __device__ __forceinline__ void down_one_token(const DecArgs &A, int dr, float *
     }
     __builtin_amdgcn_sched_barrier(0);
     uint4 *el4 = (uint4 *)ehl;
-    el4[min(tid, n16 - 1)] = e0;
-    el4[min(tid + DT, n16 - 1)] = e1;
-    el4[min(tid + 2 * DT, n16 - 1)] = e2;
-    el4[min(tid + 3 * DT, n16 - 1)] = e3;
-    el4[min(tid + 4 * DT, n16 - 1)] = e4;
+    el4[u0] = e0;
+    el4[u1] = e1;
+    el4[u2] = e2;
+    el4[u3] = e3;
+    el4[u4] = e4;
+    float *ehs = ehl + S.sums_at();
     sw[min(tid, 8)] = wk;                                   /* threads past 8 store slot 8's weight again */
     for (int i = tid; i < 9 * D_MAXR; i += DT) dbuf[i] = 0.0f;
     __syncthreads();
-    for (int r = tid; r < 9 * (I / 16); r += DT) ehs[r] = sum16(ehl + r * 16);
+    for (int r = tid; r < S.sums(); r += DT) ehs[r] = sum16(ehl + r * 16);
     __syncthreads();
     PHASE_TS(2, 1);
 #pragma unroll
@@ -994,11 +996,12 @@ extern "C" __global__ void __launch_bounds__(DT, 3) dec_down_kernel(DecArgs A, i
     const int nrb = (H + dr - 1) / dr, t = blockIdx.x / nrb, r0 = (blockIdx.x % nrb) * dr;
     const bool ffn = A.ffn_out != NULL;
     const int nslot = ffn ? A.ffn_n : 9;
+    const DownLds S = { nslot, I };
     PHASE_TS(2, 0);
-    float *ehl = lds, *ehs = lds + nslot * I;
+    float *ehl = lds, *ehs = lds + S.sums_at();
     if (A.d1) {
-        if (A.d1 == 2) down_one_token<true>(A, dr, ehl, ehs, dbuf, sw);
-        else down_one_token<false>(A, dr, ehl, ehs, dbuf, sw);
+        if (A.d1 == 2) down_one_token<true>(A, dr, S, ehl, dbuf, sw);
+        else down_one_token<false>(A, dr, S, ehl, dbuf, sw);
         return;
     }
     /* slot table (published with the plan): its loads are unconditional,
@@ -1009,14 +1012,14 @@ extern "C" __global__ void __launch_bounds__(DT, 3) dec_down_kernel(DecArgs A, i
     const float wk = A.plan_g->w[t][ks];
     const int qk = A.plan_g->dq6k[ks];
     for (int i = tid; i < 9 * D_MAXR; i += DT) dbuf[i] = 0.0f;
-    block_copy16(ehl, A.eh + (size_t)(ffn ? 0 : t * 9) * I, nslot * I / 4);
+    block_copy16(ehl, A.eh + (size_t)(ffn ? 0 : t * 9) * I, S.units());
     if (tid < 9) {
         sd[tid] = pk;
         sw[tid] = wk;
         sq[tid] = qk;
     }
     __syncthreads();
-    for (int r = tid; r < nslot * (I / 16); r += DT) ehs[r] = sum16(ehl + r * 16);
+    for (int r = tid; r < S.sums(); r += DT) ehs[r] = sum16(ehl + r * 16);
     __syncthreads();
     const int lpr = lanes_per_row(nb), rpw = 64 / lpr;
     const int ngroups = (dr + rpw - 1) / rpw;
@@ -2953,7 +2956,7 @@ static int launch_layer(const DecArgs &A0, int l, bool with_router)
     else hipLaunchKernelGGL(dec_gu_kernel, dim3(2 * R.n_cu), dim3(DT), lds, R.stream, A, l);
     if (rt_check(hipGetLastError(), "gate/up launch")) return ROASTER_EDEVICE;
     const int nslot = A.ffn_out ? A.ffn_n : 9, dr = A.B > 1 ? D_ROWS_B : D_ROWS;
-    const size_t dlds = (size_t)nslot * A.I * 4 + (size_t)nslot * (A.I / 16) * 4;
+    const size_t dlds = DownLds{ nslot, A.I }.bytes();
     const int nrb = (A.H + dr - 1) / dr;
     hipLaunchKernelGGL(dec_down_kernel, dim3(nrb * (A.ffn_out ? 1 : A.B)), dim3(DT), dlds, R.stream, A, l, dr);
     return rt_check(hipGetLastError(), "down launch") ? ROASTER_EDEVICE : 0;
