@@ -512,8 +512,13 @@ __global__ void __launch_bounds__(256, 4) pf_token_kernel(PfTokArgs A, PfPlanArg
     __shared__ TopkScratch ts[4];
     __shared__ int s_ids[4][RTOPK];
     __shared__ float s_w[4][RTOPK];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int t = min(blockIdx.x * 4 + wv, A.T - 1);    /* waves past T: token T - 1 again, the same values */
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    /* waves past T only take part in PLAN's barriers: they read token T - 1
+     * (whose logits its own wave may be replacing, logits_out == logits_in) and
+     * store nothing */
+    const bool live = (int)blockIdx.x * 4 + wv < A.T;
+    if (!PLAN && !live) return;
+    const int t = min((int)blockIdx.x * 4 + wv, A.T - 1);
     /* The token's logits (or router partial sums) and biases are loaded
      * first, then its X row (H <= 2048: at most 8 float4 per lane) and the
      * gate vector, indices clamped.  A wave's loads complete in order, so
@@ -562,7 +567,7 @@ __global__ void __launch_bounds__(256, 4) pf_token_kernel(PfTokArgs A, PfPlanArg
         if (e < A.E) {
             l = v4[i];
             if (A.bias) l = l + b4[i];
-            if (A.logits_out) A.logits_out[(size_t)t * A.E + e] = l;
+            if (A.logits_out && live) A.logits_out[(size_t)t * A.E + e] = l;
         }
         v4[i] = l;
     }
@@ -570,7 +575,7 @@ __global__ void __launch_bounds__(256, 4) pf_token_kernel(PfTokArgs A, PfPlanArg
     __builtin_amdgcn_wave_barrier();
     topk8_fast(v4, A.E, s_ids[wv], s_w[wv], &bad[wv], &ts[wv]);
     __builtin_amdgcn_wave_barrier();
-    if (lane < 8) {
+    if (live && lane < 8) {
         const int id = s_ids[wv][lane];
         const float w = s_w[wv][lane];
         if constexpr (PLAN)
@@ -603,7 +608,7 @@ __global__ void __launch_bounds__(256, 4) pf_token_kernel(PfTokArgs A, PfPlanArg
     dot = group_sum<64>(dot);
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
-    if (A.xinv) {
+    if (A.xinv && live) {
         float inv, fwd;
         if (A.x16l) row_scale_wide(mx, inv, fwd);
         else row_scale(mx, inv, fwd);
@@ -643,8 +648,10 @@ __global__ void __launch_bounds__(256, 4) pf_token_kernel(PfTokArgs A, PfPlanArg
             }
         }
     }
-    if (lane == 0) A.sg[t] = 1.0f / (1.0f + expf(-dot));
-    if (lane == 0 && bad[wv]) atomicOr(A.err, 1);
+    if (live && lane == 0) {
+        A.sg[t] = 1.0f / (1.0f + expf(-dot));
+        if (bad[wv]) atomicOr(A.err, 1);
+    }
     if constexpr (PLAN) {
         __shared__ int last;
         if (threadIdx.x == 0) last = ndone == (int)gridDim.x - 1;
