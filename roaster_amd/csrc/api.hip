@@ -259,7 +259,7 @@ extern "C" int kernel_matmul_quant_batch(const KernelMatmulJob *jobs, int n)
             rt_check(hipMemcpyAsync(dx + xoff[i], j.X, j.T * j.cols * 4, hipMemcpyHostToDevice, R.stream), "X upload"))
             return -1;
         const bool big = j.T >= MM_MFMA_MIN_T && j.rows % GEMM_ROWS == 0;
-        if (!big && (int)j.T >= dense_mfma_min_tokens() && j.cols <= 4096) {
+        if (!big && dense_mm8_takes(W, j.is_q6 ? 1 : 0, j.cols, j.T)) {
             /* a few tokens: the quants-on-MFMA product, eight tokens per launch */
             for (size_t t0 = 0; t0 < j.T; t0 += 8)
                 if (dense_mm8_launch(W, j.is_q6 ? 1 : 0, (const float *)(dx + xoff[i]) + t0 * j.cols,

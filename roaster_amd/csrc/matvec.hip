@@ -90,14 +90,15 @@ __device__ __forceinline__ uint4 u5_fix(const U5 &a, uint32_t sh)
                       __builtin_amdgcn_alignbit(a.v.w, a.v.z, sh), __builtin_amdgcn_alignbit(a.w, a.v.w, sh));
 }
 
-/* A lane's chunk as loaded (q_load's bytes) and the QChunk it stands for. */
-template <bool Q6> struct QRaw;
-template <> struct QRaw<false> {
+/* A lane's chunk as loaded (q_load's bytes) and the QChunk it stands for.  DW:
+ * as the aligned dwords around it, for Q6_K blocks at even addresses (a block
+ * is 210 bytes, so all of a matrix's are even or none). */
+template <bool Q6, bool DW> struct QRaw {
     QChunk ch;
-    __device__ __forceinline__ void load(const uint8_t *blk, int c) { ch = q_load<false>(blk, c); }
+    __device__ __forceinline__ void load(const uint8_t *blk, int c) { ch = q_load<Q6>(blk, c); }
     __device__ __forceinline__ QChunk chunk() const { return ch; }
 };
-template <> struct QRaw<true> {
+template <> struct QRaw<true, true> {
     U5 q, h;
     uint32_t s[3], dd, sh;
     __device__ __forceinline__ void load(const uint8_t *blk, int c)
@@ -125,7 +126,7 @@ template <> struct QRaw<true> {
     }
 };
 
-template <bool Q6, bool ONE, int KB>
+template <bool Q6, bool ONE, int KB, bool DW = Q6>
 __global__ void __launch_bounds__(MV_THREADS) dense_mv_kernel(const uint8_t *W, const float *X, float *Y, int rows,
                                                               int cols, int T)
 {
@@ -170,14 +171,14 @@ __global__ void __launch_bounds__(MV_THREADS) dense_mv_kernel(const uint8_t *W, 
     /* the next pass's chunks are in flight while the current one's are dotted;
      * rows and blocks past the end read the last one, unused, so that the loads
      * carry no branches and each wait counts its own loads only */
-    QRaw<Q6> cur[KB], nxt[KB];
-    auto load = [&](QRaw<Q6> (&ch)[KB], int pass) {
+    QRaw<Q6, DW> cur[KB], nxt[KB];
+    auto load = [&](QRaw<Q6, DW> (&ch)[KB], int pass) {
         const int row = min(min(pass, npass - 1) * rpw + rw, rows - 1);
 #pragma unroll
         for (int k = 0; k < KB; k++)
             ch[k].load(W + (size_t)row * row_bytes + (size_t)min(lb + 8 * k, nb - 1) * bs, c);
     };
-    auto compute = [&](const QRaw<Q6> (&ch)[KB], int pass) {
+    auto compute = [&](const QRaw<Q6, DW> (&ch)[KB], int pass) {
         const int row = pass * rpw + rw;
         const bool live = row < rows;
         QChunk qc[KB];
@@ -647,7 +648,12 @@ __global__ void __launch_bounds__(MM8S_T, 1) dense_mm8s_kernel(const uint8_t *W,
     }
 }
 
-int dense_mfma_min_tokens() { return g_dense_mfma_t; }
+static bool mat_odd(const uint8_t *W, int q6) { return q6 && ((uintptr_t)W & 1); }
+
+bool dense_mm8_takes(const uint8_t *W, int q6, size_t cols, size_t T)
+{
+    return T >= (size_t)g_dense_mfma_t && cols <= 4096 && !mat_odd(W, q6);
+}
 
 int dense_mm8_launch(const uint8_t *W, int q6, const float *X, float *Y, size_t rows, size_t cols, int T)
 {
@@ -747,7 +753,7 @@ extern "C" int roaster_matvec_q(const void *W, int q6, const float *X, float *Y,
     if (rt_init_locked()) return ROASTER_EDEVICE;
     if (!W || !X || !Y || !rows || !cols || cols % RQK || cols > 4096 || T < 1 || T > 8 || rows > (size_t)INT32_MAX)
         return rt_fail(ROASTER_EINVAL, "roaster_matvec_q: need cols a multiple of 256 and <= 4096, 1 <= T <= 8");
-    if (T >= g_dense_mfma_t)                           /* several tokens: quants on MFMA */
+    if (dense_mm8_takes((const uint8_t *)W, q6, cols, T))   /* several tokens: quants on MFMA */
         return dense_mm8_launch((const uint8_t *)W, q6, X, Y, rows, cols, T);
     const int nb = (int)(cols / RQK), rpw = 64 / lanes_per_row(nb);
     const size_t npass = (rows + rpw - 1) / rpw;
@@ -762,8 +768,13 @@ extern "C" int roaster_matvec_q(const void *W, int q6, const float *X, float *Y,
     const dim3 gd((unsigned)blocks), bd(MV_THREADS);
     const uint8_t *w = (const uint8_t *)W;
     const int r = (int)rows, cc = (int)cols;
-#define DMV(Q6_, ONE_, KB_) hipLaunchKernelGGL((dense_mv_kernel<Q6_, ONE_, KB_>), gd, bd, ONE_ ? 0 : lds, rt().stream, w, X, Y, r, cc, T)
-    if (nb <= 8) {
+#define DMV(...) hipLaunchKernelGGL((dense_mv_kernel<__VA_ARGS__>), gd, bd, lds, rt().stream, w, X, Y, r, cc, T)
+    if (mat_odd(w, q6)) {                              /* Q6_K blocks at odd addresses: loaded as they lie */
+        if (nb <= 8 && T == 1) DMV(true, true, 1, false);
+        else if (nb <= 8) DMV(true, false, 1, false);
+        else if (T == 1) DMV(true, true, 2, false);
+        else DMV(true, false, 2, false);
+    } else if (nb <= 8) {
         if (q6 && T == 1) DMV(true, true, 1);
         else if (q6) DMV(true, false, 1);
         else if (T == 1) DMV(false, true, 1);

@@ -8,10 +8,13 @@ operand).  One token runs the pipelined matvec on the same shapes.
 
 Bar 5e-6 of max|y|: 22-bit activations (2^-22 per product, random in sign) and
 f32 sums of up to 3584 terms on both sides, about 1e-6 each."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import roaster_amd as R
+from gpu_util import Dev, alloc_w
 from oracle import oracle as O
 from test_gpu_dense import run, weights
 
@@ -49,3 +52,36 @@ def test_staged(q6, rows, cols):
         for t in (t for t in ref if t < T):
             err = np.max(np.abs(Y[t] - ref[t])) / np.max(np.abs(ref[t]))
             assert err <= 5e-6, (T, t, err)
+
+
+@pytest.mark.parametrize("off", [1, 2, 3])
+@pytest.mark.parametrize("q6", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(37, 512), (37, 2304), (16400, 256)])
+def test_unaligned_matrix(q6, rows, cols, off):
+    """A matrix that begins at any byte gives what it gives at an aligned address
+    (the Q6_K kernels that read aligned dwords take even ones only)."""
+    W = weights(q6, rows, cols, 95 + cols)
+    X = np.stack([R.synth_normal(96, R.synth_stream(t, cols, 5), cols) for t in range(8)])
+    moved = Dev(np.concatenate([np.zeros(off, np.uint8), W]))
+    for T in (1, 2, 5, 8):
+        Y = run(q6, W, X[:T], rows, cols)
+        dx, dy = Dev(X[:T]), Dev(nbytes=T * rows * 4, shape=(T, rows))
+        R.check(R.lib().roaster_matvec_q(moved.p + off, q6, dx.p, dy.p, rows, cols, T), "matvec_q")
+        R.check(R.lib().roaster_sync(), "sync")
+        err = np.max(np.abs(dy.get() - Y)) / np.max(np.abs(Y))
+        assert err <= 5e-6, (T, err)
+
+
+@pytest.mark.parametrize("q6", [0, 1])
+def test_unaligned_matrix_batch(q6):
+    """The same through kernel_matmul_quant_batch, from weight memory at an odd address."""
+    rows, cols, T = 100, 512, 5
+    W = weights(q6, rows, cols, 97)
+    X = np.stack([R.synth_normal(98, R.synth_stream(t, cols, 5), cols) for t in range(T)])
+    p = alloc_w(np.concatenate([np.zeros(1, np.uint8), W]))
+    Y = np.empty((T, rows), np.float32)
+    job = R.KernelMatmulJob(q6, p + 1, X.ctypes.data, Y.ctypes.data, rows, cols, T)
+    assert R.lib().kernel_matmul_quant_batch(C.byref(job), 1) == 0
+    for t in range(T):
+        ref = O.matvec(q6, W, X[t], rows, cols)
+        assert np.max(np.abs(Y[t] - ref)) <= 5e-6 * np.max(np.abs(ref))
