@@ -233,7 +233,9 @@ __global__ void __launch_bounds__(MV_THREADS) dense_mv_kernel(const uint8_t *W, 
  *       lane;
  *   d, the scale's inverse and (Q4_K) dmin times the sub-block minima's
  *       product with the sub-block sums (one more MFMA: minima 2 g, 2 g + 1 in
- *       lane group g) are applied in f32 once per super-block
+ *       lane group g) are applied in f32 once per super-block; the sums are f32
+ *       in three fp16 parts, the third, with 5..8 tokens, beside the second in
+ *       its row (the minima stand there again)
  * (the reference's fold, kernels.c:1844-1874: d sc sum(q x) - dmin m sum(x),
  * d sc sum((q - 32) x)).  Every workgroup prepares A in LDS itself while its
  * first weights are on the way; each wave streams 16-row groups, the next
@@ -242,10 +244,16 @@ __global__ void __launch_bounds__(MV_THREADS) dense_mv_kernel(const uint8_t *W, 
 #define MM8_W (MM8_T / 64)
 
 /* LDS of one call: A fragments [cols / 256][8][64 lanes] (16 bytes), sub-block
- * sums [cols / 256][64 lanes] (2 fp16), scales [cols / 256][8 tokens] (2^-e). */
+ * sums [cols / 256][64 lanes] (MM8_SUM fp16), scales [cols / 256][8 tokens] (2^-e). */
+#define MM8_SUM(Q6, PARTS) (!(Q6) && (PARTS) == 2 ? 4 : 2)
 __host__ __device__ static inline size_t mm8_frag_bytes(size_t cols) { return cols * 32; }
-__host__ __device__ static inline size_t mm8_sum_bytes(size_t cols) { return cols; }
-__host__ __device__ static inline size_t mm8_lds_bytes(size_t cols) { return mm8_frag_bytes(cols) + mm8_sum_bytes(cols) + cols / RQK * 8 * 4; }
+template <bool Q6, int PARTS>
+__host__ __device__ static inline size_t mm8_sum_bytes(size_t cols) { return cols / 2 * MM8_SUM(Q6, PARTS); }
+template <bool Q6, int PARTS>
+__host__ __device__ static inline size_t mm8_lds_bytes(size_t cols)
+{
+    return mm8_frag_bytes(cols) + mm8_sum_bytes<Q6, PARTS>(cols) + cols / RQK * 8 * 4;
+}
 
 /* Super-block kb of the activations into LDS (one wave): lane (t = l / 8, c =
  * l % 8) takes columns 32 c .. + 31 of token t. */
@@ -258,8 +266,8 @@ __device__ __forceinline__ void mm8_prep(const float *X, int cols, int T, int kb
      * 64 (g / 2) + 32 ((f / 2) % 2) + 16 (g % 2) + 8 (f % 2) .. + 7 */
     f16x8 *frag = (f16x8 *)lds + (size_t)kb * 512 +
                   (Q6 ? 128 * (c >> 1) + 32 * (c & 1) : 256 * (c >> 2) + 128 * (c & 1) + 32 * ((c >> 1) & 1));
-    f16x2 *sums = (f16x2 *)(lds + mm8_frag_bytes(cols)) + kb * 64;
-    float *ge = (float *)(lds + mm8_frag_bytes(cols) + mm8_sum_bytes(cols)) + kb * 8;
+    _Float16 *sums = (_Float16 *)(lds + mm8_frag_bytes(cols)) + kb * 64 * MM8_SUM(Q6, PARTS);
+    float *ge = (float *)(lds + mm8_frag_bytes(cols) + mm8_sum_bytes<Q6, PARTS>(cols)) + kb * 8;
     if (t >= T) return;
     const float *xp = X + (size_t)t * cols + RQK * kb + 32 * c;
     float4 v[8];
@@ -294,13 +302,16 @@ __device__ __forceinline__ void mm8_prep(const float *X, int cols, int T, int kb
             w = w - __builtin_convertvector(h, f32x8);
         }
     }
-    /* sub-block c's sum, in lane group c / 2's slot c % 2 */
+    /* sub-block c's sum, in lane group c / 2's slot c % 2; two rows a token: the
+     * third part in the second row's slot 2 + c % 2 */
     sum *= 0.015625f;
 #pragma unroll
     for (int p = 0; p < PARTS; p++) {
         const _Float16 h = (_Float16)sum;
-        ((_Float16 *)(sums + 16 * (c >> 1) + row + p))[c & 1] = h;
+        _Float16 *o = sums + (16 * (c >> 1) + row + p) * MM8_SUM(Q6, PARTS) + (c & 1);
+        *o = h;
         sum -= (float)h;
+        if (MM8_SUM(Q6, PARTS) == 4) o[2] = p == 0 ? (_Float16)0.0f : (_Float16)sum;
     }
 }
 
@@ -346,6 +357,7 @@ __device__ __forceinline__ uint32_t q4_pair6(uint32_t own, uint32_t s811, int ni
 }
 
 /* z: the integer products of one super-block; zm: the minima's (Q4_K). */
+template <int PARTS>
 __device__ __forceinline__ void mm8_block(const Mm8Q4 &r, const uint8_t *frag, const uint8_t *sums, int lane, f32x4 (&z)[2],
                                           f32x4 &zm)
 {
@@ -355,9 +367,16 @@ __device__ __forceinline__ void mm8_block(const Mm8Q4 &r, const uint8_t *frag, c
         /* minima 2 g, 2 g + 1 of lane group g against the sums of those sub-blocks */
         const uint32_t m = q4_pair6(s47, s811, 4, 16 * (g & 1), g < 2);
         const _Float16 o = (_Float16)0.0f;
-        const f16x8 mb = { (_Float16)(int)(m & 0xFF), (_Float16)(int)(m >> 8), o, o, o, o, o, o };
-        const f16x2 xs = *(const f16x2 *)(sums + 4 * lane);
-        const f16x8 xa = { xs[0], xs[1], o, o, o, o, o, o };
+        const _Float16 m0 = (_Float16)(int)(m & 0xFF), m1 = (_Float16)(int)(m >> 8);
+        f16x8 mb = { m0, m1, o, o, o, o, o, o }, xa = { o, o, o, o, o, o, o, o };
+        if constexpr (PARTS == 2) {
+            const f16x4 xs = *(const f16x4 *)(sums + 8 * lane);
+            mb[2] = m0, mb[3] = m1;
+            xa[0] = xs[0], xa[1] = xs[1], xa[2] = xs[2], xa[3] = xs[3];
+        } else {
+            const f16x2 xs = *(const f16x2 *)(sums + 4 * lane);
+            xa[0] = xs[0], xa[1] = xs[1];
+        }
         zm = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa, mb, (f32x4){}, 0, 0, 0);
     }
     z[0] = z[1] = (f32x4){};
@@ -384,6 +403,7 @@ __device__ __forceinline__ void mm8_block(const Mm8Q4 &r, const uint8_t *frag, c
     }
 }
 
+template <int PARTS>
 __device__ __forceinline__ void mm8_block(const Mm8Q6 &r, const uint8_t *frag, const uint8_t *, int lane, f32x4 (&z)[2], f32x4 &)
 {
     const int g = lane >> 4, qs = 2 * (g >> 1);             /* qh bits of the low nibbles' columns */
@@ -431,8 +451,8 @@ __device__ __forceinline__ void mm8_add(const Raw &raw, const uint8_t *lds, int 
                                         float (&y)[2])
 {
     f32x4 z[2], zm;
-    mm8_block(raw, lds + (size_t)kb * 8192, lds + mm8_frag_bytes(cols) + kb * 256, lane, z, zm);
-    const float *ge = (const float *)(lds + mm8_frag_bytes(cols) + mm8_sum_bytes(cols)) + kb * 8;
+    mm8_block<PARTS>(raw, lds + (size_t)kb * 8192, lds + mm8_frag_bytes(cols) + kb * 128 * MM8_SUM(Q6, PARTS), lane, z, zm);
+    const float *ge = (const float *)(lds + mm8_frag_bytes(cols) + mm8_sum_bytes<Q6, PARTS>(cols)) + kb * 8;
     const int g = lane >> 4;
     float d, dm;
     if constexpr (Q6) {
@@ -560,7 +580,7 @@ __global__ void __launch_bounds__(MM8S_T, 1) dense_mm8s_kernel(const uint8_t *W,
     const int nb = cols / RQK;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g4 = lane >> 4;
     const int ngroups = (rows + 15) >> 4, nw = gridDim.x * MM8S_W;
-    uint8_t *slice = mm8_lds + mm8_lds_bytes(cols) + wv * 16 * Raw::N;
+    uint8_t *slice = mm8_lds + mm8_lds_bytes<Q6, PARTS>(cols) + wv * 16 * Raw::N;
     /* load i of this lane: chunk ck of the group's row cr (past the last chunk
      * that one again, to the same place) */
     int cr[Raw::NL], ck[Raw::NL];
@@ -657,7 +677,7 @@ bool dense_mm8_takes(const uint8_t *W, int q6, size_t cols, size_t T)
 
 int dense_mm8_launch(const uint8_t *W, int q6, const float *X, float *Y, size_t rows, size_t cols, int T)
 {
-    const size_t lds = mm8_lds_bytes(cols);
+    const size_t lds = q6 ? mm8_lds_bytes<true, 3>(cols) : T <= 4 ? mm8_lds_bytes<false, 3>(cols) : mm8_lds_bytes<false, 2>(cols);
     const size_t ng = (rows + 15) / 16;
     const size_t slds = lds + MM8S_W * 256 * (q6 ? Mm8S<true>::CH : Mm8S<false>::CH);
     const dim3 gs((unsigned)rt().n_cu), bs(MM8S_T);

@@ -85,3 +85,23 @@ def test_unaligned_matrix_batch(q6):
     for t in range(T):
         ref = O.matvec(q6, W, X[t], rows, cols)
         assert np.max(np.abs(Y[t] - ref)) <= 5e-6 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("T", [4, 5, 8])
+def test_minima_keep_f32_sums(T):
+    """Q4_K's minimum term takes the sub-block sums with all 24 bits of an f32: scales
+    of zero and one minimum of one per super-block leave y = -dmin x for an x with a
+    single 24-bit entry in each super-block's sub-block, here exactly."""
+    rows, cols = 64, 512
+    W = np.zeros((rows, cols // 256, R.Q4K_BYTES), np.uint8)
+    W[:, 0, 2:4] = np.frombuffer(np.float16(1.0).tobytes(), np.uint8)     # dmin of the first super-block
+    sub = np.arange(rows) % 8
+    for r, s in enumerate(sub):
+        W[r, 0, 8 + s] = 1 if s < 4 else 1 << 4                           # minimum 1 in sub-block s
+    rng = np.random.default_rng(6)
+    X = np.zeros((T, cols), np.float32)
+    big = rng.integers(2 ** 23, 2 ** 24, (T, 8)) | 1
+    for t in range(T):
+        X[t, 32 * np.arange(8) + t] = big[t]
+    Y = run(0, W.reshape(-1), X, rows, cols)
+    np.testing.assert_array_equal(Y, -big[:, sub].astype(np.float32))
