@@ -242,6 +242,7 @@ __global__ void __launch_bounds__(MV_THREADS) dense_mv_kernel(const uint8_t *W, 
  * super-block's quants in flight while one computes. */
 #define MM8_T 512
 #define MM8_W (MM8_T / 64)
+#define MM8_RED (2 * MM8_W * 64 * 8)      /* static LDS of dense_mm8_kernel */
 
 /* LDS of one call: A fragments [cols / 256][8][64 lanes] (16 bytes), sub-block
  * sums [cols / 256][64 lanes] (MM8_SUM fp16), scales [cols / 256][8 tokens] (2^-e). */
@@ -505,6 +506,7 @@ __global__ void __launch_bounds__(MM8_T, 4) dense_mm8_kernel(const uint8_t *W, c
     const int team = blockIdx.x * tpw + wv / split, nteam = gridDim.x * tpw;
     const int iters = (ngroups + nteam - 1) / nteam, per = (nb + split - 1) / split, total = iters * per;
     __shared__ float2 red[2][MM8_W][64];
+    static_assert(sizeof(red) == MM8_RED, "the launch counts it");
     /* item i: super-block member + (i % per) split of group team + (i / per)
      * nteam; past either end the last one again, so that every wave runs the
      * same items and barriers */
@@ -698,7 +700,8 @@ int dense_mm8_launch(const uint8_t *W, int q6, const float *X, float *Y, size_t 
 #undef MM8S
         return rt_check(hipGetLastError(), "dense MFMA launch") ? ROASTER_EDEVICE : 0;
     }
-    const size_t cap = (size_t)(lds <= 78 * 1024 ? 2 : 1) * rt().n_cu;
+    /* workgroups resident at once, by LDS (up to 2048 columns two per CU) */
+    const size_t cap = (size_t)(2 * (lds + MM8_RED) <= 160 * 1024 ? 2 : 1) * rt().n_cu;
     const int nb = (int)(cols / RQK);
     /* waves per group: the split whose waves run the fewest super-blocks one
      * after the other (a few groups need several waves each to fill the CUs) */
