@@ -632,9 +632,18 @@ __global__ void __launch_bounds__(MM8S_T, 1) dense_mm8s_kernel(const uint8_t *W,
     if (g0 >= ngroups) return;
     float y[2] = { 0.0f, 0.0f };
     int g = g0, kb = 0;                                 /* the super-block to compute */
+    /* the slice's stores and loads of one step and the next stay in order, for
+     * all lanes (LDS serves a wave's accesses in order: no instructions) */
+    auto wave_fence = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
     auto step = [&](Raw &r) {                           /* whether it was the last */
+        wave_fence();
 #pragma unroll
         for (int i = 0; i < Raw::NL; i++) *(uint4 *)(slice + 16 * min(64 * i + lane, Raw::N - 1)) = r.c[i];
+        wave_fence();
         const uint32_t tail = r.t, sh = r.sh;
         load(r);
         const uint8_t *row = slice + (lane & 15) * (16 * Raw::CH);
