@@ -56,6 +56,8 @@
 #include <stdio.h>
 #include <string.h>
 #include <type_traits>
+#include <utility>
+#include <vector>
 
 #define DT 256                        /* threads per workgroup */
 #define DW (DT / 64)                  /* waves per workgroup */
@@ -2972,35 +2974,22 @@ extern "C" int roaster_decode_cooperative_launch(int enable)
     return g_coop;
 }
 
-/* Whether every one-launch stack kernel fits one workgroup per CU on at least
- * K1_NWG CUs (registers and LDS as compiled), checked once per process: else
- * their grids could never be resident at once and the three-kernel path runs. */
-static int g_k1_fits = -1;
-
-static bool k1_fits()
+/* Whether a one-launch stack kernel fits one workgroup per CU on at least
+ * K1_NWG CUs (registers and LDS as compiled), asked once per kernel and process:
+ * else its grid could never be resident at once and another kernel, or the
+ * three-kernel path, runs in its place. */
+static bool k1_fits(const void *fn)
 {
-    if (g_k1_fits >= 0) return g_k1_fits == 1;
-    const void *fns[] = {(const void *)dec_stack1_kernel, (const void *)dec_stack1_2x2_kernel,
-                         (const void *)dec_stack1r_kernel<0, 1>, (const void *)dec_stack1r_kernel<0, -1>,
-                         (const void *)dec_stack1r_kernel<1, -1>, (const void *)dec_stackB2_kernel,
-                         (const void *)dec_stackB4_kernel, (const void *)dec_stackB8_kernel,
-                         (const void *)dec_stackB2_q4_kernel, (const void *)dec_stackB4_q4_kernel,
-                         (const void *)dec_stackB8_q4_kernel, (const void *)dec_stackB2_q6_kernel,
-                         (const void *)dec_stackB4_q6_kernel, (const void *)dec_stackB8_q6_kernel,
-                         (const void *)dec_stackB2_i256_q4_kernel, (const void *)dec_stackB4_i256_q4_kernel,
-                         (const void *)dec_stackB8_i256_q4_kernel, (const void *)dec_stackB2_i256_q6_kernel,
-                         (const void *)dec_stackB4_i256_q6_kernel, (const void *)dec_stackB8_i256_q6_kernel};
-    bool ok = rt().n_cu >= K1_NWG;
-    for (const void *f : fns) {
-        int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, K1_T, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            nb = 0;
-        }
-        ok = ok && nb >= 1;
+    static std::vector<std::pair<const void *, bool>> asked;    /* under the library's lock */
+    for (const auto &a : asked)
+        if (a.first == fn) return a.second;
+    int nb = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, K1_T, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        nb = 0;
     }
-    g_k1_fits = ok ? 1 : 0;
-    return ok;
+    asked.emplace_back(fn, rt().n_cu >= K1_NWG && nb >= 1);
+    return asked.back().second;
 }
 
 /* A one-launch stack kernel on the library stream.  Its 256 workgroups wait
@@ -3045,16 +3034,16 @@ size_t dec_xch_need1(int E, int H, int I)
 
 bool dec_layer1_ok(int E, int H, int I, int B)
 {
-    return g_layer1 && B == 1 && k1_fits() && E >= RTOPK && E <= 256 && E % K1_GW == 0 && H % RQK == 0 &&
-           H <= K1_MAXH && I % RQK == 0 && I <= K1_MAXI;
+    return g_layer1 && B == 1 && k1_fits((const void *)dec_stack1_kernel) && E >= RTOPK && E <= 256 &&
+           E % K1_GW == 0 && H % RQK == 0 && H <= K1_MAXH && I % RQK == 0 && I <= K1_MAXI;
 }
 
 /* The batched kernels' shapes: inter 512 (two gate/up rows and two down
- * tasks per wave) or 256 (one and one), hidden 512..2048 in whole 256-row blocks, at most 256
- * experts (one logit per lane of a wave's 64 for 8 tokens). */
+ * tasks per wave) or 256 (one and one), hidden 512..2048 in whole 256-row
+ * blocks, at most 256 experts (one logit per lane of a wave's 64 for 8 tokens). */
 bool dec_layerB_ok(int E, int H, int I, int B)
 {
-    return g_layer1 && B >= 2 && B <= K1B_MAXB && k1_fits() && E >= RTOPK && E <= 256 && E % K1_GW == 0 &&
+    return g_layer1 && B >= 2 && B <= K1B_MAXB && E >= RTOPK && E <= 256 && E % K1_GW == 0 &&
            (I == 512 || I == 256) && H % 256 == 0 && H >= 512 && H <= K1_MAXH;
 }
 
@@ -3156,11 +3145,14 @@ static StackKernel stack1_choice(const DecArgs &A, int c0, int cn, size_t xn)
     const int nbi = A.I / RQK, rpw = 64 / lanes_per_row(nbi);
     const int npg = (A.I / K1_GW + K1_W - 1) / K1_W, nd = ((A.H / K1_GW + rpw - 1) / rpw + K1_W - 1) / K1_W;
     const int ty = stack_types(A, c0, cn);
-    if (ty >= 0 && A.cnt && dec_r1_shape(A.E, A.H, A.I) && xn >= (size_t)XR_U64(A.E, A.H, A.I))
-        return ty == 0 ? StackKernel{ (const void *)dec_stack1r_kernel<0, 1>, "dec_stack1r_kernel" }
-             : ty == 1 ? StackKernel{ (const void *)dec_stack1r_kernel<0, -1>, "dec_stack1r_q4_kernel" }
-                       : StackKernel{ (const void *)dec_stack1r_kernel<1, -1>, "dec_stack1r_q6_kernel" };
-    return npg == 2 && nd == 2 && ty == 0 ? STACK_KERNEL(dec_stack1_2x2_kernel) : STACK_KERNEL(dec_stack1_kernel);
+    if (ty >= 0 && A.cnt && dec_r1_shape(A.E, A.H, A.I) && xn >= (size_t)XR_U64(A.E, A.H, A.I)) {
+        const StackKernel k = ty == 0 ? StackKernel{ (const void *)dec_stack1r_kernel<0, 1>, "dec_stack1r_kernel" }
+                            : ty == 1 ? StackKernel{ (const void *)dec_stack1r_kernel<0, -1>, "dec_stack1r_q4_kernel" }
+                                      : StackKernel{ (const void *)dec_stack1r_kernel<1, -1>, "dec_stack1r_q6_kernel" };
+        if (k1_fits(k.fn)) return k;
+    }
+    const bool two = npg == 2 && nd == 2 && ty == 0 && k1_fits((const void *)dec_stack1_2x2_kernel);
+    return two ? STACK_KERNEL(dec_stack1_2x2_kernel) : STACK_KERNEL(dec_stack1_kernel);
 }
 
 /* The kernel of B = 2..8 tokens (the smallest of 2, 4, 8 slots that holds B)
@@ -3170,9 +3162,9 @@ static StackKernel stack1_choice(const DecArgs &A, int c0, int cn, size_t xn)
  * the 8-slot kernel 2.7 over the fixed one); one all-Q6_K layer of 4 tokens
  * 46.4 -> 35.9.  Inter 256: 2 tokens 26.9 -> 15.3, 4 35.7 -> 21.6, 8 61.0 ->
  * 34.4; one layer of 5 tokens 41.5 -> 27.7. */
-static StackKernel stackB_choice(const DecArgs &A, int l0, int n)
+static StackKernel stackB_for(const DecArgs &A, int ty)
 {
-    const int B = A.B, ty = stack_types(A, l0, n);
+    const int B = A.B;
     if (A.I == 256) {                     /* either down type at run time */
         if (ty < 0) return StackKernel{ NULL, NULL };
         if (ty == 2)
@@ -3192,6 +3184,12 @@ static StackKernel stackB_choice(const DecArgs &A, int l0, int n)
                       : B <= 4 ? STACK_KERNEL(dec_stackB4_q6_kernel) : STACK_KERNEL(dec_stackB8_q6_kernel);
     }
     return StackKernel{ NULL, NULL };
+}
+
+static StackKernel stackB_choice(const DecArgs &A, int l0, int n)
+{
+    const StackKernel k = stackB_for(A, stack_types(A, l0, n));
+    return k.fn && k1_fits(k.fn) ? k : StackKernel{ NULL, NULL };
 }
 
 /* One launch per run of up to K1_MAXL layers (dec_stack1_kernel) on the
