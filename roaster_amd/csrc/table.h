@@ -13,7 +13,8 @@ struct TileLayer {
     const uint8_t *sgate, *sup, *sdown;
     /* the router as the prefill router's MFMA operand: [E / 32, rounded up][H /
      * 32][4][64 lanes][4]: load q of K chunk c gives lane n + 32 h columns 32 c
-     * + 8 q + 4 h .. + 3 of expert 32 b + n (zero past E).  A load of a wave is a
+     * + 8 q + 4 h .. + 3 of expert 32 b + n (zero past E); NULL past 256 experts,
+     * which prefill refuses.  A load of a wave is a
      * contiguous kilobyte; the row-major router's 32 rows, H floats apart,
      * measured 9.6 us in place of 8.5 at 45 tokens and 35.6 in place of 30.7
      * at 2048 (E 256, H 2048). */

@@ -24,6 +24,9 @@
 
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
+/* Experts of a router's operand copy: whole blocks of 32, none past the 256 that prefill takes. */
+static size_t router_tile_experts(int E) { return E <= 256 ? (size_t)(E + 31) / 32 * 32 : 0; }
+
 /* types: [n_layers][6] = routed gate, up, down, shared gate, up, down (0 = Q4_K,
  * 1 = Q6_K), or NULL for the description's types in every layer. */
 extern "C" RoasterTable *roaster_table_create_layers(const RoasterTableDesc *d, const int *types)
@@ -70,7 +73,7 @@ extern "C" RoasterTable *roaster_table_create_layers(const RoasterTableDesc *d, 
     }
     t->qbytes = qoff;
     t->tbytes = toff;
-    const size_t EB = (E + 31) / 32 * 32;         /* experts of the router's operand copy */
+    const size_t EB = router_tile_experts((int)E);
     t->fbytes = (size_t)d->n_layers * (E * H + H + EB * H) * sizeof(float);
     if (hipMalloc((void **)&t->qmem, t->qbytes + RT_TAIL_PAD) != hipSuccess ||
         hipMalloc((void **)&t->tmem, t->tbytes + RT_TAIL_PAD) != hipSuccess ||
@@ -117,7 +120,7 @@ extern "C" RoasterTable *roaster_table_create_layers(const RoasterTableDesc *d, 
         TL.sgate = tbase + G.toff_sh[0];
         TL.sup = tbase + G.toff_sh[1];
         TL.sdown = tbase + G.toff_sh[2];
-        TL.router = t->fmem + (size_t)d->n_layers * (E * H + H) + (size_t)l * EB * H;
+        TL.router = EB ? t->fmem + (size_t)d->n_layers * (E * H + H) + (size_t)l * EB * H : NULL;
     }
     if (rt_check(hipMemcpy(t->layers_d, t->layers_h.data(), sizeof(DecLayer) * d->n_layers, hipMemcpyHostToDevice),
                  "layer table upload")) {
@@ -270,6 +273,7 @@ __global__ void router_tile_kernel(const float *src, float4 *dst, int E, int H)
 static int router_tile(const RoasterTable *t, int layer)
 {
     const int E = t->d.n_experts, H = (int)t->d.hidden;
+    if (!t->tlayers_h[layer].router) return 0;
     const size_t n = (size_t)(E + 31) / 32 * 32 * H / 4;
     hipLaunchKernelGGL(router_tile_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, rt().stream,
                        t->layers_h[layer].router, (float4 *)t->tlayers_h[layer].router, E, H);

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import roaster_amd as R
-from gpu_util import SynthTable, prefill
+from gpu_util import Dev, SynthTable, prefill
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +46,21 @@ def test_router_replaced(table):
     check(table, router, 40)
     R.check(R.lib().roaster_table_set_router(table.t, 0, old.ctypes.data, gate_inp.ctypes.data), "set_router")
     check(table, old, 40)
+
+
+@pytest.mark.parametrize("E", [256, 257])
+def test_operand_copy_only_where_prefill_reads_it(E):
+    """A table of more than 256 experts, which prefill refuses, carries no operand
+    copy of the router; setting its router works, prefill refuses as before."""
+    t = SynthTable(4, n_experts=E, hidden=256, inter=256, q6=(0, 0, 1), sh_q6=(0, 0, 1))
+    try:
+        mats = 256 * (2 * R.Q4K_BYTES + R.Q6K_BYTES) + 8 * 1024 * (2 * 5 + 7)      # GGML and 32-row tile layouts
+        copies = 2 if E <= 256 else 1
+        assert R.lib().roaster_table_bytes(t.t) == (E + 1) * mats + 4 * 256 * (E * copies + 1)
+        router, gate_inp = (np.ascontiguousarray(a) for a in t.router(0))
+        R.check(R.lib().roaster_table_set_router(t.t, 0, router.ctypes.data, gate_inp.ctypes.data), "set_router")
+        x, y = Dev(np.zeros((1, 256), np.float32)), Dev(nbytes=1024)
+        assert R.lib().roaster_moe_prefill(t.t, 0, x.p, 1, y.p, None) == (0 if E <= 256 else R.EINVAL)
+        R.check(R.lib().roaster_sync(), "sync")
+    finally:
+        t.destroy()
