@@ -215,11 +215,13 @@ struct NwMeta {
     float fwd[NW_ROWS];
 };
 
-template <int NWV, bool Q6, bool SPLIT>
+#define NWG_W 4                   /* waves per gate/up workgroup */
+
+template <bool Q6, bool SPLIT>
 __device__ __forceinline__ void nw_gu_body(const PfGemmArgs &A, const PfGroup &G, NwMeta &meta, int m0, int mlen, int j0,
                                            _Float16 *Xb)
 {
-    constexpr int NT = 64 * NWV, RPP = NT / 32, NP = NW_ROWS / RPP;      /* operand rows per staging round, rounds */
+    constexpr int NT = 64 * NWG_W, RPP = NT / 32, NP = NW_ROWS / RPP;      /* operand rows per staging round, rounds */
     constexpr int ROWS = NwTile<SPLIT>::ROWS, NA = NwTile<SPLIT>::ACC, TB = TL_BYTES(Q6);
     const int t = threadIdx.x, l = t & 63, h = l >> 5, w = t >> 6, n = l & 31;
     const int nkb = A.H / GK;
@@ -334,19 +336,19 @@ __device__ __forceinline__ void nw_gu_body(const PfGemmArgs &A, const PfGroup &G
     }
 }
 
-template <int NWV, bool SPLIT>
-__global__ void __launch_bounds__(64 * NWV, 3) pfn_gu_kernel(PfGemmArgs A)
+template <bool SPLIT>
+__global__ void __launch_bounds__(64 * NWG_W, 3) pfn_gu_kernel(PfGemmArgs A)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t nw_lds[];
     __shared__ NwMeta meta;
-    const int nblk = A.I / (16 * NWV), R = *A.gu_ntiles * nblk;
+    const int nblk = A.I / (16 * NWG_W), R = *A.gu_ntiles * nblk;
     if ((int)blockIdx.x >= R) return;
     const int v = pf_virtual_block(blockIdx.x, R);
     const PfTile tile = A.gu_tiles[v / nblk];
     const PfGroup &G = A.groups[tile.grp];
-    const int mlen = min(NwTile<SPLIT>::ROWS, G.n - tile.m0), j0 = (v % nblk) * 16 * NWV;
-    if (G.gq6) nw_gu_body<NWV, true, SPLIT>(A, G, meta, tile.m0, mlen, j0, (_Float16 *)nw_lds);
-    else nw_gu_body<NWV, false, SPLIT>(A, G, meta, tile.m0, mlen, j0, (_Float16 *)nw_lds);
+    const int mlen = min(NwTile<SPLIT>::ROWS, G.n - tile.m0), j0 = (v % nblk) * 16 * NWG_W;
+    if (G.gq6) nw_gu_body<true, SPLIT>(A, G, meta, tile.m0, mlen, j0, (_Float16 *)nw_lds);
+    else nw_gu_body<false, SPLIT>(A, G, meta, tile.m0, mlen, j0, (_Float16 *)nw_lds);
 }
 
 /* ---- down (inter <= 512) -----------------------------------------------------
@@ -554,20 +556,24 @@ bool pf_narrow_f16_down(int T, int E, int q6) { return !q6 || 8 * (long long)T <
 
 int pf_narrow_gu_launch(const PfGemmArgs &A, int max_tiles, bool split)
 {
-    const int wv = 4;
-    const dim3 g((unsigned)(max_tiles * (A.I / (16 * wv)))), b(64 * wv);
+    const dim3 g((unsigned)(max_tiles * (A.I / (16 * NWG_W)))), b(64 * NWG_W);
     const size_t lds = 2 * (size_t)NW_BUF * 2;
-    if (split) hipLaunchKernelGGL((pfn_gu_kernel<4, true>), g, b, lds, rt().stream, A);
-    else hipLaunchKernelGGL((pfn_gu_kernel<4, false>), g, b, lds, rt().stream, A);
+    if (split) hipLaunchKernelGGL(pfn_gu_kernel<true>, g, b, lds, rt().stream, A);
+    else hipLaunchKernelGGL(pfn_gu_kernel<false>, g, b, lds, rt().stream, A);
     return rt_check(hipGetLastError(), "prefill gate/up launch") ? ROASTER_EDEVICE : 0;
 }
 
 /* Where the line lies: fp16 mode's wide tiles (pf_gemm.hip) dequantise a weight
  * once per 96 rows, these once per 32, but run at three waves per SIMD and
  * balance in units of 64 columns.  Measured per layer (256 experts, hidden
- * 2048, inter 512, Q6_K down; wide -> narrow, us): Q4_K gate/up 512 tokens 206
- * -> 174, 768 226 -> 190, 1024 236 -> 214, 2048 302 -> 316; Q6_K gate/up 512
- * 211 -> 200, 768 233 -> 217, 1024 239 -> 240, 2048 301 -> 347. */
+ * 2048, inter 512, Q6_K down; wide -> narrow, us): Q4_K gate/up 512 tokens 205
+ * -> 173, 768 224 -> 190, 1152 (the line) 257 -> 241, 1792 288 -> 297; Q6_K gate/up
+ * 512 210 -> 196, 896 (the line) 236 -> 225, 1152 262 -> 268, 1792 283 -> 319.  At
+ * the line of other shapes, Q4_K / Q6_K: hidden 1024 167 -> 151 / 149 -> 137, inter
+ * 256 187 -> 167 / 163 -> 148, inter 768 412 -> 402 / 382 -> 381, inter 1024 505 ->
+ * 502 / 470 -> 470, 64 experts 107 -> 81 / 99 -> 77, 8 experts 77 -> 45 / 69 -> 46.
+ * Where a few experts take every token the narrow tiles run out first: 8 of 256,
+ * 768 tokens 136 -> 122 / 135 -> 126, but 1152 166 -> 173, Q6_K 896 136 -> 141. */
 bool pf_narrow_f16(int T, int E, int q6) { return 8 * (long long)T <= (long long)E * (q6 ? 28 : 36); }
 
 int pf_narrow_down_launch(const PfGemmArgs &A, int max_tiles, bool split)

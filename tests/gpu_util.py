@@ -107,6 +107,32 @@ class SynthTable:
             self.t = None
 
 
+def wide_q6k_scales(mat, rng):
+    """Q6_K bytes with scales over all of int8, d reduced to keep the weights' size."""
+    b = mat.reshape(-1, R.Q6K_BYTES).copy()
+    b[:, 192:208] = rng.integers(0, 256, (len(b), 16), dtype=np.uint8)
+    d = b[:, 208:210].copy().view(np.float16)
+    b[:, 208:210] = (d / np.float16(4)).view(np.uint8)
+    return b.reshape(-1)
+
+
+WIDE_SCALE_TABLES = [(256, 256, 0, 1), (768, 512, 1, 0), (2048, 512, 0, 1), (2048, 512, 1, 0)]
+
+
+def wide_scale_table(H, I, gu, dn):
+    """Eight experts (every token takes all), Q6_K scales over all of int8, routed
+    and shared types opposite."""
+    q6, sq6 = (gu, gu, dn), (1 - gu, 1 - gu, 1 - dn)
+    t = SynthTable(11, n_experts=8, hidden=H, inter=I, q6=q6, sh_q6=sq6)
+    rng = np.random.default_rng(5)
+    for e in range(9):
+        types = sq6 if e == 8 else q6
+        m = [wide_q6k_scales(w, rng) if q else w for w, q in zip(t.expert(0, e), types)]
+        t._experts[(0, e)] = tuple(m)
+        R.check(R.lib().roaster_table_set_expert(t.t, 0, e, *(w.ctypes.data for w in m)), "set_expert")
+    return t
+
+
 def bf16_round(a):
     """Round f32 values to the nearest bf16 (ties to even), kept as f32."""
     u = np.ascontiguousarray(a, np.float32).view(np.uint32).astype(np.uint64)
