@@ -164,7 +164,7 @@ int roaster_moe_decode_stack(RoasterTable *t, float *h, int B, int layer0, int n
 
 /* Decode runs a call's layers as one launch (router, top-8, experts and
  * combine in 256 workgroups that exchange values through memory) wherever the
- * shapes allow it: a device with at least 256 CUs on which each one-launch
+ * shapes allow it: a device with at least 256 CUs on which the call's one-launch
  * kernel fits one workgroup per CU, experts a multiple of 32 up to 256; for
  * one token hidden up to 2048 and inter up to 1024; for 2..8 tokens inter 512 or
  * 256, hidden 512..2048 in multiples of 256, and gate and up matrices, routed and
@@ -242,20 +242,27 @@ typedef struct {
  * ascending id of w * expert(X[t]) -- model.c:1671-1791.  X, Y: [T x hidden]. */
 int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, int T, float *Y,
                         const RoasterPrefillOpts *opts);
+/* The GEMM kernels such a call of T tokens takes under the switches below
+ * (precision: ROASTER_PREC_*), or NULL (bad arguments).  In fp16 mode short
+ * prompts, up to 28 rows per expert on average (8 T <= 28 n_experts) for Q6_K gate
+ * matrices and 36 for Q4_K, run gate/up on narrow tiles (pfn_gu_kernel) where
+ * the routed and the shared gate and up types match, and there also down with
+ * Q4_K down matrices, or with Q6_K while 8 T <= n_experts (pfn_down_kernel).  Those
+ * GEMMs hold the weights exactly, so a token's fp16-mode outputs in a short and
+ * in a long call differ by the rounding of fp16 weights. */
+const char *roaster_prefill_kernels(const RoasterTable *t, int layer, int T, int precision);
 /* The fp16-mode down GEMM (inter <= 512) as one workgroup per CU over an even
  * split of its output tiles (1, default) or one workgroup per four output
- * tiles (0); -1 queries.  Both give bit-identical results.  Returns the mode
- * in force. */
+ * tiles (0); -1 queries.  Both give bit-identical results; without effect where
+ * down runs on narrow tiles.  Returns the mode in force. */
 int roaster_prefill_balanced_down(int enable);
-/* The fp16-mode gate/up GEMM of longer prompts (past 28 rows per expert on
- * average for Q6_K gate matrices, 36 for Q4_K; shorter ones run on
- * 32-row tiles where gate and up types match, whatever this says) on
- * a persistent grid, one workgroup per CU taking
+/* The fp16-mode gate/up GEMM on a persistent grid, one workgroup per CU taking
  * (tile, 128-column) units from work counters and preparing the next unit
  * while one runs (1, default; layers whose routed and shared gate and up
  * matrices share one type and whose hidden size is a multiple of 512, at
  * least 2048), or one workgroup per unit (0); -1 queries.  Both give
- * bit-identical results.  Returns the mode in force. */
+ * bit-identical results; without effect where gate/up runs on narrow tiles.
+ * Returns the mode in force. */
 int roaster_prefill_persistent_gate_up(int enable);
 /* Both fp16-mode GEMMs in one persistent kernel (1, where the persistent
  * gate/up grid and the balanced down GEMM both apply and the GPU has 8
@@ -263,7 +270,8 @@ int roaster_prefill_persistent_gate_up(int enable);
  * then their down chunks once a chunk's tile is complete, so the down work
  * fills the gate/up tail; or two kernels (0, default: the one kernel
  * measured 1-3% faster, within the spread between boxes); -1 queries.  Both
- * give bit-identical results.  Returns the mode in force. */
+ * give bit-identical results; without effect where gate/up runs on narrow
+ * tiles.  Returns the mode in force. */
 int roaster_prefill_fused_gemm(int enable);
 
 #ifdef __cplusplus

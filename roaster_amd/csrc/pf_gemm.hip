@@ -1729,3 +1729,16 @@ int pf_gemm_launch(const PfGemmArgs &A, int max_tiles, int op, int max_nw, bool 
     hipLaunchKernelGGL(pf2_down_kernel, dim3(max_tiles * (A.H / V2_DN_N / D.dn_nt)), dim3(V2_T), lds_dn, R.stream, D);
     return rt_check(hipGetLastError(), "prefill down launch") ? ROASTER_EDEVICE : 0;
 }
+
+/* The kernels pf_gemm_launch takes. */
+const char *pf_gemm_names(const PfRoute &r, int op, int I)
+{
+    static const char *const names[3][3] = {
+        { "pfn_gu_kernel + pfn_down_kernel", "pfn_gu_kernel + pf2_down_bal_kernel", "pfn_gu_kernel + pf2_down_kernel" },
+        { NULL, "pf2_gu_pers_kernel + pf2_down_bal_kernel", "pf2_gu_pers_kernel + pf2_down_kernel" },
+        { NULL, "pf2_gu_kernel + pf2_down_bal_kernel", "pf2_gu_kernel + pf2_down_kernel" },
+    };
+    if (!r.narrow && op != PF_F16) return "pf_gu_kernel + pf_down_kernel";
+    if (r.fused) return "pf2_fused_kernel";
+    return names[r.narrow ? 0 : r.gu_pers && g_pf_gu_pers ? 1 : 2][r.nw_down ? 0 : I <= 2 * GK && g_pf_dn_bal ? 1 : 2];
+}

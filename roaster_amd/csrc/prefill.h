@@ -106,6 +106,16 @@ bool pf_fused_enabled();
  * mixed_gate_up: the gate and up matrices of some group differ in type. */
 int pf_gemm_chunk(int op, bool mixed_gate_up);
 
+/* The GEMMs of one prefill call (prefill.hip), and their kernels' names under
+ * the switches in force. */
+struct PfRoute {
+    bool nw_split, nw_f16;          /* gate/up on narrow tiles, by mode */
+    bool narrow, nw_down;           /* either; down on them too */
+    int gu_pers;                    /* PfGemmArgs.gu_pers */
+    bool fused;                     /* both GEMMs in one kernel */
+};
+const char *pf_gemm_names(const PfRoute &r, int op, int I);
+
 /* Launch the gate/up and down GEMMs over up to max_tiles tiles.  op: PF_F16,
  * PF_SPLIT or PF_BF16 (gemm.h).  max_nw > 0 (PF_F16, PF_SPLIT): gate/up, and
  * down with nw_down, on up to max_nw narrow tiles (pf_narrow.hip).  0 or

@@ -27,6 +27,7 @@
 #include "internal.h"
 #include "gemm.h"
 #include "prefill.h"
+#include "pf_tile.h"
 #include "table.h"
 #include "topk.h"
 
@@ -34,15 +35,6 @@
 
 #define PF_MAX_T (1 << 16)
 #define RT_KSPLIT 8               /* router K split */
-
-/* Natural position p (multiple of 4) inside a super-block -> the slot of its
- * first element in the fp16 GEMM's permuted K order (pf_gemm.hip). */
-__device__ __forceinline__ int pf_perm_slot4(int p)
-{
-    const int h = p >> 7, q = p & 127, hi = q >> 6, r = q & 63;
-    const int l0 = r < 32 ? r : r - 32, i0 = r < 32 ? 0 : 4;
-    return (8 * hi + (l0 >> 2)) * 16 + 8 * h + i0;
-}
 
 /* Exclusive prefix sum over a 256-thread workgroup; *total gets the sum. */
 __device__ int block_scan_256(int v, int *lds, int *total)
@@ -625,7 +617,7 @@ __global__ void __launch_bounds__(256, 4) pf_token_kernel(PfTokArgs A, PfPlanArg
                     const f32x8 e = { v.x * inv, v.y * inv, v.z * inv, v.w * inv, 0.f, 0.f, 0.f, 0.f };
                     const f16x8 hi = __builtin_convertvector(e, f16x8);
                     const uint4 c = __builtin_bit_cast(uint4, hi);
-                    const size_t at = (size_t)t * A.H + (k & ~255) + pf_perm_slot4(k & 255);
+                    const size_t at = (size_t)t * A.H + (k & ~255) + perm_slot4(k & 255);
                     *(uint2 *)(A.x16 + at) = make_uint2(c.x, c.y);
                     f32x8 used = __builtin_convertvector(hi, f32x8);
                     if (A.x16l) {
@@ -788,6 +780,48 @@ extern "C" __global__ void __launch_bounds__(256) pf_combine16_kernel(const uint
 /* ---- host ---------------------------------------------------------------- */
 static inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
+/* Which GEMMs a call takes.  The narrow tiles with exact integer weights
+ * (pf_narrow.hip) take layers whose routed and shared gate and up matrices are
+ * each of one type: in split mode at any token count (inter <= 512; a layer of
+ * hidden 2048, inter 512, 256 experts, Q4_K gate/up, us against the 64 x 64 tiles
+ * of gemm.h: 1 token 81 -> 41, 1024 1294 -> 378, 8192 6403 -> 2124; 8 experts and
+ * 8192 tokens 5849 -> 1977), in fp16 mode up to a line (pf_narrow_f16). */
+static PfRoute pf_route(const LayerGeo &G, int op, int T, int E, int H, int I)
+{
+    PfRoute r;
+    const bool one_type = G.q6[0] == G.q6[1] && G.sh_q6[0] == G.sh_q6[1];
+    r.nw_split = op == PF_SPLIT && one_type && I <= 2 * GK;
+    r.nw_f16 = op == PF_F16 && one_type && pf_narrow_f16(T, E, G.q6[0]);
+    r.narrow = r.nw_split || r.nw_f16;
+    r.nw_down = r.nw_split || (r.nw_f16 && I <= 2 * GK && pf_narrow_f16_down(T, E, G.q6[2]));
+    /* the persistent gate/up grid takes layers whose routed and shared gate
+     * and up matrices share one type and whose K loop has an even number
+     * (>= 8) of super-block steps; both GEMMs in one persistent kernel: on that
+     * grid and the balanced down GEMM, 8 XCDs of equal CU counts */
+    const int q6 = G.q6[0];
+    const bool gu_one = G.q6[1] == q6 && G.sh_q6[0] == q6 && G.sh_q6[1] == q6;
+    r.gu_pers = op == PF_F16 && gu_one && (H / 256) % 2 == 0 && H / 256 >= 8 ? 1 + q6 : 0;
+    RtState &R = rt();
+    r.fused = r.gu_pers && !r.nw_f16 && I <= 2 * GK && R.n_xcd == 8 && R.n_cu % 8 == 0 && pf_fused_enabled();
+    return r;
+}
+
+static int pf_op(int precision)
+{
+    return precision == ROASTER_PREC_F16 ? PF_F16 : precision == ROASTER_PREC_SPLIT ? PF_SPLIT : PF_BF16;
+}
+
+extern "C" const char *roaster_prefill_kernels(const RoasterTable *t, int layer, int T, int precision)
+{
+    std::lock_guard<std::recursive_mutex> lk(rt_lock());
+    if (rt_init_locked()) return NULL;
+    if (!t || layer < 0 || layer >= t->d.n_layers || T < 1 || T > PF_MAX_T || t->d.n_experts > 256 ||
+        precision < ROASTER_PREC_F16 || precision > ROASTER_PREC_BF16)
+        return rt_fail(ROASTER_EINVAL, "roaster_prefill_kernels: bad arguments"), (const char *)NULL;
+    const int op = pf_op(precision), I = (int)t->d.inter;
+    return pf_gemm_names(pf_route(t->geo[layer], op, T, t->d.n_experts, (int)t->d.hidden, I), op, I);
+}
+
 extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, int T, float *Y,
                                    const RoasterPrefillOpts *o)
 {
@@ -802,18 +836,13 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
         return rt_fail(ROASTER_EINVAL, "roaster_moe_prefill: unknown precision %d", opt.precision);
     const int E = t->d.n_experts, H = (int)t->d.hidden, I = (int)t->d.inter;
     if (E > 256) return rt_fail(ROASTER_EINVAL, "roaster_moe_prefill: at most 256 routed experts");
-    const int op = opt.precision == ROASTER_PREC_F16 ? PF_F16 : opt.precision == ROASTER_PREC_SPLIT ? PF_SPLIT : PF_BF16;
+    const int op = pf_op(opt.precision);
     const size_t TT = (size_t)T, slots = 9 * TT;
     const LayerGeo &LG = t->geo[layer];
     const int chunk = pf_gemm_chunk(op, LG.q6[0] != LG.q6[1] || LG.sh_q6[0] != LG.sh_q6[1]);
     const int max_tiles = (int)((8 * TT + chunk - 1) / chunk + E + (TT + chunk - 1) / chunk);
-    /* narrow tiles with exact integer weights (pf_narrow.hip): the routed and
-     * the shared expert's gate and up matrices each of one type */
-    const bool one_type = LG.q6[0] == LG.q6[1] && LG.sh_q6[0] == LG.sh_q6[1];
-    const bool nw_split = op == PF_SPLIT && one_type && I <= 2 * GK;
-    const bool nw_f16 = op == PF_F16 && one_type && pf_narrow_f16(T, E, LG.q6[0]);
-    const bool narrow = nw_split || nw_f16;
-    const bool nw_down = nw_split || (nw_f16 && I <= 2 * GK && pf_narrow_f16_down(T, E, LG.q6[2]));
+    const PfRoute route = pf_route(LG, op, T, E, H, I);
+    const bool nw_split = route.nw_split, narrow = route.narrow, fused = route.fused;
     const int nw_rows = pf_narrow_rows(nw_split);
     const int max_nw = (int)((8 * TT + nw_rows - 1) / nw_rows + E + (TT + nw_rows - 1) / nw_rows);
 
@@ -890,12 +919,6 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     pa.gu_ctr = (int *)(ws + o_nt) + 32;            /* its own cache line of the 256-byte slot */
     pa.dn_bnd = op == PF_F16 ? (int *)(ws + o_bnd) : nullptr;
     pa.dn_tiles = op == PF_F16 ? (PfDnTile *)(ws + o_dnt) : nullptr;
-    /* both GEMMs in one persistent kernel: fp16 mode on the persistent gate/up
-     * grid and the balanced down GEMM, 8 XCDs of equal CU counts */
-    const int q6 = LG.q6[0];
-    const bool gu_one = LG.q6[1] == q6 && LG.sh_q6[0] == q6 && LG.sh_q6[1] == q6;
-    const int gu_pers = op == PF_F16 && gu_one && (H / 256) % 2 == 0 && H / 256 >= 8 ? 1 + q6 : 0;
-    const bool fused = gu_pers && !nw_f16 && I <= 2 * GK && R.n_xcd == 8 && R.n_cu % 8 == 0 && pf_fused_enabled();
     pa.fx = fused ? (int *)(ws + o_fx) : nullptr;
     pa.n_wg = R.n_cu;
     pa.nt_out = H / PF_DN_ROWS;
@@ -944,17 +967,14 @@ extern "C" int roaster_moe_prefill(RoasterTable *t, int layer, const float *X, i
     ga.dn_bnd = pa.dn_bnd;
     ga.dn_tiles = pa.dn_tiles;
     ga.dn_spare = (int)slots;                    /* o_ed holds one row past the slots */
-    /* the persistent gate/up grid takes layers whose routed and shared gate
-     * and up matrices share one type and whose K loop has an even number
-     * (>= 8) of super-block steps */
-    ga.gu_pers = gu_pers;
+    ga.gu_pers = route.gu_pers;
     ga.gu_ctr = pa.gu_ctr;
     ga.fused = fused ? 1 : 0;
     ga.xcd_tb = fused ? pa.fx : nullptr;
     ga.dn_ctr = fused ? pa.fx + 16 : nullptr;
     ga.tile_done = fused ? pa.fx + 32 : nullptr;
     ga.err = (int *)(ctrl + 16);
-    if (int rc = pf_gemm_launch(ga, max_tiles, op, narrow ? max_nw : 0, nw_down)) return rc;
+    if (int rc = pf_gemm_launch(ga, max_tiles, op, narrow ? max_nw : 0, route.nw_down)) return rc;
 
     if (op == PF_F16)
         hipLaunchKernelGGL(pf_combine16_kernel, dim3(T), dim3(256), 0, R.stream, (const uint16_t *)ga.out16,

@@ -65,6 +65,20 @@ def q6tab():
     t.destroy()
 
 
+@pytest.fixture(scope="module")
+def e8tab():
+    """Eight experts of the model's types: past the narrow tiles' line at few tokens."""
+    t = SynthTable(6, n_experts=8)
+    yield t
+    t.destroy()
+
+
+def kernels(tab, T, precision=R.PREC_F16):
+    """The GEMM kernels of a call, so that a test that is about one fails where the
+    dispatch no longer takes it."""
+    return R.lib().roaster_prefill_kernels(tab.t, 0, T, precision).decode()
+
+
 def test_prefill_config3_zipf(cfg3, cfg3_oracle):
     """T = 512, Zipf-biased routing (expert lists 0 .. ~200 rows), F16 operands."""
     T = 512
@@ -166,9 +180,11 @@ def test_prefill_balanced_down_bit_exact(cfg3, T):
     b = zipf_bias(256, 2)
     lib = R.lib()
     assert lib.roaster_prefill_balanced_down(-1) == 1
+    assert kernels(cfg3, T).endswith(" + pf2_down_bal_kernel")
     Y1, _, ids1, _, _ = prefill(cfg3, X, bias=b)
     try:
         assert lib.roaster_prefill_balanced_down(0) == 0
+        assert kernels(cfg3, T).endswith(" + pf2_down_kernel")
         Y0, _, ids0, _, _ = prefill(cfg3, X, bias=b)
     finally:
         lib.roaster_prefill_balanced_down(1)
@@ -176,20 +192,27 @@ def test_prefill_balanced_down_bit_exact(cfg3, T):
     np.testing.assert_array_equal(Y0, Y1)
 
 
-@pytest.mark.parametrize("which,T", [("cfg3", 512), ("cfg3", 37), ("q6", 2048)])
+TABLES = {"cfg3": "cfg3", "q6": "q6tab", "e8": "e8tab"}
+
+
+@pytest.mark.parametrize("which,T", [("cfg3", 1153), ("cfg3", 2048), ("e8", 37), ("e8", 101), ("q6", 897), ("q6", 2048)])
 def test_prefill_persistent_gate_up_bit_exact(request, which, T):
     """The gate/up GEMM on its persistent grid (work counters, the next unit
     prepared during the current one) gives the bits of one workgroup per
-    unit: Zipf routing on the Q4_K table (tiles of 1..96 rows; T = 37: fewer
-    units than CUs) and the all-Q6_K table at 2048 tokens."""
-    tab = request.getfixturevalue("cfg3" if which == "cfg3" else "q6tab")
+    unit: Zipf routing on the Q4_K table (tiles of 1..96 rows) and the all-Q6_K
+    table, from the first token count past the narrow tiles on, and eight experts
+    (36 units of one tile each, and a tile of 5 rows beside one of 96: fewer
+    units than CUs)."""
+    tab = request.getfixturevalue(TABLES[which])
     X = tokens(14, T, start=7000)
     b = zipf_bias(256, 2) if which == "cfg3" else None
     lib = R.lib()
     assert lib.roaster_prefill_persistent_gate_up(-1) == 1
+    assert kernels(tab, T).startswith("pf2_gu_pers_kernel")
     Y1, _, ids1, _, _ = prefill(tab, X, bias=b)
     try:
         assert lib.roaster_prefill_persistent_gate_up(0) == 0
+        assert kernels(tab, T).startswith("pf2_gu_kernel")
         Y0, _, ids0, _, _ = prefill(tab, X, bias=b)
     finally:
         lib.roaster_prefill_persistent_gate_up(1)
@@ -197,15 +220,16 @@ def test_prefill_persistent_gate_up_bit_exact(request, which, T):
     np.testing.assert_array_equal(Y0, Y1)
 
 
-@pytest.mark.parametrize("which,T", [("cfg3", 512), ("cfg3", 37), ("cfg3", 3), ("cfg3", 1), ("q6", 2048), ("q6", 300)])
+@pytest.mark.parametrize("which,T", [("cfg3", 1153), ("cfg3", 2048), ("e8", 37), ("e8", 101), ("q6", 897), ("q6", 2048)])
 def test_prefill_fused_gemm_bit_exact(request, which, T):
     """Both GEMMs in one persistent kernel (each XCD's workgroups take its
     tiles' gate/up units, then their down chunks once a tile's units are all
     counted) gives the bits of the two-kernel path: Zipf routing on the Q4_K
-    table (T = 37, 3, 1: XCDs with one tile or none) and the all-Q6_K table,
-    twice in a row (the counters are re-zeroed by each call's plan kernel);
-    no tile wait gives up (the call reports no error)."""
-    tab = request.getfixturevalue("cfg3" if which == "cfg3" else "q6tab")
+    table and the all-Q6_K table, from the first token count past the narrow
+    tiles on, and eight experts (nine tiles for eight XCDs, the least a call can
+    have, or eighteen), twice in a row (the counters are re-zeroed by each
+    call's plan kernel); no tile wait gives up (the call reports no error)."""
+    tab = request.getfixturevalue(TABLES[which])
     X = tokens(15, T, start=9000)
     b = zipf_bias(256, 2) if which == "cfg3" else None
     lib = R.lib()
@@ -213,6 +237,7 @@ def test_prefill_fused_gemm_bit_exact(request, which, T):
     Y0, _, ids0, _, _ = prefill(tab, X, bias=b)
     try:
         assert lib.roaster_prefill_fused_gemm(1) == 1
+        assert kernels(tab, T) == "pf2_fused_kernel"
         Y1, _, ids1, _, _ = prefill(tab, X, bias=b)
         Y2, _, _, _, _ = prefill(tab, X, bias=b)
         R.check(lib.roaster_sync(), "sync after the fused calls")
@@ -221,6 +246,45 @@ def test_prefill_fused_gemm_bit_exact(request, which, T):
     np.testing.assert_array_equal(ids0, ids1)
     np.testing.assert_array_equal(Y0, Y1)
     np.testing.assert_array_equal(Y0, Y2)
+
+
+def test_prefill_q4k_long_prompt(cfg3, cfg3_oracle):
+    """The persistent gate/up grid on Q4_K matrices, Zipf routing: a sample of the
+    tokens against the oracle (a token's output depends on its own input and
+    logits alone)."""
+    T = 1153
+    assert kernels(cfg3, T) == "pf2_gu_pers_kernel + pf2_down_bal_kernel"
+    X = tokens(18, T, start=11000)
+    Y, lg, ids, w, counts = prefill(cfg3, X, bias=zipf_bias(256, 2))
+    sample = np.sort(np.random.default_rng(18).choice(T, 48, replace=False))
+    sample[-1] = T - 1
+    check_routing(lg[sample], ids[sample], w[sample], np.bincount(ids[sample].ravel(), minlength=256), 256)
+    assert np.array_equal(counts, np.bincount(ids.ravel(), minlength=256))
+    rc, Y_ref, _, _, _ = cfg3_oracle.prefill(np.ascontiguousarray(X[sample]), logits_in=np.ascontiguousarray(lg[sample]))
+    assert rc == 0
+    err = rel_err(Y[sample], Y_ref)
+    log(f"Q4_K gate/up, {T} tokens: max|d|/max|y| = {err:.3e}")
+    assert err <= TOL
+
+
+@pytest.mark.parametrize("q6,I", [((0, 1, 0), 512), ((1, 0, 1), 512), ((0, 0, 1), 768)])
+def test_prefill_split_wide_tiles(q6, I):
+    """Split mode where the narrow tiles don't apply, gate and up of two types or
+    inter above 512: the 64 x 64 tiles with bf16 hi + lo operands."""
+    T, E = 70, 16
+    tab = SynthTable(43, n_experts=E, hidden=1024, inter=I, q6=q6, sh_q6=q6)
+    try:
+        assert kernels(tab, T, R.PREC_SPLIT) == "pf_gu_kernel + pf_down_kernel"
+        X = tokens(19, T, H=1024, start=700)
+        Y, lg, ids, w, counts = prefill(tab, X, precision=R.PREC_SPLIT)
+        check_routing(lg, ids, w, counts, E)
+        rc, Y_ref, _, _, _ = tab.oracle_layer(0).prefill(X, logits_in=lg)
+        assert rc == 0
+        err = rel_err(Y, Y_ref)
+        log(f"split, types {q6}, inter {I}: max|d|/max|y| = {err:.3e}")
+        assert err <= TOL_SPLIT
+    finally:
+        tab.destroy()
 
 
 def test_prefill_fp16_products_scaled_by_their_bound():
@@ -371,22 +435,26 @@ def test_prefill_all_q6k_2048_every_token():
         tab.destroy()
 
 
-@pytest.mark.parametrize("E,H,I", [(64, 1024, 256), (64, 2048, 256), (32, 1536, 1024)])
-def test_prefill_other_shapes(E, H, I):
+@pytest.mark.parametrize("E,H,I,gu", [(64, 1024, 256, "pfn_gu_kernel"), (64, 2048, 256, "pfn_gu_kernel"),
+                                      (32, 1024, 256, "pf2_gu_kernel"), (32, 2048, 256, "pf2_gu_pers_kernel"),
+                                      (32, 1536, 1024, "pf2_gu_kernel")])
+def test_prefill_other_shapes(E, H, I, gu):
     """Shapes beside the model's: inter 256 (the down GEMM's one-K-step
     tile ranges, four part maxima per row) at hidden 1024 (four output tiles
-    per tile; the gate/up GEMM one workgroup per unit) and 2048 (the
-    persistent gate/up grid, two units per tile), and inter 1024 at hidden
-    1536 (the down GEMM's per-tile grid over four K steps).  fp16 mode
-    against the oracle at the prefill bar, and the down GEMM's balanced
-    split, its per-tile grid and the one-kernel GEMMs bit for bit against
-    each other where they apply."""
+    per tile) and 2048, with 64 experts on narrow gate/up tiles, with 32 past their
+    line (at 1024 one workgroup per unit, at 2048 the persistent gate/up grid,
+    two units per tile), and inter 1024 at hidden 1536 (the down GEMM's
+    per-tile grid over four K steps).  fp16 mode against the oracle at the
+    prefill bar, and the down GEMM's balanced split, its per-tile grid and the
+    one-kernel GEMMs bit for bit against each other where they apply."""
     T = 150
     tab = SynthTable(41, n_experts=E, hidden=H, inter=I)
     lib = R.lib()
     try:
         X = tokens(16, T, H=H, start=500)
         lg_in = np.stack([R.synth_normal(17, R.synth_stream(0, t, 7), E) for t in range(T)]).astype(np.float32)
+        down = "pf2_down_bal_kernel" if I <= 512 else "pf2_down_kernel"
+        assert kernels(tab, T) == f"{gu} + {down}"
         Y, lg, ids, w, counts = prefill(tab, X, logits_in=lg_in)
         rc, Y_ref, ids_ref, _, _ = tab.oracle_layer(0).prefill(X, logits_in=lg_in)
         assert rc == 0 and np.array_equal(ids_ref, ids)
@@ -395,12 +463,14 @@ def test_prefill_other_shapes(E, H, I):
         assert err <= TOL
         try:
             assert lib.roaster_prefill_balanced_down(0) == 0
+            assert kernels(tab, T) == f"{gu} + pf2_down_kernel"
             Y0, _, _, _, _ = prefill(tab, X, logits_in=lg_in)
         finally:
             lib.roaster_prefill_balanced_down(1)
         np.testing.assert_array_equal(Y0, Y)
         try:
             assert lib.roaster_prefill_fused_gemm(1) == 1
+            assert (kernels(tab, T) == "pf2_fused_kernel") == (gu == "pf2_gu_pers_kernel")
             Y1, _, _, _, _ = prefill(tab, X, logits_in=lg_in)
         finally:
             lib.roaster_prefill_fused_gemm(0)
