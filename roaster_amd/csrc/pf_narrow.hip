@@ -20,7 +20,10 @@
  * one MFMA per slice forms both products and a lane adds its accumulators i
  * and i + 8.  Against the bf16 hi + lo operands of gemm.h, which serve
  * PF_SPLIT where this file does not, the weights lose nothing and the
- * activations 6 bits less.
+ * activations 6 bits less, down to about 2^-22 of their row's largest; below that
+ * an element's error stays at 2^-39 of the largest, where bf16 hi + lo has 2^-17 of
+ * the element.  Against 64 bits, N(0, 1) activations, 256 tokens of a layer: 7.2e-6
+ * -> 3.0e-7.
  */
 #include <type_traits>
 
