@@ -304,15 +304,24 @@ __device__ __forceinline__ void mm8_prep(const float *X, int cols, int T, int kb
         }
     }
     /* sub-block c's sum, in lane group c / 2's slot c % 2; two rows a token: the
-     * third part in the second row's slot 2 + c % 2 */
+     * third part in the second row's slot 2 + c % 2, lanes c and c ^ 1 swapping
+     * what the other's row holds, so that each stores one row's four slots */
     sum *= 0.015625f;
+    _Float16 sp[3];
 #pragma unroll
-    for (int p = 0; p < PARTS; p++) {
-        const _Float16 h = (_Float16)sum;
-        _Float16 *o = sums + (16 * (c >> 1) + row + p) * MM8_SUM(Q6, PARTS) + (c & 1);
-        *o = h;
-        sum -= (float)h;
-        if (MM8_SUM(Q6, PARTS) == 4) o[2] = p == 0 ? (_Float16)0.0f : (_Float16)sum;
+    for (int p = 0; p < 3; p++) {
+        sp[p] = (_Float16)sum;
+        sum -= (float)sp[p];
+    }
+    if constexpr (MM8_SUM(Q6, PARTS) == 4) {
+        const bool odd = (c & 1) != 0;
+        const f16x2 mine = odd ? (f16x2){ sp[0], (_Float16)0.0f } : (f16x2){ sp[1], sp[2] };
+        const f16x2 got = __builtin_bit_cast(f16x2, dpp_i<DPP_XOR1>(__builtin_bit_cast(int, mine)));
+        *(f16x4 *)(sums + (16 * (c >> 1) + row + (odd ? 1 : 0)) * 4) =
+            odd ? (f16x4){ got[0], sp[1], got[1], sp[2] } : (f16x4){ sp[0], got[0], (_Float16)0.0f, (_Float16)0.0f };
+    } else {
+#pragma unroll
+        for (int p = 0; p < PARTS; p++) sums[(16 * (c >> 1) + row + p) * 2 + (c & 1)] = sp[p];
     }
 }
 
