@@ -2,7 +2,7 @@
 reference's own CPU kernels (_ref/libref.so).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and
-bench.py's cpu_baseline leg as the checker, never by the product.
+bench.py's cpu_baseline leg as the oracle, never by the product.
 """
 import ctypes as C
 import os

@@ -1,7 +1,7 @@
 /*
  * roaster_oracle.c -- CPU restatement of the reference's MoE-FFN CPU path.
  *
- * TEST INFRASTRUCTURE ONLY (the checker, never the product): loaded by tests/,
+ * TEST INFRASTRUCTURE ONLY (never the product): loaded by tests/,
  * __graft_entry__.smoke() and bench.py's cpu_baseline leg, nothing else.
  *
  * The reference computes its dots with 8-lane AVX2 vectors.  This file keeps

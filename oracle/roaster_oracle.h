@@ -1,7 +1,7 @@
 /*
  * roaster_oracle.h -- CPU restatement of the reference's MoE-FFN CPU path.
  *
- * TEST INFRASTRUCTURE ONLY.  This library is the checker, never the product:
+ * TEST INFRASTRUCTURE ONLY.  This library is the oracle, never the product:
  * only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may
  * load it.  The product path (libroaster_moe.so) never links or calls it.
  *

@@ -893,8 +893,9 @@ __device__ void down_slots(const DecArgs &A, const uint8_t *const *sd, int k0, i
 /* Down rows and combine for one token when the slots' down matrices (nine, or
  * kernel_ffn_fused's experts) share one type D6 (A.d1, set per launch): each
  * wave reads its tasks' slot pointers straight from the published plan and
- * issues the weight-row loads as soon as they arrive, before the SiLU*up rows are stored to LDS, so the rows'
- * memory latency overlaps the copy, the barriers and the run sums.  Tasks as
+ * issues the weight-row loads as soon as they arrive, before the SiLU*up rows
+ * are stored to LDS, so the rows' memory latency overlaps the copy, the
+ * barriers and the run sums.  Tasks as
  * in down_slots (q = k * ngroups + g, wave w takes q = w, w + 4, ...; the
  * host checks that D_PF tasks per wave cover them); loads are unconditional
  * (clamped task, row and block; an unselected slot reads the shared slot's

@@ -61,8 +61,9 @@ __global__ void __launch_bounds__(MV_THREADS) matvec_jobs_kernel(const MvJob *jo
  * tokens: the dense projections around the MoE block and the LM head
  * (model.c:795-800, 1284-1290, 1344-1347, 1368-1370; the same products
  * tensor_matvec_f32_or_quant, model.c:113-121, sends to kernel_matvec_q*_k).
- * cols <= 2048, so one lane group covers a whole row (8 lanes per
- * super-block, lanes_per_row(blocks) lanes per row, 64 / lpr rows per wave pass).
+ * cols <= 4096: one lane group covers a whole row (8 lanes per super-block,
+ * lanes_per_row(blocks) lanes per row, 64 / lpr rows per wave pass), past 2048
+ * columns with two super-blocks a lane.
  * Each lane's activation runs are fixed for every row it serves: with one
  * token they sit in registers for the whole kernel, with more in LDS.  Every
  * wave keeps the next row pass's loads in flight while it computes one. */
@@ -326,8 +327,9 @@ __device__ __forceinline__ void mm8_prep(const float *X, int cols, int T, int kb
 }
 
 /* Lane group g's share of a super-block: 16-byte runs, so that the four lanes
- * of a row read 64 contiguous bytes a load.  Q4_K: qs bytes 64 k + 16 g (sub-blocks 4 k + 2 (g / 2), + 1); Q6_K, by half n:
- * ql bytes 64 n + 16 g (scales 8 n + g, + 4) and the qh bytes under them. */
+ * of a row read 64 contiguous bytes a load.  Q4_K: qs bytes 64 k + 16 g
+ * (sub-blocks 4 k + 2 (g / 2), + 1); Q6_K, by half n: ql bytes 64 n + 16 g
+ * (scales 8 n + g, + 4) and the qh bytes under them. */
 struct Mm8Q4 { uint4 hd, p[2]; };
 struct Mm8Q6 { U5 l[2], h[2], sc; uint32_t d, sh; };
 

@@ -2,8 +2,8 @@
 against the oracle: sc (q - 32) and the fp16 constants around it must not
 overflow.  Routed and shared types are opposite, so each call runs both weight
 types; the gate/up GEMM is the narrow one at T = 1, the wide one from T = 29 with
-routed Q6_K gate matrices and from 37 with Q4_K ones (shared Q6_K).  The bar is the fp16 operands' 2e-3 of max|y|, as in every fp16 prefill
-test."""
+routed Q6_K gate matrices and from 37 with Q4_K ones (shared Q6_K).  The bar is
+the fp16 operands' 2e-3 of max|y|, as in every fp16 prefill test."""
 import numpy as np
 import pytest
 
